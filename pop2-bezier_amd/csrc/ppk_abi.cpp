@@ -828,6 +828,8 @@ void run_attention(ppk_context* ctx, hipStream_t stream, const PpkAttentionArgs&
   }
   d.rows = a.rows;
   d.heads = a.heads;
+  d.row_div = fast_divisor(a.rows);
+  d.head_div = fast_divisor(a.heads);
   d.capacity = a.capacity;
   d.split_tokens = plan.split;
   d.ngroups = plan.ngroups;

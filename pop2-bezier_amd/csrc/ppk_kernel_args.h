@@ -11,6 +11,20 @@ constexpr int kWave = 64;
 // Bytes one lane moves per global load in the attention kernels (dwordx4).
 constexpr int kLaneBytes = 16;
 
+// Division of x < 2^31 by a fixed d >= 1 as a multiply-high and a shift: with
+// l = ceil(log2 d) and mul = floor(2^(31 + l) / d) + 1, mul * d exceeds 2^(31 +
+// l) by at most d <= 2^l, so x / d = (x * mul) >> (31 + l) exactly. mul = 0
+// stands for d = 1.
+struct FastDiv {
+  uint32_t mul, shift;      // (x * mul >> 32) >> shift
+};
+inline FastDiv fast_divisor(uint32_t d) {
+  if (d <= 1) return {0, 0};
+  uint32_t l = 0;
+  while ((uint64_t(1) << l) < d) ++l;
+  return {uint32_t((uint64_t(1) << (31 + l)) / d + 1), l - 1};
+}
+
 // Quantize one (row, token) of D channels per wave, either densely
 // (dst index = src index) or into an arena slot past[b] + token.
 struct QuantizeArgs {
@@ -100,6 +114,7 @@ struct DecodeArgs {
   uint32_t span;            // max_past or capacity: balanced plan, rows with past[b] > span give NaN; per-row
                             // plan, a past[b] <= span past the plan's coverage flags stale host lengths
   uint32_t speculate;       // per-row plan: request each wave's first K batches before past[] arrives
+  FastDiv row_div, head_div;  // by rows, by heads
   uint32_t clock_seq;       // wave-clock builds only: the launch's sequence number in the records
   uint32_t clock_cap;       // wave-clock builds only: records the buffer holds (from its size on the host)
   uint64_t* clock;          // wave-clock builds only (kWaveClock*): record buffer, or null

@@ -78,6 +78,10 @@ __device__ __forceinline__ void clock_record(uint64_t* clock, uint32_t seq, uint
 using u2 = uint32_t __attribute__((ext_vector_type(2)));
 using u4 = uint32_t __attribute__((ext_vector_type(4)));
 using f4 = float __attribute__((ext_vector_type(4)));
+// Views of LDS that the compiler may not reorder against accesses of another type.
+typedef uint16_t __attribute__((may_alias)) u16_alias;
+typedef uint32_t __attribute__((may_alias)) u32_alias;
+typedef uint32_t __attribute__((ext_vector_type(4), may_alias)) u4_alias;
 
 enum { kF32 = 0, kBF16 = 1, kF16 = 2 };
 
@@ -110,6 +114,38 @@ __device__ __forceinline__ void load_vec(const void* p, size_t i, uint32_t dtype
 #pragma unroll
       for (int e = 0; e < N; ++e) out[e] = f16_to_f32(b[e]);
     }
+  }
+}
+
+// The same elements as they are stored, to be widened later: one load (per
+// dtype branch) whose result no instruction of the branch reads. A widening
+// inside the branch makes the wave wait for the load there, and for every
+// load before it, so a kernel that reads several small operands in both
+// 16-bit dtypes that way pays one memory round trip after another before its
+// stream starts; raw words let them all travel together.
+template <int N>
+struct RawVec {
+  uint32_t w[N];  // f32: one element each; 16-bit: element e in half e % 2 of word e / 2
+};
+template <int N>
+__device__ __forceinline__ void load_raw(const void* p, size_t i, uint32_t dtype, RawVec<N>& r) {
+  if (dtype == kF32) {
+    __builtin_memcpy(r.w, __builtin_assume_aligned(static_cast<const float*>(p) + i, 4), 4 * N);
+  } else if constexpr (N == 1) {
+    r.w[0] = static_cast<const uint16_t*>(p)[i];
+  } else {
+    __builtin_memcpy(r.w, __builtin_assume_aligned(static_cast<const uint16_t*>(p) + i, 2), 2 * N);
+  }
+}
+template <int N>
+__device__ __forceinline__ void widen(const RawVec<N>& r, uint32_t dtype, float (&x)[N]) {
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    // All three readings are formed and one is selected: no branch per element.
+    const uint16_t h = uint16_t(r.w[e / 2] >> (16 * (e % 2)));
+    const float as_f32 = __uint_as_float(r.w[e]), as_bf16 = bf16_to_f32(h), as_f16 = f16_to_f32(h);
+    const float as_half = dtype == kBF16 ? as_bf16 : as_f16;
+    x[e] = dtype == kF32 ? as_f32 : as_half;
   }
 }
 
@@ -148,6 +184,23 @@ __device__ __forceinline__ uint16_t f32_to_f16_bits(float x) {
 __device__ __forceinline__ void store_elem(void* p, size_t i, uint32_t dtype, float x) {
   if (dtype == kF32) static_cast<float*>(p)[i] = x;
   else static_cast<uint16_t*>(p)[i] = dtype == kBF16 ? f32_to_bf16_bits(x) : f32_to_f16_bits(x);
+}
+
+// x / d for x < 2^31 by the host's precomputed FastDiv of d (scalar: one
+// multiply-high and a shift, where the compiler's division takes ~30
+// dependent instructions, on the path of every wave's first load).
+__device__ __forceinline__ uint32_t fast_div(uint32_t x, const ppk::FastDiv& d) {
+  const uint32_t q = uint32_t((uint64_t(x) * d.mul) >> 32) >> d.shift;
+  return d.mul ? q : x;
+}
+// A zero the compiler takes for a per-lane value: added to a uniform index it
+// makes the load a vector load, which waits in order with the wave's other
+// vector loads. A scalar load of the same word shares its counter with the
+// kernel-argument loads, which can only be waited for all together.
+__device__ __forceinline__ uint32_t lane_zero() {
+  uint32_t z;
+  __asm__("v_mov_b32 %0, 0" : "=v"(z));
+  return z;
 }
 
 // Signed byte k of a dword as float; hipcc folds the sign-extension into an
@@ -721,7 +774,7 @@ __device__ __forceinline__ void quantize_stream_dtype(const ppk::QuantizeArgs& a
 
 
 template <int LPT>
-__device__ __forceinline__ QInt quantize_query(const float (&qr)[16]) {
+__device__ __forceinline__ QInt quantize_query_chunk(const float (&qr)[16]) {
   constexpr float Q = 266338304.0f;  // 127 * 2^21
   float amax = 0.f;
   bool finite = true;
@@ -761,44 +814,160 @@ __device__ __forceinline__ QInt quantize_query(const float (&qr)[16]) {
   return r;
 }
 
+// The query of one wave, from x = channels lane * D/64 ... of q: each lane
+// forms the slices of its own D/64 channels and the wave exchanges them
+// through `region` (LDS of this wave alone, 4 * D bytes, 16-byte aligned), so
+// that every lane ends with the slices of its 16-channel chunk. Quantising
+// the whole chunk in every lane instead, 64/LPT times the same work, was ~380
+// instructions on the critical path of every wave: at two waves per SIMD over
+// 1 us of a launch that takes 4-6 us for short rows.
+template <int D>
+__device__ __forceinline__ QInt quantize_query(const float (&x)[D / ppk::kWave], void* region, int lane) {
+  constexpr float Q = 266338304.0f;  // 127 * 2^21
+  constexpr int EPL = D / ppk::kWave;
+  float amax = 0.f;
+  bool finite = true;
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) {
+    amax = fmaxf(amax, fabsf(x[e]));
+    finite = finite && __builtin_isfinite(x[e]);
+  }
+  amax = wave_max(amax);
+  const bool bad = __any(!finite);
+  const float inv = amax > 0.f ? Q / amax : 0.f;
+  QInt r;
+  r.unscale = bad ? __builtin_nanf("") : amax / Q;
+  uint32_t part[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) {
+    const float v = fminf(fmaxf(rintf(x[e] * inv), -Q), Q);
+    const int qi = finite ? int(v) : 0;
+    const int hi = (qi + (1 << 20)) >> 21;  // [-127, 127]
+    const int r1 = qi - hi * (1 << 21);     // [-2^20, 2^20)
+    const int m1 = (r1 + 8192) >> 14;       // [-64, 64]
+    const int r2 = r1 - m1 * 16384;         // [-8192, 8191]
+    const int m2 = (r2 + 64) >> 7;          // [-64, 64]
+    const int lo = r2 - m2 * 128;           // [-64, 63]
+    part[0] |= (uint32_t(hi) & 0xffu) << (8 * e);
+    part[1] |= (uint32_t(m1) & 0xffu) << (8 * e);
+    part[2] |= (uint32_t(m2) & 0xffu) << (8 * e);
+    part[3] |= (uint32_t(lo) & 0xffu) << (8 * e);
+  }
+  uint8_t* b = static_cast<uint8_t*>(region);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint8_t* to = b + i * D + lane * EPL;
+    if constexpr (EPL == 1) *to = uint8_t(part[i]);
+    else if constexpr (EPL == 2) *reinterpret_cast<u16_alias*>(to) = uint16_t(part[i]);
+    else *reinterpret_cast<u32_alias*>(to) = part[i];
+  }
+  __builtin_amdgcn_wave_barrier();  // LDS serves a wave's accesses in order
+  const u4_alias* from = reinterpret_cast<const u4_alias*>(b + (lane % (D / 16)) * 16);
+  const u4 h = from[0], m1 = from[D / 16], m2 = from[2 * (D / 16)], l = from[3 * (D / 16)];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    r.hi[w] = int(h[w]);
+    r.m1[w] = int(m1[w]);
+    r.m2[w] = int(m2[w]);
+    r.lo[w] = int(l[w]);
+  }
+  __builtin_amdgcn_wave_barrier();
+  return r;
+}
+
+// What phase K needs of the query: the integer slices (fp32 history) or the
+// lane's 16 channels (bf16 history), and the factor of its scores.
+template <bool BF16H>
+struct Query {
+  QInt qi;
+  float qr[16];
+  float sl2;
+};
+template <int D, bool BF16H>
+__device__ __forceinline__ void make_query(const float (&x)[D / ppk::kWave], float scale_log2, void* region, int lane,
+                                           Query<BF16H>& q) {
+  if constexpr (BF16H) {
+    constexpr int EPL = D / ppk::kWave;
+    float* f = static_cast<float*>(region);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) f[lane * EPL + e] = x[e];
+    __builtin_amdgcn_wave_barrier();
+    const float* from = f + (lane % (D / 16)) * 16;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) q.qr[i] = from[i];
+    __builtin_amdgcn_wave_barrier();
+    q.sl2 = scale_log2;
+  } else {
+    q.qi = quantize_query<D>(x, region, lane);
+    q.sl2 = scale_log2 * q.qi.unscale;
+  }
+}
+
+// One tile's K codes against the query: the log2-domain score of the lane
+// group's token (the same in each of its LPT lanes).
+template <int D, bool BF16H>
+__device__ __forceinline__ float tile_score(const u4& raw, float kscale, const Query<BF16H>& q) {
+  constexpr int LPT = D / 16;
+  if constexpr (BF16H) {
+    // pp_i8_load semantics: every element is bf16(code * scale) before the fp32 dot.
+    float d = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (int k = 0; k < 4; k += 2) {
+        float e0, e1;
+        round_bf16_pair(sbyte(raw[w], k) * kscale, sbyte(raw[w], k + 1) * kscale, e0, e1);
+        d = fmaf(q.qr[4 * w + k], e0, d);
+        d = fmaf(q.qr[4 * w + k + 1], e1, d);
+      }
+    return group_sum<LPT>(d) * q.sl2;
+  } else {
+    int sh = 0, s1 = 0, s2 = 0, sl = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      sh = __builtin_amdgcn_sdot4(int(raw[w]), q.qi.hi[w], sh, false);
+      s1 = __builtin_amdgcn_sdot4(int(raw[w]), q.qi.m1[w], s1, false);
+      s2 = __builtin_amdgcn_sdot4(int(raw[w]), q.qi.m2[w], s2, false);
+      sl = __builtin_amdgcn_sdot4(int(raw[w]), q.qi.lo[w], sl, false);
+    }
+    const int hm = group_sum_i32<LPT>(sh * 128 + s1);
+    const int lm = group_sum_i32<LPT>(s2 * 128 + sl);
+    return fmaf(float(hm), 16384.f, float(lm)) * (kscale * q.sl2);
+  }
+}
+
+// One tile's V codes added with weight p (the lane group's token).
+template <bool BF16H>
+__device__ __forceinline__ void tile_accumulate(const u4& raw, float p, float vscale, float (&acc)[16]) {
+  if constexpr (BF16H) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (int k = 0; k < 4; k += 2) {
+        float e0, e1;
+        round_bf16_pair(sbyte(raw[w], k) * vscale, sbyte(raw[w], k + 1) * vscale, e0, e1);
+        acc[4 * w + k] = fmaf(p, e0, acc[4 * w + k]);
+        acc[4 * w + k + 1] = fmaf(p, e1, acc[4 * w + k + 1]);
+      }
+  } else {
+    const float wgt = p * vscale;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[4 * w + k] = fmaf(wgt, sbyte(raw[w], k), acc[4 * w + k]);
+  }
+}
+
 // Phase K for one batch of U tiles: scores (log2 domain) into LDS, running max.
 template <int D, bool BF16H, int U>
 __device__ __forceinline__ float score_batch(const u4 (&raw)[U], float scale_lane, uint32_t t0, uint32_t n, int j,
-                                             int c, const float (&qr)[16], const QInt& qi, float sl2, float* s_lds,
-                                             float mloc) {
+                                             int c, const Query<BF16H>& q, float* s_lds, float mloc) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t tok = (t0 + u) * TPL + j;
-    const float kscale = __shfl(scale_lane, u * TPL + j);
-    float sc;
-    if constexpr (BF16H) {
-      // pp_i8_load semantics: every element is bf16(code * scale) before the fp32 dot.
-      float d = 0.f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-#pragma unroll
-        for (int k = 0; k < 4; k += 2) {
-          float e0, e1;
-          round_bf16_pair(sbyte(raw[u][w], k) * kscale, sbyte(raw[u][w], k + 1) * kscale, e0, e1);
-          d = fmaf(qr[4 * w + k], e0, d);
-          d = fmaf(qr[4 * w + k + 1], e1, d);
-        }
-      sc = group_sum<LPT>(d) * sl2;
-    } else {
-      int sh = 0, s1 = 0, s2 = 0, sl = 0;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        sh = __builtin_amdgcn_sdot4(int(raw[u][w]), qi.hi[w], sh, false);
-        s1 = __builtin_amdgcn_sdot4(int(raw[u][w]), qi.m1[w], s1, false);
-        s2 = __builtin_amdgcn_sdot4(int(raw[u][w]), qi.m2[w], s2, false);
-        sl = __builtin_amdgcn_sdot4(int(raw[u][w]), qi.lo[w], sl, false);
-      }
-      const int hm = group_sum_i32<LPT>(sh * 128 + s1);
-      const int lm = group_sum_i32<LPT>(s2 * 128 + sl);
-      sc = fmaf(float(hm), 16384.f, float(lm)) * (kscale * sl2);
-    }
+    float sc = tile_score<D, BF16H>(raw[u], __shfl(scale_lane, u * TPL + j), q);
     sc = tok < n ? sc : -INFINITY;
     mloc = fmaxf(mloc, sc);
     if (c == 0 && tok < n) s_lds[tok] = sc;
@@ -825,23 +994,8 @@ __device__ __forceinline__ void accumulate_batch(const u4 (&raw)[U], float scale
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const float wgt = __shfl(w_lane, u * TPL + j);
-    if constexpr (BF16H) {
-      const float vscale = __shfl(scale_lane, u * TPL + j);
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-#pragma unroll
-        for (int k = 0; k < 4; k += 2) {
-          float e0, e1;
-          round_bf16_pair(sbyte(raw[u][w], k) * vscale, sbyte(raw[u][w], k + 1) * vscale, e0, e1);
-          acc[4 * w + k] = fmaf(wgt, e0, acc[4 * w + k]);
-          acc[4 * w + k + 1] = fmaf(wgt, e1, acc[4 * w + k + 1]);
-        }
-    } else {
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[4 * w + k] = fmaf(wgt, sbyte(raw[u][w], k), acc[4 * w + k]);
-    }
+    const float vscale = BF16H ? __shfl(scale_lane, u * TPL + j) : 1.f;
+    tile_accumulate<BF16H>(raw[u], wgt, vscale, acc);
   }
 }
 
@@ -856,244 +1010,279 @@ __device__ __forceinline__ float current_score(const ppk::DecodeArgs& a, const f
   return group_sum<D / 16>(d) * a.scale_log2;
 }
 
-// Streams this wave's n tokens (from `begin`) of one row: phase K scores,
-// phase V accumulation. A ring of NB batches (rr[b], rs[b]) keeps NB - 1
-// batches' loads in flight while one is consumed: batch i of the sequence
+// A stream of at most NBATCH batches per phase, K and V already requested:
+// scores, weights and sums stay in the registers of the token groups (no LDS
+// round trip between the phases). Tokens at or past n may hold anything: their
+// scores are masked and their V scales zeroed.
+template <int D, bool BF16H, int NBATCH, int NB>
+__device__ __forceinline__ void short_attention(const u4 (&k)[NB][4], const float (&ks)[NB], const u4 (&v)[2][4],
+                                                const float (&vs)[2], uint32_t n, int lane, const Query<BF16H>& q,
+                                                WavePartial& out) {
+  constexpr int LPT = D / 16;
+  constexpr int TPL = ppk::kWave / LPT;
+  constexpr int TPB = 4 * TPL;
+  const int j = lane / LPT;
+  PPK_CLK_AT(out.t_first, k[0][0][0]);
+  float sc[NBATCH][4], vsc[NBATCH][4];
+  float m = -INFINITY;
+#pragma unroll
+  for (int b = 0; b < NBATCH; ++b) {
+    const float vl = uint32_t(b * TPB + lane % TPB) < n ? vs[b] : 0.f;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) vsc[b][u] = __shfl(vl, u * TPL + j);
+  }
+#pragma unroll
+  for (int b = 0; b < NBATCH; ++b) {
+    float kscale[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) kscale[u] = __shfl(ks[b], u * TPL + j);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float x = tile_score<D, BF16H>(k[b][u], kscale[u], q);
+      sc[b][u] = uint32_t((b * 4 + u) * TPL + j) < n ? x : -INFINITY;
+      m = fmaxf(m, sc[b][u]);
+    }
+  }
+  m = groups_max<LPT>(m);
+  float z = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) out.acc[i] = 0.f;
+#pragma unroll
+  for (int b = 0; b < NBATCH; ++b)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float e = __builtin_amdgcn_exp2f(sc[b][u] - m);
+      const float p = uint32_t((b * 4 + u) * TPL + j) < n ? e : 0.f;
+      z += p;
+      tile_accumulate<BF16H>(v[b][u], p, vsc[b][u], out.acc);
+    }
+  out.m = m;
+  out.z = groups_reduce<LPT>(z, [](float x, float y) { return x + y; });
+  reduce_scatter_groups<LPT, 16>(out.acc, lane);
+}
+
+// Streams this wave's n tokens (n beyond two batches per phase): phase K
+// scores, phase V accumulation. A ring of NB batches (rr[b], rs[b]) keeps NB -
+// 1 batches' loads in flight while one is consumed: batch i of the sequence
 // K_0 .. K_{nb-1}, (padding to a whole ring), V_0 .. V_{nb-1} lives in slot
 // i % NB, and each slot is refilled with batch i + NB as soon as batch i is
 // used, so phase V's first batches are requested during phase K's last ones.
-// Addresses past the end clamp to the last token and those tokens are masked
-// out. With `pre` (nspec beyond the short window) the caller has already
-// issued the first K batches into the ring, clamped to nspec instead of n
-// (tokens at or past n are masked by their scores, so the wider clamp only
-// reads other slots of the same arena row).
+// The caller has issued the first NB K batches, clamped to tokens of the
+// same arena row. Addresses past the end clamp to the last token and those
+// tokens are masked out. Every ring load is issued unconditionally (batches
+// past the end clamp to the row's last token, a cached line) so that each
+// wait is for exactly the oldest batch: a conditional load leaves the
+// compiler's count of loads in flight unknown on one path, and it then waits
+// for all of them (vmcnt(0)), which drains the ring every batch. Only the
+// arithmetic of batches past the end is skipped (uniform branches).
 template <int D, bool BF16H, int NB>
-__device__ __forceinline__ void wave_attention(const ppk::DecodeArgs& a, uint32_t row, uint32_t begin, uint32_t n,
-                                               uint32_t nspec, const float (&qr)[16], float* s_lds, int lane,
-                                               WavePartial& out, bool pre, u4 (&rr)[NB][4], float (&rs)[NB]) {
-  static_assert(NB >= 2, "the short-stream path keeps its K batches in ring slots 0 and 1");
+__device__ __forceinline__ void ring_attention(const uint8_t* kb, const uint8_t* vb, const float* ksb,
+                                               const float* vsb, uint32_t n, const Query<BF16H>& q, float* s_lds,
+                                               int lane, WavePartial& out, u4 (&rr)[NB][4], float (&rs)[NB]) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
   constexpr int U = 4;  // tiles per batch
   const int j = lane / LPT;  // token within a load tile
   const int c = lane % LPT;  // 16-channel chunk
-  out.m = -INFINITY;
-  out.z = 0.f;
 #pragma unroll
   for (int i = 0; i < 16; ++i) out.acc[i] = 0.f;
-
-  const size_t tok0 = size_t(row) * a.capacity + begin;
-  const uint8_t* kb = a.k + tok0 * D + size_t(c) * 16;
-  const uint8_t* vb = a.v + tok0 * D + size_t(c) * 16;
-  const float* ksb = a.ks + tok0;
-  const float* vsb = a.vs + tok0;
-  if (nspec > 0 && nspec <= uint32_t(2 * U * TPL)) {
-    // Short window (at most two batches per phase): K and V are requested
-    // before the row's length is known, clamped to the window's slots inside
-    // the arena (always in bounds); slots at or past the length n are masked
-    // below and their scales zeroed, so stale or uninitialised arena memory
-    // never reaches the result.
-    const bool two = nspec > uint32_t(U * TPL);  // uniform per wave
-    u4 ka[U], kb2[U], va[U], vb2[U];
-    float ksa, ksb2, vsa, vsb2;
-    load_batch<D, U>(kb, ksb, 0, nspec, j, lane, ka, ksa);
-    load_batch<D, U>(vb, vsb, 0, nspec, j, lane, va, vsa);
-    if (two) {
-      load_batch<D, U>(kb, ksb, U, nspec, j, lane, kb2, ksb2);
-      load_batch<D, U>(vb, vsb, U, nspec, j, lane, vb2, vsb2);
+  float mloc = -INFINITY, z = 0.f;
+  const uint32_t nb = ((n + TPL - 1) / TPL + U - 1) / U;  // K batches (and V batches)
+  const uint32_t nbp = (nb + NB - 1) / NB * NB;           // rounded up to whole rings
+  PPK_CLK_AT(out.t_first, rr[0][0][0]);
+  for (uint32_t k0 = 0; k0 < nbp; k0 += NB) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const uint32_t i = k0 + uint32_t(b);
+      if (i < nb) mloc = score_batch<D, BF16H, U>(rr[b], rs[b], i * U, n, j, c, q, s_lds, mloc);
+      // Refill slot b with item i + NB: K batch i + NB, or V batch i + NB - nbp.
+      const bool isv = i + NB >= nbp;
+      load_batch<D, U>(isv ? vb : kb, isv ? vsb : ksb, (isv ? i + NB - nbp : i + NB) * U, n, j, lane, rr[b],
+                       rs[b]);
     }
-    QInt qi{};
-    float sl2 = a.scale_log2;
-    if constexpr (!BF16H) {
-      qi = quantize_query<LPT>(qr);
-      sl2 *= qi.unscale;
-    }
-    if (n == 0) return;  // uniform per wave
-    PPK_CLK_AT(out.t_first, ka[0][0]);
-    const uint32_t tl = uint32_t(lane % (U * TPL));
-    ksa = tl < n ? ksa : 0.f;
-    vsa = tl < n ? vsa : 0.f;
-    float mloc = -INFINITY;
-    mloc = score_batch<D, BF16H, U>(ka, ksa, 0, n, j, c, qr, qi, sl2, s_lds, mloc);
-    if (two) {
-      ksb2 = U * TPL + tl < n ? ksb2 : 0.f;
-      vsb2 = U * TPL + tl < n ? vsb2 : 0.f;
-      mloc = score_batch<D, BF16H, U>(kb2, ksb2, U, n, j, c, qr, qi, sl2, s_lds, mloc);
-    }
-    float m = mloc, z = 0.f;
-    m = groups_max<LPT>(m);
-    __builtin_amdgcn_wave_barrier();
-    accumulate_batch<D, BF16H, U>(va, vsa, 0, n, j, lane, m, s_lds, z, out.acc);
-    if (two) accumulate_batch<D, BF16H, U>(vb2, vsb2, U, n, j, lane, m, s_lds, z, out.acc);
-    z = wave_sum(z);
-    reduce_scatter_groups<LPT, 16>(out.acc, lane);
-    out.m = m;
-    out.z = z;
-    return;
   }
-  if (n == 0) return;  // uniform per wave
-  const uint32_t ntiles = (n + TPL - 1) / TPL;
-  float mloc = -INFINITY;
-  float m, z = 0.f;
-  QInt qi{};
-  float sl2 = a.scale_log2;
-  if (ntiles <= 2 * U) {
-    // Short stream (at most two batches per phase, e.g. many small splits of
-    // short rows): K and V of the whole wave are requested together, so the
-    // wave waits on one memory round trip instead of a K trip and a V trip.
-    const bool two = ntiles > U;  // uniform per wave
-    u4 va[U], vb2[U];
-    float vsa, vsb2;
-    if (!pre) load_batch<D, U>(kb, ksb, 0, n, j, lane, rr[0], rs[0]);
-    load_batch<D, U>(vb, vsb, 0, n, j, lane, va, vsa);
-    if (two) {
-      if (!pre) load_batch<D, U>(kb, ksb, U, n, j, lane, rr[1], rs[1]);
-      load_batch<D, U>(vb, vsb, U, n, j, lane, vb2, vsb2);
-    }
-    if constexpr (!BF16H) {
-      qi = quantize_query<LPT>(qr);
-      sl2 *= qi.unscale;
-    }
-    PPK_CLK_AT(out.t_first, rr[0][0][0]);
-    mloc = score_batch<D, BF16H, U>(rr[0], rs[0], 0, n, j, c, qr, qi, sl2, s_lds, mloc);
-    if (two) mloc = score_batch<D, BF16H, U>(rr[1], rs[1], U, n, j, c, qr, qi, sl2, s_lds, mloc);
-    m = mloc;
-    m = groups_max<LPT>(m);
-    __builtin_amdgcn_wave_barrier();
-    accumulate_batch<D, BF16H, U>(va, vsa, 0, n, j, lane, m, s_lds, z, out.acc);
-    if (two) accumulate_batch<D, BF16H, U>(vb2, vsb2, U, n, j, lane, m, s_lds, z, out.acc);
-  } else {
-    // The first K batches do not depend on q: issue them before the query is
-    // quantised, so the q load and its reductions overlap the first memory
-    // round trip. Every ring load is issued unconditionally (batches past the
-    // end clamp to the row's last token, a cached line) so that each wait is
-    // for exactly the oldest batch: a conditional load leaves the compiler's
-    // count of loads in flight unknown on one path, and it then waits for
-    // all of them (vmcnt(0)), which drains the ring every batch. Only the
-    // arithmetic of batches past the end is skipped (uniform branches).
-    const uint32_t nb = (ntiles + U - 1) / U;       // K batches (and V batches)
-    const uint32_t nbp = (nb + NB - 1) / NB * NB;   // rounded up to whole rings
-    if (!pre) {
+  const float m = groups_max<LPT>(mloc);
+  __builtin_amdgcn_wave_barrier();
+  for (uint32_t v0 = 0; v0 < nbp; v0 += NB) {
 #pragma unroll
-      for (int b = 0; b < NB; ++b) load_batch<D, U>(kb, ksb, uint32_t(b) * U, n, j, lane, rr[b], rs[b]);
-    }
-    if constexpr (!BF16H) {
-      qi = quantize_query<LPT>(qr);
-      sl2 *= qi.unscale;
-    }
-    PPK_CLK_AT(out.t_first, rr[0][0][0]);
-    for (uint32_t k0 = 0; k0 < nbp; k0 += NB) {
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const uint32_t i = k0 + uint32_t(b);
-        if (i < nb) mloc = score_batch<D, BF16H, U>(rr[b], rs[b], i * U, n, j, c, qr, qi, sl2, s_lds, mloc);
-        // Refill slot b with item i + NB: K batch i + NB, or V batch i + NB - nbp.
-        const bool isv = i + NB >= nbp;
-        load_batch<D, U>(isv ? vb : kb, isv ? vsb : ksb, (isv ? i + NB - nbp : i + NB) * U, n, j, lane, rr[b],
-                         rs[b]);
-      }
-    }
-    m = mloc;
-    m = groups_max<LPT>(m);
-    __builtin_amdgcn_wave_barrier();
-    for (uint32_t v0 = 0; v0 < nbp; v0 += NB) {
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const uint32_t i = v0 + uint32_t(b);
-        if (i < nb) accumulate_batch<D, BF16H, U>(rr[b], rs[b], i * U, n, j, lane, m, s_lds, z, out.acc);
-        load_batch<D, U>(vb, vsb, (i + NB) * U, n, j, lane, rr[b], rs[b]);  // past the end on the last ring
-      }
+    for (int b = 0; b < NB; ++b) {
+      const uint32_t i = v0 + uint32_t(b);
+      if (i < nb) accumulate_batch<D, BF16H, U>(rr[b], rs[b], i * U, n, j, lane, m, s_lds, z, out.acc);
+      load_batch<D, U>(vb, vsb, (i + NB) * U, n, j, lane, rr[b], rs[b]);  // past the end on the last ring
     }
   }
   // Each token's p was added once, by its owning lane: sum over the wave.
-  z = wave_sum(z);
-  reduce_scatter_groups<LPT, 16>(out.acc, lane);
   out.m = m;
-  out.z = z;
+  out.z = wave_sum(z);
+  reduce_scatter_groups<LPT, 16>(out.acc, lane);
 }
 
 template <int D, bool BF16H, int NB>
 __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   constexpr int LPT = D / 16;
+  constexpr int TPL = ppk::kWave / LPT;
+  constexpr int U = 4;  // tiles per batch
   constexpr int EPL = D / ppk::kWave;
+  static_assert(NB >= 2, "a short stream keeps its K batches in ring slots 0 and 1");
   PPK_CLK_DECL;
   PPK_CLK(0);
-  extern __shared__ float lds[];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  // The arguments on the way to the first loads, requested together (the
+  // compiler would load each where it is first used, one round trip after
+  // another).
+  __asm__ volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.ks), "s"(a.vs), "s"(a.sk), "s"(a.sv), "s"(a.past),
+                   "s"(a.k_new), "s"(a.v_new), "s"(a.rows), "s"(a.capacity), "s"(a.split_tokens), "s"(a.ngroups),
+                   "s"(a.q_dtype), "s"(a.scratch_dtype), "s"(a.new_dtype), "s"(a.append), "s"(a.speculate),
+                   "s"(a.row_div.mul), "s"(a.row_div.shift), "s"(a.head_div.mul), "s"(a.head_div.shift),
+                   "s"(blockDim.x));
   const int lane = threadIdx.x & 63;
   // The wave index is uniform: in a scalar register, every quantity derived
   // from it (the wave's range, its length, its batch counts) is too, and the
   // stream's loop and batch conditions become scalar branches.
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int W = blockDim.x >> 6;
+  const int j = lane / LPT;
   const int c = lane % LPT;
   // Blocks are numbered group-major: consecutive blocks belong to different
   // rows, so the empty tail groups of short rows (ragged batches) spread over
   // the CUs instead of leaving some CUs with only live blocks.
-  const uint32_t row = blockIdx.x % a.rows;
-  const uint32_t group = blockIdx.x / a.rows;
+  const uint32_t group = fast_div(blockIdx.x, a.row_div);
+  const uint32_t row = blockIdx.x - group * a.rows;
   const uint32_t S = a.split_tokens;
-  const uint32_t p = a.past[row / a.heads];
-  const uint64_t cover = uint64_t(a.ngroups) * W * S;
-  const bool valid = p <= a.capacity && uint64_t(p) <= cover;
 
-  // Everything the wave reads before its stream is requested first, in one
-  // round trip: q, the current token (wave 0 of a block that covers its
-  // row), the new K/V row of the fused commit (waves 0 and 1 of group 0) and
-  // the stream's first two K batches, clamped to the arena (not to the
-  // row's length, which arrives with them). The commit and the current
-  // token's score then run while the K batches are in flight. Measured at
-  // B=32 x 8192 tokens against committing first and loading the stream after
-  // the length: D=64 94.8 -> 91.6 us, D=128 165.5 -> 165.0 us, bitwise the
-  // same output. The slot the commit writes is past every wave's length, so
-  // the speculative reads of it are masked. The host turns this off (a.speculate
-  // = 0) when it knows many waves have no history (ragged host lengths, or
-  // waves past the span): their speculative reads would be wasted bandwidth
-  // (config 4: 9 % more HBM traffic than the history, 18.7 -> 18.3 us without).
-  float qr[16];
-  load_vec<16>(a.q, size_t(row) * D + size_t(c) * 16, a.q_dtype, qr);
+  // Everything the wave reads is requested first, in one round trip: the
+  // row's length, q, the current token (wave 0 of a block that covers its
+  // row), the new K/V row of the fused commit (waves 0 and 1 of group 0), all
+  // as raw words, and the stream's first batches, clamped to the arena (not
+  // to the row's length, which arrives with them; the tokens past it are
+  // masked). The commit, the current token's score and the query's slices
+  // are then formed while the batches are in flight. What bounds short rows
+  // is this chain of round trips, not bytes; with the small operands widened
+  // where they were loaded (each load waited for before the next), the row's
+  // length and late kernel arguments read in between and the query quantised
+  // by every lane group: H = 16, 512 tokens f32 at D = 64 5.88 us, now 4.43;
+  // 24 layers of 2048 tokens at D = 128 204.8, now 187.8; B = 16 x 1500 at D =
+  // 64 11.16, now 10.62; B = 32 x 8192 unchanged (162.2). The slot the commit
+  // writes is past every wave's length, so the speculative reads of it are
+  // masked. The host turns the early batches off (a.speculate = 0) when it
+  // knows many waves have no history (ragged host lengths, or waves past the
+  // span): their speculative reads would be wasted bandwidth (config 4: 9 %
+  // more HBM traffic than the history, 18.7 -> 18.3 us without).
+  const uint32_t p_raw = a.past[fast_div(row, a.head_div) + lane_zero()];
   const bool final_out = a.ngroups == 1;
-  float s_cur = -INFINITY;
-  float sv[EPL], kv[16];
-  if (final_out && wave == 0) {
-    load_vec<16>(a.sk, size_t(row) * D + size_t(c) * 16, a.scratch_dtype, kv);
-    load_vec<EPL>(a.sv, size_t(row) * D + size_t(lane) * EPL, a.scratch_dtype, sv);
-  }
+  const bool cur = final_out && wave == 0;
   const bool kw = a.append && group == 0 && wave == 0;
   const bool vw = a.append && group == 0 && wave == (W > 1 ? 1 : 0);
-  float kx[EPL], vx[EPL];
-  if (kw) load_vec<EPL>(a.k_new, size_t(row) * D + size_t(lane) * EPL, a.new_dtype, kx);
-  if (vw) load_vec<EPL>(a.v_new, size_t(row) * D + size_t(lane) * EPL, a.new_dtype, vx);
+  const size_t first = size_t(row) * D + size_t(lane) * EPL;
+  RawVec<EPL> q_raw, sk_raw, sv_raw, kn_raw, vn_raw;
+  load_raw<EPL>(a.q, first, a.q_dtype, q_raw);
+  if (cur) {
+    load_raw<EPL>(a.sk, first, a.scratch_dtype, sk_raw);
+    load_raw<EPL>(a.sv, first, a.scratch_dtype, sv_raw);
+  }
+  if (kw) load_raw<EPL>(a.k_new, first, a.new_dtype, kn_raw);
+  if (vw) load_raw<EPL>(a.v_new, first, a.new_dtype, vn_raw);
+
   const uint32_t begin = (group * W + wave) * S;
   const uint32_t nspec = (a.speculate && begin < a.capacity) ? min(S, a.capacity - begin) : 0u;
-  constexpr int TPL = ppk::kWave / LPT;
-  const bool pre = nspec > uint32_t(8 * TPL);  // the wave takes a streamed (not short-window) path
-  u4 rr[NB][4];
-  float rs[NB];
-  if (pre) {
-    const size_t tok0 = size_t(row) * a.capacity + begin;
-    const int j = lane / LPT;
+  const size_t tok0 = size_t(row) * a.capacity + begin;
+  const uint8_t* kb = a.k + tok0 * D + size_t(c) * 16;
+  const uint8_t* vb = a.v + tok0 * D + size_t(c) * 16;
+  const float* ksb = a.ks + tok0;
+  const float* vsb = a.vs + tok0;
+  // LDS of this wave alone: the query's exchange, then a score per token of
+  // its range, at last its (m, z, pad, pad, y[D]) record.
+  const uint32_t lds_stride = max(S, uint32_t(D + 4));
+  float* s_lds = lds + size_t(wave) * lds_stride;
+
+  float s_cur = -INFINITY, sv[EPL];
+  bool valid = false;
+  uint32_t n = 0;
+  Query<BF16H> query;
+  // Everything that waits for the small loads; runs with the stream's first
+  // batches in flight.
+  auto prologue = [&]() {
+    PPK_CLK(1);
+    const uint32_t p = __builtin_amdgcn_readfirstlane(p_raw);
+    PPK_CLK_AFTER(2, p_raw);
+    const uint64_t cover = uint64_t(a.ngroups) * W * S;
+    valid = p <= a.capacity && uint64_t(p) <= cover;
+    n = (valid && begin < p) ? min(S, p - begin) : 0u;
+    float x[EPL];
+    widen<EPL>(q_raw, a.q_dtype, x);
+    if (n > 0) make_query<D, BF16H>(x, a.scale_log2, s_lds, lane, query);
+    if (cur) {
+      // Log2-domain score of the current token, which comes from the scratch copy, not the arena.
+      float kv[EPL], d = 0.f;
+      widen<EPL>(sk_raw, a.scratch_dtype, kv);
+      widen<EPL>(sv_raw, a.scratch_dtype, sv);
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-      load_batch<D, 4>(a.k + tok0 * D + size_t(c) * 16, a.ks + tok0, uint32_t(b) * 4, nspec, j, lane, rr[b], rs[b]);
-  }
-  PPK_CLK(1);
-  // A length within the caller's span that the plan does not cover: the plan
-  // was sized from a stale host copy of the lengths (the row gives NaN).
-  if (kw && lane == 0 && a.flags && p <= a.capacity && p <= a.span && uint64_t(p) > cover) atomicOr(a.flags, 4u);
-  if (kw || vw) {
-    if (p >= a.capacity) {
-      if (lane == 0 && a.flags) atomicOr(a.flags, 2u);
+      for (int e = 0; e < EPL; ++e) d = fmaf(x[e], kv[e], d);
+      s_cur = wave_sum(d) * a.scale_log2;
+    }
+    // A length within the caller's span that the plan does not cover: the plan
+    // was sized from a stale host copy of the lengths (the row gives NaN).
+    if (kw && lane == 0 && a.flags && p <= a.capacity && p <= a.span && uint64_t(p) > cover) atomicOr(a.flags, 4u);
+    if (kw || vw) {
+      if (p >= a.capacity) {
+        if (lane == 0 && a.flags) atomicOr(a.flags, 2u);
+      } else {
+        const size_t slot = size_t(row) * a.capacity + p;
+        float t[EPL];
+        if (kw) {
+          widen<EPL>(kn_raw, a.new_dtype, t);
+          quantize_values<D>(t, a.k + slot * D, a.ks + slot, a.flags, lane);
+        }
+        if (vw) {
+          widen<EPL>(vn_raw, a.new_dtype, t);
+          quantize_values<D>(t, a.v + slot * D, a.vs + slot, a.flags, lane);
+        }
+      }
+    }
+  };
+
+  WavePartial part;
+  part.m = -INFINITY;
+  part.z = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) part.acc[i] = 0.f;
+  u4 rr[NB][U], va[2][U];
+  float rs[NB], vsa[2];
+  // The paths differ in what is in flight when the prologue runs; each runs
+  // its own copy of it, so that its waits count that path's loads only.
+  if (nspec > 0 && nspec <= uint32_t(U * TPL)) {
+    // A window of one batch: K and V at once, one memory round trip in all.
+    load_batch<D, U>(kb, ksb, 0, nspec, j, lane, rr[0], rs[0]);
+    load_batch<D, U>(vb, vsb, 0, nspec, j, lane, va[0], vsa[0]);
+    prologue();
+    if (n > 0) short_attention<D, BF16H, 1>(rr, rs, va, vsa, n, lane, query, part);
+  } else if (nspec > 0 && nspec <= uint32_t(2 * U * TPL)) {
+    load_batch<D, U>(kb, ksb, 0, nspec, j, lane, rr[0], rs[0]);
+    load_batch<D, U>(kb, ksb, U, nspec, j, lane, rr[1], rs[1]);
+    load_batch<D, U>(vb, vsb, 0, nspec, j, lane, va[0], vsa[0]);
+    load_batch<D, U>(vb, vsb, U, nspec, j, lane, va[1], vsa[1]);
+    prologue();
+    if (n > 0) short_attention<D, BF16H, 2>(rr, rs, va, vsa, n, lane, query, part);
+  } else {
+    if (nspec > 0) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) load_batch<D, U>(kb, ksb, uint32_t(b) * U, nspec, j, lane, rr[b], rs[b]);
+      prologue();
     } else {
-      const size_t slot = size_t(row) * a.capacity + p;
-      if (kw) quantize_values<D>(kx, a.k + slot * D, a.ks + slot, a.flags, lane);
-      if (vw) quantize_values<D>(vx, a.v + slot * D, a.vs + slot, a.flags, lane);
+      prologue();
+      if (n > 0) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) load_batch<D, U>(kb, ksb, uint32_t(b) * U, n, j, lane, rr[b], rs[b]);
+      }
+    }
+    if (n > uint32_t(2 * U * TPL)) {
+      ring_attention<D, BF16H, NB>(kb, vb, ksb, vsb, n, query, s_lds, lane, part, rr, rs);
+    } else if (n > 0) {
+      load_batch<D, U>(vb, vsb, 0, n, j, lane, va[0], vsa[0]);
+      load_batch<D, U>(vb, vsb, U, n, j, lane, va[1], vsa[1]);
+      short_attention<D, BF16H, 2>(rr, rs, va, vsa, n, lane, query, part);
     }
   }
-  if (final_out && wave == 0) s_cur = current_score<D>(a, kv, qr);
-  PPK_CLK_AFTER(2, p);
-  const uint32_t n = (valid && begin < p) ? min(S, p - begin) : 0u;
-  WavePartial part;
-  wave_attention<D, BF16H, NB>(a, row, begin, n, nspec, qr, lds + size_t(wave) * S, lane, part, pre, rr, rs);
   PPK_CLK(4);
 #ifdef PPK_WAVE_CLOCK
   clk_[3] = part.t_first;
@@ -1402,7 +1591,7 @@ __device__ __forceinline__ void wave_attention_window(const ppk::DecodeArgs& a, 
   QInt qi{};
   float sl2 = a.scale_log2;
   if constexpr (!BF16H) {
-    qi = quantize_query<LPT>(qr);
+    qi = quantize_query_chunk<LPT>(qr);
     sl2 *= qi.unscale;
   }
   early();
