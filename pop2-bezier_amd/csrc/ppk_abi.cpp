@@ -866,6 +866,7 @@ void run_attention(ppk_context* ctx, hipStream_t stream, const PpkAttentionArgs&
     m.m.out = a.out;
     m.m.rows = a.rows;
     m.m.heads = a.heads;
+    m.m.head_div = d.head_div;
     m.m.capacity = a.capacity;
     m.m.split_tokens = plan.split;
     m.m.nsplits = plan.ngroups;
@@ -896,6 +897,7 @@ void run_attention(ppk_context* ctx, hipStream_t stream, const PpkAttentionArgs&
     m.out = a.out;
     m.rows = a.rows;
     m.heads = a.heads;
+    m.head_div = d.head_div;
     m.capacity = a.capacity;
     m.split_tokens = plan.split * plan.waves;  // tokens per group
     m.nsplits = plan.ngroups;
@@ -1056,6 +1058,7 @@ void run_float_attention(ppk_context* ctx, hipStream_t stream, const PpkFloatAtt
   m.out = a.out;
   m.rows = a.rows;
   m.heads = a.heads;
+  m.head_div = fast_divisor(a.heads);
   m.size = a.size;
   m.nsplits = plan.ngroups;
   m.out_dtype = a.out_dtype;

@@ -132,6 +132,7 @@ struct MergeArgs {
   uint32_t q_dtype, scratch_dtype, out_dtype;
   float scale_log2;
   uint32_t span;            // rows with past[b] > span give NaN (balanced plan)
+  FastDiv head_div;         // by heads
   uint32_t clock_seq;       // wave-clock builds only, as in DecodeArgs
   uint32_t clock_cap;
   uint64_t* clock;
@@ -212,6 +213,7 @@ struct FloatMergeArgs {
   uint32_t rows, heads, size, split_tokens, nsplits, out_dtype, span;
   uint32_t step, q_dtype, new_dtype, kv_bf16;
   float scale_log2;
+  FastDiv head_div;         // by heads
 };
 
 // Float-KV decode over the balanced work list: the table as for the int8

@@ -88,12 +88,6 @@ enum { kF32 = 0, kBF16 = 1, kF16 = 2 };
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float(uint32_t(h) << 16); }
 __device__ __forceinline__ float f16_to_f32(uint16_t h) { return float(__builtin_bit_cast(_Float16, h)); }
 
-__device__ __forceinline__ float load_elem(const void* p, size_t i, uint32_t dtype) {
-  if (dtype == kF32) return static_cast<const float*>(p)[i];
-  const uint16_t h = static_cast<const uint16_t*>(p)[i];
-  return dtype == kBF16 ? bf16_to_f32(h) : f16_to_f32(h);
-}
-
 // N consecutive elements starting at element i, widened to f32: one dtype
 // branch, then N independent loads in flight together.
 template <int N>
@@ -1117,6 +1111,65 @@ __device__ __forceinline__ void ring_attention(const uint8_t* kb, const uint8_t*
   reduce_scatter_groups<LPT, 16>(out.acc, lane);
 }
 
+// A wave's record for its block: m, z, two pad floats, y[D] (16-byte aligned)
+// at `rec`; this lane holds the totals of channels ch .. ch + D/64 - 1.
+template <int D, int N>
+__device__ __forceinline__ void write_block_record(float* rec, int ch, int lane, float m, float z,
+                                                   const float (&acc)[N]) {
+#pragma unroll
+  for (int e = 0; e < D / ppk::kWave; ++e) rec[4 + ch + e] = acc[e];
+  if (lane == 0) {
+    rec[0] = m;
+    rec[1] = z;
+  }
+}
+
+// Log-sum-exp combine of a block's W <= MAXW records (stride floats apart) and
+// a score s0 that joins the maximum (-inf for none), by one wave: lane w takes
+// record w's (m, z), the y rows of this lane's channels are requested eight
+// records at a time (past W: the last record again, with weight 0). One LDS
+// round trip for the weights and one for the rows; a loop over the records
+// took two per record, ~0.7 us at the end of every 8-wave block.
+template <int D, int MAXW>
+__device__ __forceinline__ void combine_block(const float* recs, uint32_t stride, uint32_t W, int lane, float s0,
+                                              float& m, float& z, float (&y)[D / ppk::kWave]) {
+  constexpr int EPL = D / ppk::kWave;
+  const float* mine = recs + min(uint32_t(lane), W - 1) * stride;
+  float mw = mine[0], zw = mine[1];
+  float v[8][EPL];
+  auto rows = [&](uint32_t w0) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) v[k][e] = recs[min(w0 + uint32_t(k), W - 1) * stride + 4 + lane * EPL + e];
+  };
+  rows(0);
+  if (uint32_t(lane) >= W) {
+    mw = -INFINITY;
+    zw = 0.f;
+  }
+  m = fmaxf(wave_max(mw), s0);
+  const float wt = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - m);
+  z = wave_sum(wt * zw);
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) y[e] = 0.f;
+  auto add = [&](uint32_t w0) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wt), int(w0) + k));
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) y[e] = fmaf(wk, v[k][e], y[e]);
+    }
+  };
+  add(0);
+  if constexpr (MAXW > 8) {
+    if (W > 8) {  // uniform
+      rows(8);
+      add(8);
+    }
+  }
+}
+
 template <int D, bool BF16H, int NB>
 __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   constexpr int LPT = D / 16;
@@ -1288,20 +1341,9 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   clk_[3] = part.t_first;
 #endif
 
-  // Combine the block's waves through LDS (the staging area is reused).
-  // Record of wave w at mrg + w * R: m, z, 2 pad floats, y[D] (16-byte aligned).
-  constexpr int R = D + 4;
-  __syncthreads();
-  float* mrg = lds;
-  {
-    const int ch = c * 16 + scatter_base<LPT, 16>(lane);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) mrg[wave * R + 4 + ch + e] = part.acc[e];
-  }
-  if (lane == 0) {
-    mrg[wave * R] = part.m;
-    mrg[wave * R + 1] = part.z;
-  }
+  // Combine the block's waves through LDS: each wave's record replaces its
+  // scores (its own LDS, so no barrier is needed before).
+  write_block_record<D>(s_lds, c * 16 + scatter_base<LPT, 16>(lane), lane, part.m, part.z, part.acc);
   __syncthreads();
   PPK_CLK(5);
   if (wave != 0) {
@@ -1309,17 +1351,8 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
     return;
   }
 
-  float m = s_cur;
-  for (int w = 0; w < W; ++w) m = fmaxf(m, mrg[w * R]);
-  float y[EPL], zsum = 0.f;
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) y[e] = 0.f;
-  for (int w = 0; w < W; ++w) {
-    const float wt = mrg[w * R] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mrg[w * R] - m);
-    zsum = fmaf(wt, mrg[w * R + 1], zsum);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) y[e] = fmaf(wt, mrg[w * R + 4 + lane * EPL + e], y[e]);
-  }
+  float m, y[EPL], zsum;
+  combine_block<D, 8>(lds, lds_stride, uint32_t(W), lane, s_cur, m, zsum, y);
   if (final_out) {
     const float wc = __builtin_amdgcn_exp2f(s_cur - m);
     zsum += wc;
@@ -1347,21 +1380,25 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
 // Rows with past > capacity (or beyond the launched coverage) give NaN.
 // ---------------------------------------------------------------------------
 // Log-sum-exp combine of one row's `nsplits` partial records, one wave: the
-// combined max m (at least m0), the sum z of 2^(m_s - m) z_s, and y for this
-// lane's D/64 channels, sum_s 2^(m_s - m) y_s, added in split order. Lane s
-// loads record s's (m, z); the y rows load eight splits at a time with all
-// eight loads issued before the first use, so the chain costs one memory
-// round trip per eight splits instead of one per split.
-template <int D, class CurrentScore>
+// combined max m, the sum z of 2^(m_s - m) z_s, and y for this lane's D/64
+// channels, sum_s 2^(m_s - m) y_s, added in split order. Lane s loads record
+// s's (m, z); the y rows load eight splits at a time with all eight loads
+// issued before the first use, so the chain costs one memory round trip per
+// eight splits instead of one per split. request() issues whatever else the
+// caller loads (as raw words: nothing in it may wait), score() then returns
+// the extra score that joins the max (-inf for none).
+template <int D, class Request, class Score>
 __device__ __forceinline__ void combine_records(const float* mz, const float* py, uint32_t nsplits, int lane,
-                                                CurrentScore current_score, float& m, float& z,
+                                                Request request, Score score, float& m, float& z,
                                                 float (&y)[D / ppk::kWave]) {
   constexpr int EPL = D / ppk::kWave;
   // Everything that does not depend on the max is requested first, in one
-  // round trip: the y rows of the first sixteen splits, the (m, z) pairs of
-  // the first 64 splits (kept in registers for the weights), and then
-  // whatever current_score() loads before it returns the extra score that
-  // joins the max (-inf for none).
+  // round trip, in the order of use: the (m, z) pairs of the first 64 splits
+  // (kept in registers for the weights), the caller's operands, the y rows of
+  // the first sixteen splits.
+  const uint32_t s_first = min(uint32_t(lane), nsplits - 1);
+  float m_first = mz[2 * s_first], z_first = mz[2 * s_first + 1];
+  request();
   float first[16][EPL];
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
@@ -1369,13 +1406,13 @@ __device__ __forceinline__ void combine_records(const float* mz, const float* py
 #pragma unroll
     for (int e = 0; e < EPL; ++e) first[k][e] = py[size_t(si) * D + size_t(lane) * EPL + e];
   }
-  const uint32_t s_first = min(uint32_t(lane), nsplits - 1);
-  const float m_first = uint32_t(lane) < nsplits ? mz[2 * s_first] : -INFINITY;
-  const float z_first = uint32_t(lane) < nsplits ? mz[2 * s_first + 1] : 0.f;
+  if (uint32_t(lane) >= nsplits) {
+    m_first = -INFINITY;
+    z_first = 0.f;
+  }
   float mm = m_first;
   for (uint32_t s = lane + ppk::kWave; s < nsplits; s += ppk::kWave) mm = fmaxf(mm, mz[2 * s]);
-  mm = fmaxf(mm, current_score());
-  m = wave_max(mm);
+  m = fmaxf(wave_max(mm), score());
   z = 0.f;
 #pragma unroll
   for (int e = 0; e < EPL; ++e) y[e] = 0.f;
@@ -1418,43 +1455,60 @@ __device__ __forceinline__ void combine_records(const float* mz, const float* py
   z = wave_sum(z);
 }
 
+// The current token of an int8 merge: q, sk and sv of one row as raw words,
+// then the log2-domain score q . sk (sv widened beside it).
+template <int D>
+struct MergeCurrent {
+  static constexpr int EPL = D / ppk::kWave;
+  RawVec<EPL> q, sk, sv_raw;
+  float sv[EPL], s_cur;
+  __device__ __forceinline__ void request(const ppk::MergeArgs& a, size_t base) {
+    load_raw<EPL>(a.q, base, a.q_dtype, q);
+    load_raw<EPL>(a.sk, base, a.scratch_dtype, sk);
+    load_raw<EPL>(a.sv, base, a.scratch_dtype, sv_raw);
+  }
+  __device__ __forceinline__ float score(const ppk::MergeArgs& a) {
+    float qv[EPL], kv[EPL], d = 0.f;
+    widen<EPL>(q, a.q_dtype, qv);
+    widen<EPL>(sk, a.scratch_dtype, kv);
+    widen<EPL>(sv_raw, a.scratch_dtype, sv);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) d = fmaf(qv[e], kv[e], d);
+    s_cur = wave_sum(d) * a.scale_log2;
+    return s_cur;
+  }
+};
+
 template <int D>
 __device__ __forceinline__ void attn_merge_body(const ppk::MergeArgs& a) {
   constexpr int EPL = D / ppk::kWave;
   PPK_CLK_DECL;
   PPK_CLK(0);
+  // Every argument on the way to the loads, requested together.
+  __asm__ volatile("" ::"s"(a.q), "s"(a.sk), "s"(a.sv), "s"(a.past), "s"(a.part_y), "s"(a.part_mz), "s"(a.out),
+                   "s"(a.capacity), "s"(a.split_tokens), "s"(a.nsplits), "s"(a.q_dtype), "s"(a.scratch_dtype),
+                   "s"(a.out_dtype), "s"(a.scale_log2), "s"(a.head_div.mul), "s"(a.head_div.shift));
   const int lane = threadIdx.x;
   const uint32_t row = blockIdx.x;
-
-  float sv[EPL];
-  float s_cur = -INFINITY;
   const size_t base = size_t(row) * D + size_t(lane) * EPL;
-  // The current token (q . sk, and sv): loaded after the records are requested.
-  auto current = [&]() {
-    float qv[EPL], kv[EPL];
-    load_vec<EPL>(a.q, base, a.q_dtype, qv);
-    load_vec<EPL>(a.sk, base, a.scratch_dtype, kv);
-    load_vec<EPL>(a.sv, base, a.scratch_dtype, sv);
-    float d = 0.f;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) d = fmaf(qv[e], kv[e], d);
-    s_cur = wave_sum(d) * a.scale_log2;
-    return s_cur;
+  // The row's length travels with the records (as a vector load, see lane_zero).
+  MergeCurrent<D> cur;
+  uint32_t p_raw = 0;
+  auto request = [&]() {
+    cur.request(a, base);
+    p_raw = a.past[fast_div(row, a.head_div) + lane_zero()];
   };
   float m, zsum, y[EPL];
   combine_records<D>(a.part_mz + size_t(row) * a.nsplits * 2, a.part_y + size_t(row) * a.nsplits * D, a.nsplits,
-                     lane, current, m, zsum, y);
+                     lane, request, [&]() { return cur.score(a); }, m, zsum, y);
   PPK_CLK_AFTER(1, y[0]);
-  // The row's length is first needed here: read after the records went out
-  // (deciding validity up front would hold every record load back by the
-  // length's round trip).
-  const uint32_t p = a.past[row / a.heads];
+  const uint32_t p = __builtin_amdgcn_readfirstlane(p_raw);
   const bool valid = p <= a.capacity && uint64_t(p) <= uint64_t(a.nsplits) * a.split_tokens;
-  const float wc = __builtin_amdgcn_exp2f(s_cur - m);
+  const float wc = __builtin_amdgcn_exp2f(cur.s_cur - m);
   zsum += wc;
 #pragma unroll
   for (int e = 0; e < EPL; ++e) {
-    const float o = valid ? fmaf(wc, sv[e], y[e]) / zsum : __builtin_nanf("");
+    const float o = valid ? fmaf(wc, cur.sv[e], y[e]) / zsum : __builtin_nanf("");
     store_elem(a.out, base + e, a.out_dtype, o);
   }
   PPK_CLK(2);
@@ -1747,34 +1801,23 @@ __device__ __forceinline__ void attn_merge_flat_body(const ppk::MergeFlatArgs& f
   constexpr int EPL = D / ppk::kWave;
   const int lane = threadIdx.x;
   const uint32_t row = blockIdx.x;
-  const uint32_t b = row / a.heads;
+  const uint32_t b = fast_div(row, a.head_div);
   const uint32_t units = t.units[b];
   if (units < 2) return;  // uniform per wave
   const uint32_t phost = t.past[b];
-  const uint32_t pdev = a.past[b];
+  const uint32_t pdev = a.past[b + lane_zero()];
   const size_t base = size_t(row) * D + size_t(lane) * EPL;
-  float sv[EPL];
-  float s_cur = -INFINITY;
-  auto current = [&]() {
-    float qv[EPL], kv[EPL];
-    load_vec<EPL>(a.q, base, a.q_dtype, qv);
-    load_vec<EPL>(a.sk, base, a.scratch_dtype, kv);
-    load_vec<EPL>(a.sv, base, a.scratch_dtype, sv);
-    float d = 0.f;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) d = fmaf(qv[e], kv[e], d);
-    s_cur = wave_sum(d) * a.scale_log2;
-    return s_cur;
-  };
+  MergeCurrent<D> cur;
   float m, zsum, y[EPL];
   combine_records<D>(a.part_mz + size_t(row) * a.nsplits * 2, a.part_y + size_t(row) * a.nsplits * D,
-                     min(units, a.nsplits), lane, current, m, zsum, y);
+                     min(units, a.nsplits), lane, [&]() { cur.request(a, base); }, [&]() { return cur.score(a); }, m,
+                     zsum, y);
   const bool valid = pdev == phost && phost <= a.capacity && phost <= a.span;
-  const float wc = __builtin_amdgcn_exp2f(s_cur - m);
+  const float wc = __builtin_amdgcn_exp2f(cur.s_cur - m);
   zsum += wc;
 #pragma unroll
   for (int e = 0; e < EPL; ++e)
-    store_elem(a.out, base + e, a.out_dtype, valid ? fmaf(wc, sv[e], y[e]) / zsum : __builtin_nanf(""));
+    store_elem(a.out, base + e, a.out_dtype, valid ? fmaf(wc, cur.sv[e], y[e]) / zsum : __builtin_nanf(""));
 }
 
 // ---------------------------------------------------------------------------
@@ -2038,44 +2081,26 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
   const uint32_t begin = (group * W + wave) * S;
   const uint32_t n = (valid && begin < len) ? min(S, len - begin) : 0u;
   FloatWavePartial<D, BF16KV> part;
-  fwave_attention<D, BF16KV>(a, row, begin, n, qr, lds + size_t(wave) * S, lane, part);
+  // LDS of this wave alone: a score per token of its range, then its record.
+  const uint32_t lds_stride = max(S, uint32_t(D + 4));
+  float* s_lds = lds + size_t(wave) * lds_stride;
+  fwave_attention<D, BF16KV>(a, row, begin, n, qr, s_lds, lane, part);
 
-  // Combine the block's waves through LDS: record of wave w at mrg + w * R
-  // holds m, z, 2 pad floats, y[D] (16-byte aligned).
-  constexpr int R = D + 4;
-  __syncthreads();
-  float* mrg = lds;
-  {
-    const int ch = c * G::kEpc + scatter_base<G::kLpt, G::kEpc>(lane);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) mrg[wave * R + 4 + ch + e] = part.acc[e];
-  }
-  if (lane == 0) {
-    mrg[wave * R] = part.m;
-    mrg[wave * R + 1] = part.z;
-  }
+  // Combine the block's waves through LDS: each wave's record replaces its
+  // scores (its own LDS, so no barrier is needed before).
+  write_block_record<D>(s_lds, c * G::kEpc + scatter_base<G::kLpt, G::kEpc>(lane), lane, part.m, part.z, part.acc);
   __syncthreads();
   if (wave != 0) return;
 
-  float m = -INFINITY;
-  for (int w = 0; w < W; ++w) m = fmaxf(m, mrg[w * R]);
   float s_cur = -INFINITY;
   if (cur) {
     float d = 0.f;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) d = fmaf(qcur[e], kcur[e], d);
     s_cur = wave_sum(d) * a.scale_log2;
-    m = fmaxf(m, s_cur);
   }
-  float y[EPL], zsum = 0.f;
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) y[e] = 0.f;
-  for (int w = 0; w < W; ++w) {
-    const float wt = mrg[w * R] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mrg[w * R] - m);
-    zsum = fmaf(wt, mrg[w * R + 1], zsum);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) y[e] = fmaf(wt, mrg[w * R + 4 + lane * EPL + e], y[e]);
-  }
+  float m, y[EPL], zsum;
+  combine_block<D, 16>(lds, lds_stride, uint32_t(W), lane, s_cur, m, zsum, y);
   if (cur) {
     const float wc = __builtin_amdgcn_exp2f(s_cur - m);
     zsum += wc;
@@ -2102,54 +2127,70 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
 // Cross-group merge of the float path (pp_attention_merge,
 // decode_attention.hip:55-66): one wave per row, log-sum-exp weights, NaN for
 // invalid rows or a non-positive total weight.
-// The fused step's current token in a merge: q . k_new (rounded to the
-// store's dtype) as a log2-domain score, with v_new kept for the fold.
+// The fused step's current token in a merge: its row as raw words, then q .
+// k_new (rounded to the store's dtype) as a log2-domain score, with v_new kept
+// for the fold. Nothing without the step.
 template <int D>
-__device__ __forceinline__ float merge_current(const ppk::FloatMergeArgs& a, uint32_t row, int lane,
-                                               float (&vcur)[D / ppk::kWave]) {
-  constexpr int EPL = D / ppk::kWave;
-  float qv[EPL], kv[EPL];
-  load_vec<EPL>(a.q, size_t(row) * a.q_stride + size_t(lane) * EPL, a.q_dtype, qv);
-  load_vec<EPL>(a.k_new, size_t(row) * D + size_t(lane) * EPL, a.new_dtype, kv);
-  load_vec<EPL>(a.v_new, size_t(row) * D + size_t(lane) * EPL, a.new_dtype, vcur);
-  if (a.kv_bf16) {
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      kv[e] = bf16_to_f32(f32_to_bf16_bits(kv[e]));
-      vcur[e] = bf16_to_f32(f32_to_bf16_bits(vcur[e]));
-    }
+struct FloatMergeCurrent {
+  static constexpr int EPL = D / ppk::kWave;
+  RawVec<EPL> q, k, v;
+  float vcur[EPL], s_cur = -INFINITY;
+  __device__ __forceinline__ void request(const ppk::FloatMergeArgs& a, uint32_t row, int lane) {
+    if (!a.step) return;  // uniform
+    const size_t own = size_t(lane) * EPL;
+    load_raw<EPL>(a.q, size_t(row) * a.q_stride + own, a.q_dtype, q);
+    load_raw<EPL>(a.k_new, size_t(row) * D + own, a.new_dtype, k);
+    load_raw<EPL>(a.v_new, size_t(row) * D + own, a.new_dtype, v);
   }
-  float d = 0.f;
+  __device__ __forceinline__ float score(const ppk::FloatMergeArgs& a) {
+    if (!a.step) return s_cur;
+    float qv[EPL], kv[EPL], d = 0.f;
+    widen<EPL>(q, a.q_dtype, qv);
+    widen<EPL>(k, a.new_dtype, kv);
+    widen<EPL>(v, a.new_dtype, vcur);
+    if (a.kv_bf16) {
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) d = fmaf(qv[e], kv[e], d);
-  return wave_sum(d) * a.scale_log2;
-}
+      for (int e = 0; e < EPL; ++e) {
+        kv[e] = bf16_to_f32(f32_to_bf16_bits(kv[e]));
+        vcur[e] = bf16_to_f32(f32_to_bf16_bits(vcur[e]));
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) d = fmaf(qv[e], kv[e], d);
+    s_cur = wave_sum(d) * a.scale_log2;
+    return s_cur;
+  }
+};
 
 template <int D>
 __device__ __forceinline__ void fmerge_body(const ppk::FloatMergeArgs& a) {
   constexpr int EPL = D / ppk::kWave;
+  // Every argument on the way to the loads, requested together.
+  __asm__ volatile("" ::"s"(a.lengths), "s"(a.part_y), "s"(a.part_mz), "s"(a.out), "s"(a.q), "s"(a.k_new),
+                   "s"(a.v_new), "s"(a.size), "s"(a.split_tokens), "s"(a.nsplits), "s"(a.out_dtype), "s"(a.span),
+                   "s"(a.step), "s"(a.q_dtype), "s"(a.new_dtype), "s"(a.kv_bf16), "s"(a.scale_log2),
+                   "s"(a.head_div.mul), "s"(a.head_div.shift));
   const int lane = threadIdx.x;
   const uint32_t row = blockIdx.x;
-  float m, zsum, y[EPL], vcur[EPL];
-  float s_cur = -INFINITY;
-  auto current = [&]() {
-    if (a.step) s_cur = merge_current<D>(a, row, lane, vcur);
-    return s_cur;
+  float m, zsum, y[EPL];
+  FloatMergeCurrent<D> cur;
+  // The row's length travels with the records (as a vector load, see lane_zero).
+  uint32_t len_raw = a.size;
+  auto request = [&]() {
+    cur.request(a, row, lane);
+    if (a.lengths) len_raw = a.lengths[fast_div(row, a.head_div) + lane_zero()];
   };
   combine_records<D>(a.part_mz + size_t(row) * a.nsplits * 2, a.part_y + size_t(row) * a.nsplits * D, a.nsplits,
-                     lane, current, m, zsum, y);
-  // The row's length is first needed here: read after the records went out
-  // (deciding validity up front would hold every record load back by the
-  // length's round trip).
-  const uint32_t len = float_row_length(a.lengths, row, a.heads, a.size);
+                     lane, request, [&]() { return cur.score(a); }, m, zsum, y);
+  const uint32_t len = __builtin_amdgcn_readfirstlane(len_raw);
   const bool cover = uint64_t(len) <= uint64_t(a.nsplits) * a.split_tokens;
   const bool valid = a.step ? (len < a.size && len + 1 <= a.span && cover)
                             : (len > 0 && len <= a.span && len <= a.size && cover);
   if (a.step) {
-    const float wc = __builtin_amdgcn_exp2f(s_cur - m);
+    const float wc = __builtin_amdgcn_exp2f(cur.s_cur - m);
     zsum += wc;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) y[e] = fmaf(wc, vcur[e], y[e]);
+    for (int e = 0; e < EPL; ++e) y[e] = fmaf(wc, cur.vcur[e], y[e]);
   }
   const size_t base = size_t(row) * D + size_t(lane) * EPL;
 #pragma unroll
@@ -2370,23 +2411,20 @@ __device__ __forceinline__ void fmerge_flat_body(const ppk::FloatMergeFlatArgs& 
   constexpr int EPL = D / ppk::kWave;
   const int lane = threadIdx.x;
   const uint32_t row = blockIdx.x;
-  const uint32_t b = row / a.heads;
+  const uint32_t b = fast_div(row, a.head_div);
   const uint32_t units = t.units[b];
   if (units < 2) return;  // uniform per wave
-  const uint32_t ldev = a.lengths[b];
-  float m, zsum, y[EPL], vcur[EPL];
-  float s_cur = -INFINITY;
-  auto current = [&]() {
-    if (a.step) s_cur = merge_current<D>(a, row, lane, vcur);
-    return s_cur;
-  };
+  const uint32_t ldev = a.lengths[b + lane_zero()];
+  float m, zsum, y[EPL];
+  FloatMergeCurrent<D> cur;
   combine_records<D>(a.part_mz + size_t(row) * a.nsplits * 2, a.part_y + size_t(row) * a.nsplits * D,
-                     min(units, a.nsplits), lane, current, m, zsum, y);
+                     min(units, a.nsplits), lane, [&]() { cur.request(a, row, lane); },
+                     [&]() { return cur.score(a); }, m, zsum, y);
   if (a.step) {
-    const float wc = __builtin_amdgcn_exp2f(s_cur - m);
+    const float wc = __builtin_amdgcn_exp2f(cur.s_cur - m);
     zsum += wc;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) y[e] = fmaf(wc, vcur[e], y[e]);
+    for (int e = 0; e < EPL; ++e) y[e] = fmaf(wc, cur.vcur[e], y[e]);
   }
   const bool valid = a.step ? (ldev == t.past[b] && t.past[b] < a.size && t.past[b] + 1 <= a.span)
                             : (t.len[b] > 0 && ldev == t.past[b]);
