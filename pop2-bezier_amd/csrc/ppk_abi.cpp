@@ -497,12 +497,14 @@ uint64_t flat_cu_peak(const AttentionPlan& p, uint32_t heads, uint32_t cus) {
   std::vector<uint64_t> load(cus, 0);
   const FlatTable& t = p.table;
   uint64_t unit = 0;  // unit u on block u / waves (the int8 kernel's assignment)
-  for (uint32_t b = 0; b < t.batch; ++b)
+  for (uint32_t b = 0; b < t.batch; ++b) {
+    const uint32_t len = t.seq[b].len, units = t.seq[b].units & 0xffffffu;
     for (uint32_t h = 0; h < heads; ++h)
-      for (uint32_t s = 0; s < t.units[b]; ++s, ++unit) {
+      for (uint32_t s = 0; s < units; ++s, ++unit) {
         const uint64_t t0 = uint64_t(s) * t.share;
-        if (t.len[b] > t0) load[(unit / p.waves) % cus] += std::min<uint64_t>(t.share, t.len[b] - t0);
+        if (len > t0) load[(unit / p.waves) % cus] += std::min<uint64_t>(t.share, len - t0);
       }
+  }
   return *std::max_element(load.begin(), load.end());
 }
 
@@ -616,16 +618,16 @@ AttentionPlan plan_flat(const ppk_context* ctx, uint32_t rows, uint32_t heads, c
   t.batch = rows / heads;
   uint64_t total = 0;
   for (uint32_t b = 0; b < t.batch; ++b) {
-    t.past[b] = host[b];
-    t.len[b] = host[b] <= limit ? host[b] : 0u;
-    total += uint64_t(t.len[b]) * heads;
+    t.seq[b].past = host[b];
+    t.seq[b].len = host[b] <= limit ? host[b] : 0u;
+    total += uint64_t(t.seq[b].len) * heads;
   }
   // The least share whose units fit the waves: units(Q) = sum over rows of
   // max(1, ceil(len / Q)) falls as Q grows, and Q = ceil(T / (waves - rows))
   // always fits (units <= T / Q + rows), so a binary search between 64 and it.
   auto units_for = [&](uint64_t q) {
     uint64_t u = 0;
-    for (uint32_t b = 0; b < t.batch; ++b) u += uint64_t(heads) * std::max<uint64_t>(1, (t.len[b] + q - 1) / q);
+    for (uint32_t b = 0; b < t.batch; ++b) u += uint64_t(heads) * std::max<uint64_t>(1, (t.seq[b].len + q - 1) / q);
     return u;
   };
   const uint64_t spare = waves - rows;
@@ -643,11 +645,15 @@ AttentionPlan plan_flat(const ppk_context* ctx, uint32_t rows, uint32_t heads, c
       t.first[b] = 0xffffffffu;
       continue;
     }
-    t.units[b] = std::max<uint32_t>(1, (t.len[b] + t.share - 1) / t.share);
+    const uint32_t units = std::max<uint32_t>(1, (t.seq[b].len + t.share - 1) / t.share);
+    const FastDiv div = fast_divisor(units);  // units <= waves < 2^24
+    t.seq[b].units = units | div.shift << 24;
+    t.seq[b].div_mul = div.mul;
     t.first[b] = uint32_t(first);
-    first += uint64_t(t.units[b]) * heads;
-    most = std::max(most, t.units[b]);
+    first += uint64_t(units) * heads;
+    most = std::max(most, units);
   }
+  for (int i = 0; i < kFlatMaxBatch / 8; ++i) t.pivot[i] = t.first[8 * i];
   require(first <= waves, "balanced plan: units exceed the launched waves");
   t.units_total = uint32_t(first);
   plan.split = t.share;
@@ -1037,6 +1043,8 @@ void run_float_attention(ppk_context* ctx, hipStream_t stream, const PpkFloatAtt
   d.v_stride = a.v_row_stride ? a.v_row_stride : row_elems;
   d.rows = a.rows;
   d.heads = a.heads;
+  d.row_div = fast_divisor(a.rows);
+  d.head_div = fast_divisor(a.heads);
   d.size = a.size;
   d.split_tokens = plan.split;
   d.ngroups = plan.ngroups;

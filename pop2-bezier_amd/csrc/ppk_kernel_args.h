@@ -148,18 +148,23 @@ struct MergeArgs {
 // finished by its wave; unit s of a longer row leaves the record at slot s
 // of the row's ngroups slots (y at part_y + (row * ngroups + s) * D, (m, z)
 // at part_mz + (row * ngroups + s) * 2) for the balanced merge kernel.
-// past[] is compared with the device's past: a sequence whose values differ
-// gives NaN rows.
+// past is compared with the device's: a sequence whose values differ gives
+// NaN rows.
 constexpr int kFlatMaxBatch = 64;
+struct FlatSequence {
+  uint32_t past;                   // the host's past[b]
+  uint32_t len;                    // live history tokens of each row
+  uint32_t units;                  // bits 0-23: units per row; 24-31: the shift of their FastDiv
+  uint32_t div_mul;                // the multiplier of their FastDiv
+};
 struct FlatTable {
   uint32_t batch;                  // sequences
   uint32_t share;                  // most tokens of a unit
   uint32_t units_total;            // units over all rows
   uint32_t pad;
-  uint32_t past[kFlatMaxBatch];    // the host's past[b]
-  uint32_t len[kFlatMaxBatch];     // live history tokens of each row of sequence b
-  uint32_t units[kFlatMaxBatch];   // units per row of sequence b
+  uint32_t pivot[kFlatMaxBatch / 8];  // first[0], first[8], ...
   uint32_t first[kFlatMaxBatch];   // index of sequence b's first unit
+  FlatSequence seq[kFlatMaxBatch];
 };
 struct DecodeFlatArgs {
   DecodeArgs d;             // ngroups = record slots per row
@@ -197,6 +202,7 @@ struct FloatDecodeArgs {
   float scale_log2;         // softmax_scale * log2(e)
   uint32_t span;            // most tokens a row may attend (<= size)
   uint32_t new_dtype;
+  FastDiv row_div, head_div;  // by rows, by heads
 };
 
 struct FloatMergeArgs {
@@ -217,7 +223,7 @@ struct FloatMergeArgs {
 };
 
 // Float-KV decode over the balanced work list: the table as for the int8
-// path, with past[b] the host's lengths[b] and len[b] its live tokens (0 for
+// path, with past the host's lengths[b] and len its live tokens (0 for
 // a length outside (0, min(size, max_length)], whose rows give NaN).
 struct FloatDecodeFlatArgs {
   FloatDecodeArgs d;

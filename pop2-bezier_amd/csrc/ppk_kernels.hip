@@ -578,15 +578,6 @@ struct QInt {
   float unscale;  // qmax / Q (NaN if q held a non-finite value)
 };
 
-template <int LPT>
-__device__ __forceinline__ float group_max(float x) {
-  x = fmaxf(x, dpp_xor1(x));
-  x = fmaxf(x, dpp_xor2(x));
-  if constexpr (LPT >= 8) x = fmaxf(x, dpp_half_mirror(x));
-  if constexpr (LPT >= 16) x = fmaxf(x, dpp_mirror(x));
-  return x;
-}
-
 // Max over G consecutive lanes (G a power of two <= 64) of values that are
 // >= +0 and never NaN: such floats order like their bit patterns, so the
 // reduction runs as unsigned integer max (the DPP move folds into the max,
@@ -766,47 +757,6 @@ __device__ __forceinline__ void quantize_stream_dtype(const ppk::QuantizeArgs& a
   else quantize_stream_units<D, 8, kF16, ARENA>(a);
 }
 
-
-template <int LPT>
-__device__ __forceinline__ QInt quantize_query_chunk(const float (&qr)[16]) {
-  constexpr float Q = 266338304.0f;  // 127 * 2^21
-  float amax = 0.f;
-  bool finite = true;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    amax = fmaxf(amax, fabsf(qr[i]));
-    finite = finite && __builtin_isfinite(qr[i]);
-  }
-  amax = group_max<LPT>(amax);  // every lane of a token group holds the whole row of q
-  const float bad = group_max<LPT>(finite ? 0.f : 1.f);
-  const float inv = amax > 0.f ? Q / amax : 0.f;
-  QInt r;
-  r.unscale = bad > 0.f ? __builtin_nanf("") : amax / Q;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    uint32_t h = 0, a = 0, b = 0, l = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float x = fminf(fmaxf(rintf(qr[4 * w + k] * inv), -Q), Q);
-      const int qi = finite ? int(x) : 0;
-      const int hi = (qi + (1 << 20)) >> 21;  // [-127, 127]
-      const int r1 = qi - hi * (1 << 21);     // [-2^20, 2^20)
-      const int m1 = (r1 + 8192) >> 14;       // [-64, 64]
-      const int r2 = r1 - m1 * 16384;         // [-8192, 8191]
-      const int m2 = (r2 + 64) >> 7;          // [-64, 64]
-      const int lo = r2 - m2 * 128;           // [-64, 63]
-      h |= (uint32_t(hi) & 0xffu) << (8 * k);
-      a |= (uint32_t(m1) & 0xffu) << (8 * k);
-      b |= (uint32_t(m2) & 0xffu) << (8 * k);
-      l |= (uint32_t(lo) & 0xffu) << (8 * k);
-    }
-    r.hi[w] = int(h);
-    r.m1[w] = int(a);
-    r.m2[w] = int(b);
-    r.lo[w] = int(l);
-  }
-  return r;
-}
 
 // The query of one wave, from x = channels lane * D/64 ... of q: each lane
 // forms the slices of its own D/64 channels and the wave exchanges them
@@ -991,17 +941,6 @@ __device__ __forceinline__ void accumulate_batch(const u4 (&raw)[U], float scale
     const float vscale = BF16H ? __shfl(scale_lane, u * TPL + j) : 1.f;
     tile_accumulate<BF16H>(raw[u], wgt, vscale, acc);
   }
-}
-
-// Log2-domain score of the current token (q . sk * scale), which comes from
-// the scratch copy, not the arena: each lane dots its 16-channel chunk.
-template <int D>
-__device__ __forceinline__ float current_score(const ppk::DecodeArgs& a, const float (&kv)[16],
-                                               const float (&qr)[16]) {
-  float d = 0.f;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) d = fmaf(qr[i], kv[i], d);
-  return group_sum<D / 16>(d) * a.scale_log2;
 }
 
 // A stream of at most NBATCH batches per phase, K and V already requested:
@@ -1531,166 +1470,126 @@ __device__ __forceinline__ void attn_merge_body(const ppk::MergeArgs& a) {
 // (current token included); the units of a longer row leave log-sum-exp
 // records that the balanced merge kernel joins.
 //
-// A unit is streamed as (K, V) pairs of batches through a window of two
-// pairs in registers with an online softmax (running max per token group,
-// one rescale per batch). Measured against four pairs and one, and against
-// the per-row kernel's two-phase stream inside the same assignment, on
-// configs 3 and 4 and ragged batches of 16 to 64 sequences: two pairs and the
-// two-phase stream tie, four pairs is 2-12 % slower.
+// A unit is streamed as (K, V) pairs of batches through a window of NP pairs
+// in registers with an online softmax (running max per token group, one
+// rescale per batch that raises it). What bounds a unit is its waves' latency
+// more than its bytes: the table is searched with two dependent scalar loads,
+// every small operand travels as raw words beside the window's first pairs,
+// and the window's refills are unconditional (past the end they read the
+// unit's last token again), so that each wait is for the oldest pair only.
+// @MEASURED_FLAT@
 // ---------------------------------------------------------------------------
 // One (K, V) batch pair of a unit under the online softmax. Token group j
 // (the LPT lanes holding one token of each tile) keeps its own running max m,
 // sum z and 16-channel accumulator: the batch's four scores are formed, the
-// state is rescaled once to the new max, then each tile's V codes are added
-// with weight 2^(s - m) * vscale.
+// state is rescaled to the new max if any group of the wave has one, then
+// each tile's V codes are added with weight 2^(s - m) * vscale.
 template <int D, bool BF16H>
 __device__ __forceinline__ void online_pair(const u4 (&kraw)[4], const u4 (&vraw)[4], float ks_lane, float vs_lane,
-                                            uint32_t t0, uint32_t n, int j, const float (&qr)[16], const QInt& qi,
-                                            float sl2, float& m, float& z, float (&acc)[16]) {
+                                            uint32_t t0, uint32_t n, int j, const Query<BF16H>& q, float& m, float& z,
+                                            float (&acc)[16]) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
-  float s[4];
+  float s[4], kscale[4], vscale[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) kscale[u] = __shfl(ks_lane, u * TPL + j);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) vscale[u] = __shfl(vs_lane, u * TPL + j);
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const uint32_t tok = (t0 + u) * TPL + j;
-    const float kscale = __shfl(ks_lane, u * TPL + j);
-    float sc;
-    if constexpr (BF16H) {
-      float d = 0.f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-#pragma unroll
-        for (int k = 0; k < 4; k += 2) {
-          float e0, e1;
-          round_bf16_pair(sbyte(kraw[u][w], k) * kscale, sbyte(kraw[u][w], k + 1) * kscale, e0, e1);
-          d = fmaf(qr[4 * w + k], e0, d);
-          d = fmaf(qr[4 * w + k + 1], e1, d);
-        }
-      sc = group_sum<LPT>(d) * sl2;
-    } else {
-      int sh = 0, s1 = 0, s2 = 0, slo = 0;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        sh = __builtin_amdgcn_sdot4(int(kraw[u][w]), qi.hi[w], sh, false);
-        s1 = __builtin_amdgcn_sdot4(int(kraw[u][w]), qi.m1[w], s1, false);
-        s2 = __builtin_amdgcn_sdot4(int(kraw[u][w]), qi.m2[w], s2, false);
-        slo = __builtin_amdgcn_sdot4(int(kraw[u][w]), qi.lo[w], slo, false);
-      }
-      const int hm = group_sum_i32<LPT>(sh * 128 + s1);
-      const int lm = group_sum_i32<LPT>(s2 * 128 + slo);
-      sc = fmaf(float(hm), 16384.f, float(lm)) * (kscale * sl2);
-    }
-    s[u] = tok < n ? sc : -INFINITY;
+    const float sc = tile_score<D, BF16H>(kraw[u], kscale[u], q);
+    s[u] = (t0 + u) * TPL + j < n ? sc : -INFINITY;
   }
   const float mb = fmaxf(fmaxf(m, fmaxf(s[0], s[1])), fmaxf(s[2], s[3]));
-  const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mb);
-  z *= f;
+  if (__any(mb > m)) {  // a new max somewhere (always on a group's first token)
+    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mb);
+    z *= f;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] *= f;
+    for (int i = 0; i < 16; ++i) acc[i] *= f;
+    m = mb;
+  }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const float pr = s[u] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[u] - mb);
-    z += pr;
-    const float vscale = __shfl(vs_lane, u * TPL + j);
-    if constexpr (BF16H) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-#pragma unroll
-        for (int k = 0; k < 4; k += 2) {
-          float e0, e1;
-          round_bf16_pair(sbyte(vraw[u][w], k) * vscale, sbyte(vraw[u][w], k + 1) * vscale, e0, e1);
-          acc[4 * w + k] = fmaf(pr, e0, acc[4 * w + k]);
-          acc[4 * w + k + 1] = fmaf(pr, e1, acc[4 * w + k + 1]);
-        }
-    } else {
-      const float wgt = pr * vscale;
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[4 * w + k] = fmaf(wgt, sbyte(vraw[u][w], k), acc[4 * w + k]);
-    }
+    const float p = s[u] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[u] - m);
+    z += p;
+    tile_accumulate<BF16H>(vraw[u], p, vscale[u], acc);
   }
-  m = mb;
 }
 
-// Streams tokens [begin, begin + n) of one row (n >= 1) through the window
-// of two (K, V) pairs; returns the wave's partial (m, z in every lane, the
-// 16-channel sums in lanes j == 0), as wave_attention does. early() runs
-// once the window's first loads are in flight (work whose own loads were
-// issued before, so that waiting for them does not hold the window back).
-template <int D, bool BF16H, class Early>
-__device__ __forceinline__ void wave_attention_window(const ppk::DecodeArgs& a, uint32_t row, uint32_t begin,
-                                                      uint32_t n, const float (&qr)[16], int lane,
+// Streams tokens [0, n) (n >= 1) of the given K / V / scale ranges through the
+// window of NP (K, V) pairs; returns the wave's partial as short_attention
+// does. early() runs once the window's first loads are in flight and leaves
+// the query.
+template <int D, bool BF16H, int NP, class Early>
+__device__ __forceinline__ void wave_attention_window(const uint8_t* kb, const uint8_t* vb, const float* ksb,
+                                                      const float* vsb, uint32_t n, const Query<BF16H>& q, int lane,
                                                       WavePartial& out, Early early) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
-  constexpr int U = 4, NP = 2;
+  constexpr int U = 4;
   const int j = lane / LPT;
-  const int c = lane % LPT;
-  const size_t tok0 = size_t(row) * a.capacity + begin;
-  const uint8_t* kb = a.k + tok0 * D + size_t(c) * 16;
-  const uint8_t* vb = a.v + tok0 * D + size_t(c) * 16;
-  const float* ksb = a.ks + tok0;
-  const float* vsb = a.vs + tok0;
   const uint32_t nb = (n + U * TPL - 1) / (U * TPL);  // batches per phase
   u4 kr[NP][U], vr[NP][U];
   float ksl[NP], vsl[NP];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    if (uint32_t(p) < nb) {  // uniform per wave
-      load_batch<D, U>(kb, ksb, uint32_t(p) * U, n, j, lane, kr[p], ksl[p]);
-      load_batch<D, U>(vb, vsb, uint32_t(p) * U, n, j, lane, vr[p], vsl[p]);
-    }
-  }
-  QInt qi{};
-  float sl2 = a.scale_log2;
-  if constexpr (!BF16H) {
-    qi = quantize_query_chunk<LPT>(qr);
-    sl2 *= qi.unscale;
+    load_batch<D, U>(kb, ksb, uint32_t(p) * U, n, j, lane, kr[p], ksl[p]);
+    load_batch<D, U>(vb, vsb, uint32_t(p) * U, n, j, lane, vr[p], vsl[p]);
   }
   early();
-  float m = -INFINITY, z = 0.f, acc[16];
+  float m = -INFINITY, z = 0.f;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int i = 0; i < 16; ++i) out.acc[i] = 0.f;
   for (uint32_t b0 = 0; b0 < nb; b0 += NP) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       const uint32_t bi = b0 + uint32_t(p);
-      if (bi < nb) {  // uniform per wave
-        // Scales of tokens at or past n are never used (their scores are -inf).
-        online_pair<D, BF16H>(kr[p], vr[p], ksl[p], vsl[p], bi * U, n, j, qr, qi, sl2, m, z, acc);
-        if (bi + NP < nb) {
-          load_batch<D, U>(kb, ksb, (bi + NP) * U, n, j, lane, kr[p], ksl[p]);
-          load_batch<D, U>(vb, vsb, (bi + NP) * U, n, j, lane, vr[p], vsl[p]);
-        }
-      }
+      // Scales of tokens at or past n are never used (their scores are -inf).
+      if (bi < nb) online_pair<D, BF16H>(kr[p], vr[p], ksl[p], vsl[p], bi * U, n, j, q, m, z, out.acc);
+      load_batch<D, U>(kb, ksb, (bi + NP) * U, n, j, lane, kr[p], ksl[p]);
+      load_batch<D, U>(vb, vsb, (bi + NP) * U, n, j, lane, vr[p], vsl[p]);
     }
   }
   // Join the token groups: common max, then sums across groups.
-  float mm = m;
-  mm = groups_max<LPT>(mm);
+  const float mm = groups_max<LPT>(m);
   const float w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mm);
   z *= w;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] *= w;
-  z = groups_reduce<LPT>(z, [](float a, float b) { return a + b; });
-  reduce_scatter_groups<LPT, 16>(acc, lane);
+  for (int i = 0; i < 16; ++i) out.acc[i] *= w;
   out.m = mm;
-  out.z = z;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) out.acc[i] = acc[i];
+  out.z = groups_reduce<LPT>(z, [](float a, float b) { return a + b; });
+  reduce_scatter_groups<LPT, 16>(out.acc, lane);
 }
 
-// The table's sequence holding unit `unit` (< units_total): the last b with
-// first[b] <= unit. A uniform binary search over the kernel arguments.
-__device__ __forceinline__ uint32_t flat_sequence(const ppk::FlatTable& t, uint32_t unit) {
-  uint32_t lo = 0, hi = t.batch - 1;
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi + 1) / 2;
-    if (t.first[mid] <= unit) lo = mid;
-    else hi = mid - 1;
+// The table's entry of unit `unit` (< units_total, uniform): the last
+// sequence whose first unit is at most `unit`. Counting the group heads and
+// then the group's eight first units costs two dependent scalar loads.
+struct FlatUnit {
+  uint32_t b, past, len, units;
+  uint32_t head, slot;  // the unit's head, its place within the head's row
+};
+__device__ __forceinline__ FlatUnit flat_unit(const ppk::FlatTable& t, uint32_t unit) {
+  uint32_t g = 0;
+#pragma unroll
+  for (int i = 1; i < ppk::kFlatMaxBatch / 8; ++i) g += t.pivot[i] <= unit ? 1u : 0u;
+  uint32_t first = t.first[8 * g], b = 8 * g;
+#pragma unroll
+  for (int i = 1; i < 8; ++i) {
+    const uint32_t f = t.first[8 * g + i];
+    if (f <= unit) {
+      first = f;
+      ++b;
+    }
   }
-  return lo;
+  const ppk::FlatSequence s = t.seq[b];
+  FlatUnit u;
+  u.b = b;
+  u.past = s.past;
+  u.len = s.len;
+  u.units = s.units & 0xffffffu;
+  u.head = fast_div(unit - first, ppk::FastDiv{s.div_mul, s.units >> 24});
+  u.slot = unit - first - u.head * u.units;
+  return u;
 }
 
 template <int D, bool BF16H>
@@ -1699,88 +1598,106 @@ __device__ __forceinline__ void decode_flat_body(const ppk::DecodeFlatArgs& fa) 
   const ppk::FlatTable& t = fa.t;
   constexpr int LPT = D / 16;
   constexpr int EPL = D / ppk::kWave;
+  __shared__ u4 s_query[8][D / 4];  // per wave: the query's exchange
+  // The arguments on the way to the first loads, requested together.
+  __asm__ volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.ks), "s"(a.vs), "s"(a.sk), "s"(a.sv), "s"(a.past),
+                   "s"(a.k_new), "s"(a.v_new), "s"(a.rows), "s"(a.heads), "s"(a.capacity), "s"(a.q_dtype),
+                   "s"(a.scratch_dtype), "s"(a.new_dtype), "s"(a.append), "s"(a.head_div.mul), "s"(a.head_div.shift),
+                   "s"(t.share), "s"(t.units_total), "s"(t.pivot[1]), "s"(t.pivot[2]), "s"(t.pivot[3]),
+                   "s"(t.pivot[4]), "s"(blockDim.x));
   const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform, as everything derived from it
   const uint32_t W = blockDim.x >> 6;
-  const uint32_t wid = blockIdx.x * W + (threadIdx.x >> 6);
+  const uint32_t wid = blockIdx.x * W + wave;
   const int c = lane % LPT;
 
   // Append job (a decode step): wave q < 2 rows quantises tensor q & 1 of
   // row q >> 1 into slot past[b] (the device value) of the arenas. Its loads
   // are issued first, beside everything else this wave reads.
-  const bool append = a.append && wid < 2 * a.rows;  // uniform per wave (the host keeps waves >= 2 rows)
+  const bool append = a.append && wid < 2 * a.rows;  // the host keeps waves >= 2 rows
   const uint32_t arow = wid >> 1;
-  float ax[EPL];
-  uint32_t ap = 0;
+  RawVec<EPL> new_raw;
+  uint32_t ap_raw = 0;
   if (append) {
-    ap = a.past[arow / a.heads];
-    load_vec<EPL>((wid & 1u) ? a.v_new : a.k_new, size_t(arow) * D + size_t(lane) * EPL, a.new_dtype, ax);
-  }
-  const bool work = wid < t.units_total;  // uniform per wave
-  uint32_t b = 0, units = 1, len = 0, row = 0, slot = 0, t0 = 0, n = 0, pdev = 0;
-  float qr[16], kv[16], sv[EPL];
-  const int ch = c * 16 + scatter_base<LPT, 16>(lane);  // this lane's output channels: ch .. ch + EPL - 1
-  if (work) {
-    b = flat_sequence(t, wid);
-    units = t.units[b];
-    len = t.len[b];
-    const uint32_t k = wid - t.first[b];
-    const uint32_t h = k / units;
-    slot = k - h * units;
-    row = b * a.heads + h;
-    t0 = slot * t.share;
-    n = len > t0 ? min(t.share, len - t0) : 0u;
-    pdev = a.past[b];
-    if (n > 0) load_vec<16>(a.q, size_t(row) * D + size_t(c) * 16, a.q_dtype, qr);
-    if (units == 1) {  // the whole row: its current token too
-      if (n > 0) load_vec<16>(a.sk, size_t(row) * D + size_t(c) * 16, a.scratch_dtype, kv);
-      load_vec<EPL>(a.sv, size_t(row) * D + size_t(ch), a.scratch_dtype, sv);
-    }
+    ap_raw = a.past[fast_div(arow, a.head_div) + lane_zero()];
+    load_raw<EPL>((wid & 1u) ? a.v_new : a.k_new, size_t(arow) * D + size_t(lane) * EPL, a.new_dtype, new_raw);
   }
   auto commit = [&]() {
     if (!append) return;
+    const uint32_t ap = __builtin_amdgcn_readfirstlane(ap_raw);
     if (ap >= a.capacity) {
       if (lane == 0 && a.flags) atomicOr(a.flags, 2u);
     } else {
       const size_t dst = size_t(arow) * a.capacity + ap;
-      if (wid & 1u) quantize_values<D>(ax, a.v + dst * D, a.vs + dst, a.flags, lane);
-      else quantize_values<D>(ax, a.k + dst * D, a.ks + dst, a.flags, lane);
+      float x[EPL];
+      widen<EPL>(new_raw, a.new_dtype, x);
+      if (wid & 1u) quantize_values<D>(x, a.v + dst * D, a.vs + dst, a.flags, lane);
+      else quantize_values<D>(x, a.k + dst * D, a.ks + dst, a.flags, lane);
     }
   };
-  if (!work) {
+  if (wid >= t.units_total) {
     commit();
     return;
   }
-  // The row is valid when the host's length is in range and the device agrees.
-  const uint32_t phost = t.past[b];
-  const bool host_ok = phost <= a.capacity && phost <= a.span;
+  const FlatUnit u = flat_unit(t, wid);
+  const uint32_t row = u.b * a.heads + u.head;
+  const uint32_t t0 = u.slot * t.share;
+  const uint32_t n = u.len > t0 ? min(t.share, u.len - t0) : 0u;
+  const int ch = c * 16 + scatter_base<LPT, 16>(lane);  // this lane's output channels: ch .. ch + EPL - 1
+  const bool whole = u.units == 1;                      // the whole row: its current token too
+  const uint32_t p_raw = a.past[u.b + lane_zero()];
+  RawVec<EPL> q_raw, sk_raw, sv_raw;
+  load_raw<EPL>(a.q, size_t(row) * D + size_t(lane) * EPL, a.q_dtype, q_raw);
+  if (whole) {
+    load_raw<EPL>(a.sk, size_t(row) * D + size_t(lane) * EPL, a.scratch_dtype, sk_raw);
+    load_raw<EPL>(a.sv, size_t(row) * D + size_t(ch), a.scratch_dtype, sv_raw);
+  }
   WavePartial part;
   part.m = -INFINITY;
   part.z = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) part.acc[i] = 0.f;
   float s_cur = -INFINITY;
   if (n > 0) {
+    Query<BF16H> query;
+    const size_t tok0 = size_t(row) * a.capacity + t0;
     auto early = [&]() {  // with the unit's first loads in flight
+      float x[EPL];
+      widen<EPL>(q_raw, a.q_dtype, x);
+      make_query<D, BF16H>(x, a.scale_log2, s_query[wave], lane, query);
+      if (whole) {
+        float kv[EPL], d = 0.f;
+        widen<EPL>(sk_raw, a.scratch_dtype, kv);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) d = fmaf(x[e], kv[e], d);
+        s_cur = wave_sum(d) * a.scale_log2;
+      }
       commit();
-      if (units == 1) s_cur = current_score<D>(a, kv, qr);
     };
-    wave_attention_window<D, BF16H>(a, row, t0, n, qr, lane, part, early);
+    wave_attention_window<D, BF16H, 2>(a.k + tok0 * D + size_t(c) * 16, a.v + tok0 * D + size_t(c) * 16,
+                                       a.ks + tok0, a.vs + tok0, n, query, lane, part, early);
   } else {
     commit();
   }
-  const bool fresh = pdev == phost;
+  // The row is valid when the host's length is in range and the device agrees.
+  const bool host_ok = u.past <= a.capacity && u.past <= a.span;
+  const bool fresh = __builtin_amdgcn_readfirstlane(p_raw) == u.past;
   if (!fresh && lane == 0 && a.flags) atomicOr(a.flags, 4u);
-  if (units == 1) {
+  if (whole) {
     const bool valid = fresh && host_ok;
     const float m = fmaxf(part.m, s_cur);
     const float wp = n > 0 ? __builtin_amdgcn_exp2f(part.m - m) : 0.f;
     const float wc = n > 0 ? __builtin_amdgcn_exp2f(s_cur - m) : 1.f;
     const float zsum = n > 0 ? fmaf(wp, part.z, wc) : 1.f;
+    float sv[EPL];
+    widen<EPL>(sv_raw, a.scratch_dtype, sv);
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
       const float o = valid ? fmaf(wc, sv[e], n > 0 ? wp * part.acc[e] : 0.f) / zsum : __builtin_nanf("");
       store_elem(a.out, size_t(row) * D + size_t(ch + e), a.out_dtype, o);
     }
-  } else if (slot < a.ngroups) {  // always, by the host's count of slots
-    const size_t rec = size_t(row) * a.ngroups + slot;
+  } else if (u.slot < a.ngroups) {  // always, by the host's count of slots
+    const size_t rec = size_t(row) * a.ngroups + u.slot;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a.part_y[rec * D + size_t(ch + e)] = part.acc[e];
     if (lane == 0) {
@@ -1799,19 +1716,27 @@ __device__ __forceinline__ void attn_merge_flat_body(const ppk::MergeFlatArgs& f
   const ppk::MergeArgs& a = fa.m;
   const ppk::FlatTable& t = fa.t;
   constexpr int EPL = D / ppk::kWave;
+  __asm__ volatile("" ::"s"(a.q), "s"(a.sk), "s"(a.sv), "s"(a.past), "s"(a.part_y), "s"(a.part_mz), "s"(a.out),
+                   "s"(a.capacity), "s"(a.nsplits), "s"(a.q_dtype), "s"(a.scratch_dtype), "s"(a.out_dtype),
+                   "s"(a.scale_log2), "s"(a.head_div.mul), "s"(a.head_div.shift));
   const int lane = threadIdx.x;
   const uint32_t row = blockIdx.x;
   const uint32_t b = fast_div(row, a.head_div);
-  const uint32_t units = t.units[b];
+  const ppk::FlatSequence seq = t.seq[b];
+  const uint32_t units = seq.units & 0xffffffu;
   if (units < 2) return;  // uniform per wave
-  const uint32_t phost = t.past[b];
-  const uint32_t pdev = a.past[b + lane_zero()];
+  const uint32_t phost = seq.past;
   const size_t base = size_t(row) * D + size_t(lane) * EPL;
   MergeCurrent<D> cur;
+  uint32_t p_raw = 0;
+  auto request = [&]() {
+    cur.request(a, base);
+    p_raw = a.past[b + lane_zero()];
+  };
   float m, zsum, y[EPL];
   combine_records<D>(a.part_mz + size_t(row) * a.nsplits * 2, a.part_y + size_t(row) * a.nsplits * D,
-                     min(units, a.nsplits), lane, [&]() { cur.request(a, base); }, [&]() { return cur.score(a); }, m,
-                     zsum, y);
+                     min(units, a.nsplits), lane, request, [&]() { return cur.score(a); }, m, zsum, y);
+  const uint32_t pdev = __builtin_amdgcn_readfirstlane(p_raw);
   const bool valid = pdev == phost && phost <= a.capacity && phost <= a.span;
   const float wc = __builtin_amdgcn_exp2f(cur.s_cur - m);
   zsum += wc;
@@ -2212,7 +2137,8 @@ __device__ __forceinline__ void fmerge_body(const ppk::FloatMergeArgs& a) {
 // ---------------------------------------------------------------------------
 // One (K, V) batch pair under the online softmax: token group j (the lanes
 // of one token of each tile) keeps its running max m, sum z and channel
-// accumulators; the batch's four scores, one rescale, then the V rows.
+// accumulators; the batch's four scores, a rescale if any group of the wave
+// has a new max, then the V rows.
 template <int D, bool BF16KV>
 __device__ __forceinline__ void fonline_pair(const u4 (&kraw)[4], const u4 (&vraw)[4], uint32_t t0, uint32_t n, int j,
                                              const float (&qr)[FloatGeom<D, BF16KV>::kEpc], float sl2, float& m,
@@ -2231,31 +2157,34 @@ __device__ __forceinline__ void fonline_pair(const u4 (&kraw)[4], const u4 (&vra
     s[u] = tok < n ? sc : -INFINITY;
   }
   const float mb = fmaxf(fmaxf(m, fmaxf(s[0], s[1])), fmaxf(s[2], s[3]));
-  const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mb);
-  z *= f;
+  if (__any(mb > m)) {
+    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mb);
+    z *= f;
 #pragma unroll
-  for (int e = 0; e < G::kEpc; ++e) acc[e] *= f;
+    for (int e = 0; e < G::kEpc; ++e) acc[e] *= f;
+    m = mb;
+  }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const float pr = s[u] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[u] - mb);
+    const float pr = s[u] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[u] - m);
     z += pr;
     float x[G::kEpc];
     unpack_chunk<BF16KV>(vraw[u], x);
 #pragma unroll
     for (int e = 0; e < G::kEpc; ++e) acc[e] = fmaf(pr, x[e], acc[e]);
   }
-  m = mb;
 }
 
 // Streams tokens [begin, begin + n) of one row (n >= 1) through the window
-// of two (K, V) pairs; the partial (m, z in every lane, the channel sums in
-// lanes j == 0), as fwave_attention returns it.
-template <int D, bool BF16KV>
+// of NP (K, V) pairs; the partial as fwave_attention returns it. The refills
+// are unconditional, as in the int8 window (wave_attention_window). early()
+// leaves the query chunk in qr, with the window's first loads in flight.
+template <int D, bool BF16KV, int NP, class Early>
 __device__ __forceinline__ void fwave_attention_window(const ppk::FloatDecodeArgs& a, uint32_t row, uint32_t begin,
                                                        uint32_t n, const float (&qr)[FloatGeom<D, BF16KV>::kEpc],
-                                                       int lane, FloatWavePartial<D, BF16KV>& out) {
+                                                       int lane, FloatWavePartial<D, BF16KV>& out, Early early) {
   using G = FloatGeom<D, BF16KV>;
-  constexpr int U = 4, NP = 2;
+  constexpr int U = 4;
   const int j = lane / G::kLpt;
   const int c = lane % G::kLpt;
   const char* kb = static_cast<const char*>(a.k) +
@@ -2266,11 +2195,10 @@ __device__ __forceinline__ void fwave_attention_window(const ppk::FloatDecodeArg
   u4 kr[NP][U], vr[NP][U];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    if (uint32_t(p) < nb) {  // uniform per wave
-      load_fbatch<D, BF16KV, U>(kb, uint32_t(p) * U, n, j, kr[p]);
-      load_fbatch<D, BF16KV, U>(vb, uint32_t(p) * U, n, j, vr[p]);
-    }
+    load_fbatch<D, BF16KV, U>(kb, uint32_t(p) * U, n, j, kr[p]);
+    load_fbatch<D, BF16KV, U>(vb, uint32_t(p) * U, n, j, vr[p]);
   }
+  early();
   float m = -INFINITY, z = 0.f, acc[G::kEpc];
 #pragma unroll
   for (int e = 0; e < G::kEpc; ++e) acc[e] = 0.f;
@@ -2278,17 +2206,12 @@ __device__ __forceinline__ void fwave_attention_window(const ppk::FloatDecodeArg
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       const uint32_t bi = b0 + uint32_t(p);
-      if (bi < nb) {  // uniform per wave
-        fonline_pair<D, BF16KV>(kr[p], vr[p], bi * U, n, j, qr, a.scale_log2, m, z, acc);
-        if (bi + NP < nb) {
-          load_fbatch<D, BF16KV, U>(kb, (bi + NP) * U, n, j, kr[p]);
-          load_fbatch<D, BF16KV, U>(vb, (bi + NP) * U, n, j, vr[p]);
-        }
-      }
+      if (bi < nb) fonline_pair<D, BF16KV>(kr[p], vr[p], bi * U, n, j, qr, a.scale_log2, m, z, acc);
+      load_fbatch<D, BF16KV, U>(kb, (bi + NP) * U, n, j, kr[p]);
+      load_fbatch<D, BF16KV, U>(vb, (bi + NP) * U, n, j, vr[p]);
     }
   }
-  float mm = m;
-  mm = groups_max<G::kLpt>(mm);
+  const float mm = groups_max<G::kLpt>(m);
   const float w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mm);
   z *= w;
 #pragma unroll
@@ -2306,6 +2229,12 @@ __device__ __forceinline__ void fdecode_flat_body(const ppk::FloatDecodeFlatArgs
   const ppk::FloatDecodeArgs& a = fa.d;
   const ppk::FlatTable& t = fa.t;
   using G = FloatGeom<D, BF16KV>;
+  constexpr int EPL = D / ppk::kWave;
+  // The arguments on the way to the first loads, requested together.
+  __asm__ volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.lengths), "s"(a.q_stride), "s"(a.k_stride),
+                   "s"(a.v_stride), "s"(a.rows), "s"(a.heads), "s"(a.q_dtype), "s"(a.new_dtype), "s"(a.scale_log2),
+                   "s"(t.share), "s"(t.units_total), "s"(t.pivot[1]), "s"(t.pivot[2]), "s"(t.pivot[3]),
+                   "s"(t.pivot[4]), "s"(gridDim.x));
   const int lane = threadIdx.x & 63;
   // Wave w of block x takes unit w * blocks + x: the waves that share a CU
   // take units far apart in the list (rows of different lengths, idle waves
@@ -2315,66 +2244,79 @@ __device__ __forceinline__ void fdecode_flat_body(const ppk::FloatDecodeFlatArgs
   // 68.9 -> 67.0 us; f32 1 of 8192 beside 31 of 256, 52.5 -> 48.0 us;
   // within 2 % elsewhere. (The int8 kernel keeps consecutive units per
   // block: this mapping did not help it.)
-  const uint32_t wid = (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-  if constexpr (STEP) {
-    // The step's writes: wave q < 2 rows writes tensor q & 1 of row q >> 1 at
-    // slot lengths[b] (the device value; every stream stops before it).
-    if (wid < 2 * a.rows) {  // uniform per wave (the host keeps waves >= 2 rows)
-      constexpr int EPL = D / ppk::kWave;
-      const uint32_t arow = wid >> 1;
-      const bool value = (wid & 1u) != 0;
-      float x[EPL];
-      load_current<EPL, BF16KV>(value ? a.v_new : a.k_new, arow, a.new_dtype, lane, x);
-      write_current<EPL, BF16KV>(const_cast<void*>(value ? a.v : a.k), value ? a.v_stride : a.k_stride, arow,
-                                 a.lengths[arow / a.heads], a.size, x, a.flags, lane);
-    }
+  const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+  // The step's writes: wave q < 2 rows writes tensor q & 1 of row q >> 1 at
+  // slot lengths[b] (the device value; every stream stops before it).
+  const bool put = STEP && wid < 2 * a.rows;  // the host keeps waves >= 2 rows
+  const uint32_t arow = wid >> 1;
+  const bool value = (wid & 1u) != 0;
+  RawVec<EPL> new_raw;
+  uint32_t slot_raw = 0;
+  if (put) {
+    slot_raw = a.lengths[fast_div(arow, a.head_div) + lane_zero()];
+    load_raw<EPL>(value ? a.v_new : a.k_new, size_t(arow) * D + size_t(lane) * EPL, a.new_dtype, new_raw);
   }
-  if (wid >= t.units_total) return;  // uniform per wave
-  constexpr int EPL = D / ppk::kWave;
+  auto write = [&]() {
+    if (!put) return;
+    float x[EPL];
+    widen<EPL>(new_raw, a.new_dtype, x);
+    write_current<EPL, BF16KV>(const_cast<void*>(value ? a.v : a.k), value ? a.v_stride : a.k_stride, arow,
+                               __builtin_amdgcn_readfirstlane(slot_raw), a.size, x, a.flags, lane);
+  };
+  if (wid >= t.units_total) {
+    write();
+    return;
+  }
+  const FlatUnit u = flat_unit(t, wid);
   const int c = lane % G::kLpt;
   const int ch = c * G::kEpc + scatter_base<G::kLpt, G::kEpc>(lane);  // this lane's output channels
-  const uint32_t b = flat_sequence(t, wid);
-  const uint32_t units = t.units[b];
-  const uint32_t len = t.len[b];
-  const uint32_t k = wid - t.first[b];
-  const uint32_t h = k / units;
-  const uint32_t slot = k - h * units;
-  const uint32_t row = b * a.heads + h;
-  const uint32_t t0 = slot * t.share;
-  const uint32_t n = len > t0 ? min(t.share, len - t0) : 0u;
-  const uint32_t ldev = a.lengths[b];
+  const uint32_t row = u.b * a.heads + u.head;
+  const uint32_t t0 = u.slot * t.share;
+  const uint32_t n = u.len > t0 ? min(t.share, u.len - t0) : 0u;
+  const uint32_t l_raw = a.lengths[u.b + lane_zero()];
   // The step's current token, folded by the wave of a one-unit row (longer
   // rows: by the merge), in this kernel's lane layout and token arithmetic.
-  const bool cur = STEP && units == 1;
-  float qr[G::kEpc], kx[G::kEpc], vx[EPL];
-  if (n > 0 || cur) load_vec<G::kEpc>(a.q, size_t(row) * a.q_stride + size_t(c) * G::kEpc, a.q_dtype, qr);
+  const bool whole = u.units == 1;
+  const bool cur = STEP && whole;
+  RawVec<G::kEpc> q_raw, kx_raw;
+  RawVec<EPL> vx_raw;
+  load_raw<G::kEpc>(a.q, size_t(row) * a.q_stride + size_t(c) * G::kEpc, a.q_dtype, q_raw);
   if (cur) {
-    load_vec<G::kEpc>(a.k_new, size_t(row) * D + size_t(c) * G::kEpc, a.new_dtype, kx);
-    load_vec<EPL>(a.v_new, size_t(row) * D + size_t(ch), a.new_dtype, vx);
-    if constexpr (BF16KV) {
-#pragma unroll
-      for (int e = 0; e < G::kEpc; ++e) kx[e] = bf16_to_f32(f32_to_bf16_bits(kx[e]));
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) vx[e] = bf16_to_f32(f32_to_bf16_bits(vx[e]));
-    }
+    load_raw<G::kEpc>(a.k_new, size_t(row) * D + size_t(c) * G::kEpc, a.new_dtype, kx_raw);
+    load_raw<EPL>(a.v_new, size_t(row) * D + size_t(ch), a.new_dtype, vx_raw);
   }
   FloatWavePartial<D, BF16KV> part;
   part.m = -INFINITY;
   part.z = 0.f;
 #pragma unroll
   for (int e = 0; e < G::kEpc; ++e) part.acc[e] = 0.f;
-  if (n > 0) fwave_attention_window<D, BF16KV>(a, row, t0, n, qr, lane, part);
+  float qr[G::kEpc];
+  auto early = [&]() {
+    widen<G::kEpc>(q_raw, a.q_dtype, qr);
+    write();
+  };
+  if (n > 0) fwave_attention_window<D, BF16KV, 2>(a, row, t0, n, qr, lane, part, early);
+  else early();
+  const uint32_t ldev = __builtin_amdgcn_readfirstlane(l_raw);
   bool valid;
   if constexpr (STEP) {
-    valid = ldev == t.past[b] && t.past[b] < a.size && t.past[b] + 1 <= a.span;
+    valid = ldev == u.past && u.past < a.size && u.past + 1 <= a.span;
     // A device length that differs from the host copy the table was built
     // from: the row gives NaN, and a decode step says why in its flags.
-    if (ldev != t.past[b] && lane == 0 && a.flags) atomicOr(a.flags, 4u);
+    if (ldev != u.past && lane == 0 && a.flags) atomicOr(a.flags, 4u);
   } else {
-    valid = len > 0 && ldev == t.past[b];
+    valid = u.len > 0 && ldev == u.past;
   }
   if (cur) {
-    float d = 0.f;
+    float kx[G::kEpc], vx[EPL], d = 0.f;
+    widen<G::kEpc>(kx_raw, a.new_dtype, kx);
+    widen<EPL>(vx_raw, a.new_dtype, vx);
+    if constexpr (BF16KV) {
+#pragma unroll
+      for (int e = 0; e < G::kEpc; ++e) kx[e] = bf16_to_f32(f32_to_bf16_bits(kx[e]));
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) vx[e] = bf16_to_f32(f32_to_bf16_bits(vx[e]));
+    }
 #pragma unroll
     for (int e = 0; e < G::kEpc; ++e) d = fmaf(qr[e], kx[e], d);
     const float s_cur = token_sum<G::kLpt>(d) * a.scale_log2;
@@ -2385,14 +2327,14 @@ __device__ __forceinline__ void fdecode_flat_body(const ppk::FloatDecodeFlatArgs
 #pragma unroll
     for (int e = 0; e < EPL; ++e) part.acc[e] = fmaf(part.acc[e], w1, wc * vx[e]);
   }
-  if (units == 1) {
+  if (whole) {
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
       const float o = (valid && part.z > 0.f) ? part.acc[e] / part.z : __builtin_nanf("");
       store_elem(a.out, size_t(row) * D + size_t(ch + e), a.out_dtype, o);
     }
-  } else if (slot < a.ngroups) {  // always, by the host's count of slots
-    const size_t rec = size_t(row) * a.ngroups + slot;
+  } else if (u.slot < a.ngroups) {  // always, by the host's count of slots
+    const size_t rec = size_t(row) * a.ngroups + u.slot;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a.part_y[rec * D + size_t(ch + e)] = part.acc[e];
     if (lane == 0) {
@@ -2409,25 +2351,34 @@ __device__ __forceinline__ void fmerge_flat_body(const ppk::FloatMergeFlatArgs& 
   const ppk::FloatMergeArgs& a = fa.m;
   const ppk::FlatTable& t = fa.t;
   constexpr int EPL = D / ppk::kWave;
+  __asm__ volatile("" ::"s"(a.lengths), "s"(a.part_y), "s"(a.part_mz), "s"(a.out), "s"(a.q), "s"(a.k_new),
+                   "s"(a.v_new), "s"(a.size), "s"(a.nsplits), "s"(a.out_dtype), "s"(a.span), "s"(a.step),
+                   "s"(a.q_dtype), "s"(a.new_dtype), "s"(a.kv_bf16), "s"(a.scale_log2), "s"(a.head_div.mul),
+                   "s"(a.head_div.shift));
   const int lane = threadIdx.x;
   const uint32_t row = blockIdx.x;
   const uint32_t b = fast_div(row, a.head_div);
-  const uint32_t units = t.units[b];
+  const ppk::FlatSequence seq = t.seq[b];
+  const uint32_t units = seq.units & 0xffffffu;
   if (units < 2) return;  // uniform per wave
-  const uint32_t ldev = a.lengths[b + lane_zero()];
+  uint32_t l_raw = 0;
   float m, zsum, y[EPL];
   FloatMergeCurrent<D> cur;
+  auto request = [&]() {
+    cur.request(a, row, lane);
+    l_raw = a.lengths[b + lane_zero()];
+  };
   combine_records<D>(a.part_mz + size_t(row) * a.nsplits * 2, a.part_y + size_t(row) * a.nsplits * D,
-                     min(units, a.nsplits), lane, [&]() { cur.request(a, row, lane); },
-                     [&]() { return cur.score(a); }, m, zsum, y);
+                     min(units, a.nsplits), lane, request, [&]() { return cur.score(a); }, m, zsum, y);
+  const uint32_t ldev = __builtin_amdgcn_readfirstlane(l_raw);
   if (a.step) {
     const float wc = __builtin_amdgcn_exp2f(cur.s_cur - m);
     zsum += wc;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) y[e] = fmaf(wc, cur.vcur[e], y[e]);
   }
-  const bool valid = a.step ? (ldev == t.past[b] && t.past[b] < a.size && t.past[b] + 1 <= a.span)
-                            : (t.len[b] > 0 && ldev == t.past[b]);
+  const bool valid = a.step ? (ldev == seq.past && seq.past < a.size && seq.past + 1 <= a.span)
+                            : (seq.len > 0 && ldev == seq.past);
   const size_t base = size_t(row) * D + size_t(lane) * EPL;
 #pragma unroll
   for (int e = 0; e < EPL; ++e)
