@@ -146,6 +146,37 @@ DeviceGuard::~DeviceGuard() {
   if (changed_ && previous_ >= 0) (void)hipSetDevice(previous_);
 }
 
+// The most tokens of one wave's batches (four tiles, `batch` tokens) when its
+// share is `split` tokens: whole batches, and from six batches on (where they
+// are taken two at a time) whole pairs.
+static uint32_t score_tokens(uint32_t split, uint32_t batch) {
+  const uint32_t unit = split > 5 * batch ? 2 * batch : batch;
+  return (split + unit - 1) / unit * unit;
+}
+
+// How a row's waves take its batches, by the batches of one wave's share
+// (q = ceil(split / batch)). Shares of six batches or more within 1/16 of
+// whole pairs: two batches at a time in turn. Shares of three, at least 2.5
+// batches: one contiguous range per wave (the whole of K is in flight at
+// once, and turns only mix the waves' pages). Others: one batch at a time.
+// Same-box A/B, H = 16, us per step, contiguous ranges / turns of one / turns
+// of two / turns of four: B = 32 x 8192 D = 128 161.2 / 159.1 / 160.3 /
+// 161.3, D = 64 89.0 / 85.7 / 86.6 / 86.6; B = 16 x 4096 D = 128 46.3 / 44.5 /
+// 43.9 / 44.5, x 3000 32.8 / 35.1 / 32.9 / 33.5, x 1500 18.3 / 19.7 / 18.3 / -,
+// x 1400 (5.5 batches) 17.3 / 16.9 / 17.7 / -; B = 32 x 1100 (9 batches) 25.0
+// / 24.3 / 26.1 / -; D = 64, B = 16 x 1500 (three batches) 10.8 / 11.3 / - /
+// -, x 1600 (3.25) 13.2 / 11.5 / - / -, x 300..700 7.4 / 6.8 / - / -.
+static Turns plan_turns(const AttentionPlan& p, uint32_t batch) {
+  Turns t;
+  const uint32_t q = (p.split + batch - 1) / batch;
+  const uint32_t pairs = (p.split + 2 * batch - 1) / (2 * batch) * 2 * batch;
+  t.shift = q >= 6 && 16 * (pairs - p.split) <= p.split ? 1 : q == 3 && 2 * p.split >= 5 * batch ? 31 : 0;
+  t.chunk = t.shift == 31 ? 3 : 1u << t.shift;
+  t.tokens = score_tokens(p.split, batch);
+  t.div = fast_divisor(p.ngroups * p.waves);
+  return t;
+}
+
 AttentionPlan plan_rows(const ppk_context* ctx, uint32_t rows, uint64_t span, uint32_t explicit_split,
                         uint32_t tpl, uint64_t token_bytes, uint32_t head_dim, uint32_t min_split,
                         uint32_t block_waves) {
@@ -194,8 +225,12 @@ AttentionPlan plan_rows(const ppk_context* ctx, uint32_t rows, uint64_t span, ui
     }
   }
   uint64_t waves_per_row = std::max<uint64_t>(1, (span + split - 1) / split);
-  // Up to block_waves waves per block; one float of LDS per history token of the block.
-  uint64_t max_waves = std::max<uint64_t>(1, std::min<uint64_t>(block_waves, 16384 / split));
+  // Up to block_waves waves per block; a wave keeps one float of LDS per token
+  // of its batches (score_tokens), 64 KiB per block.
+  auto lds_waves = [&](uint32_t s) {
+    return std::max<uint64_t>(1, std::min<uint64_t>(block_waves, 16384 / score_tokens(s, 4 * tpl)));
+  };
+  uint64_t max_waves = lds_waves(split);
   const uint64_t cus = uint64_t(std::max(ctx ? ctx->cu_count : 256, 1));
   const uint64_t row_bytes = span * token_bytes;
   if (!explicit_split && rows < cus && row_bytes > (128u << 10)) {
@@ -233,7 +268,7 @@ AttentionPlan plan_rows(const ppk_context* ctx, uint32_t rows, uint64_t span, ui
            rows * ((span + split / 2 - 1) / (split / 2)) <= budget) {
       split /= 2;
       waves_per_row = std::max<uint64_t>(1, (span + split - 1) / split);
-      max_waves = std::max<uint64_t>(1, std::min<uint64_t>(block_waves, 16384 / split));
+      max_waves = lds_waves(split);
       w = fit(std::max<uint64_t>(1, std::min<uint64_t>(max_waves, (256u << 10) / (uint64_t(split) * token_bytes))));
       while (w > 1 && rows * ((waves_per_row + w - 1) / w) < cus) w = shrink(w);
     }
@@ -356,7 +391,7 @@ AttentionPlan plan_rows(const ppk_context* ctx, uint32_t rows, uint64_t span, ui
       while (p * 2 <= waves_per_row) p *= 2;
       split = uint32_t(std::max<uint64_t>(((span + p - 1) / p + tpl - 1) / tpl * tpl, tpl));
       waves_per_row = std::max<uint64_t>(1, (span + split - 1) / split);
-      max_waves = std::max<uint64_t>(1, std::min<uint64_t>(block_waves, 16384 / split));
+      max_waves = lds_waves(split);
     } else if (two_rounds || (excess(max_waves) > limit && 20 * rows <= 17 * per_cu * cus)) {
       // The largest blocks (powers of two for int8) within the excess, else
       // the smallest excess.
@@ -396,9 +431,9 @@ AttentionPlan plan_rows(const ppk_context* ctx, uint32_t rows, uint64_t span, ui
     plan.waves = uint32_t((waves_per_row + plan.ngroups - 1) / plan.ngroups);
   }
   require(uint64_t(plan.ngroups) * rows <= 0x7fffffffu, "attention grid too large");
-  // Per wave: one log2-domain score per token; after the waves are done the
-  // same LDS holds one (m, z, pad, pad, y[D]) record per wave.
-  plan.lds_bytes = 4u * std::max<uint32_t>(plan.waves * split, plan.waves * (head_dim + 4u));
+  // Per wave: one log2-domain score per token of its batches; after the waves
+  // are done the same LDS holds one (m, z, pad, pad, y[D]) record per wave.
+  plan.lds_bytes = 4u * plan.waves * std::max<uint32_t>(score_tokens(split, 4 * tpl), head_dim + 4u);
   if (plan.ngroups > 1) {
     plan.y_bytes = (uint64_t(rows) * plan.ngroups * head_dim * 4 + 255) / 256 * 256;
     plan.mz_bytes = (uint64_t(rows) * plan.ngroups * 2 * 4 + 255) / 256 * 256;
@@ -456,6 +491,7 @@ AttentionPlan plan_attention(const ppk_context* ctx, const PpkAttentionArgs& a) 
     }
   }
   if (!plan.flat) {
+    plan.turn = plan_turns(plan, 4 * tpl);
     plan.speculate = per_row_speculates(plan, a.rows, a.heads, host, cover, limit);
     plan.span = uint32_t(span);
   }
@@ -468,11 +504,11 @@ uint64_t row_cover(const uint32_t* host, uint32_t batch, uint64_t limit) {
 
 bool per_row_speculates(const AttentionPlan& p, uint32_t rows, uint32_t heads, const uint32_t* host, uint64_t span,
                         uint64_t limit) {
-  const uint64_t per_row = uint64_t(p.ngroups) * p.waves;
+  const uint64_t per_row = uint64_t(p.ngroups) * p.waves, batch = 4096 / p.head_dim;
   uint64_t live = 0;
   for (uint32_t b = 0; b < rows / heads; ++b) {
     const uint64_t len = host ? (host[b] <= limit ? host[b] : 0) : span;
-    live += heads * std::min<uint64_t>(per_row, (len + p.split - 1) / p.split);
+    live += heads * std::min<uint64_t>(per_row, (len + batch - 1) / batch);
   }
   const uint64_t total = per_row * rows;
   return (total - live) * 16 < total;
@@ -839,6 +875,7 @@ void run_attention(ppk_context* ctx, hipStream_t stream, const PpkAttentionArgs&
   d.capacity = a.capacity;
   d.split_tokens = plan.split;
   d.ngroups = plan.ngroups;
+  d.turn = plan.turn;
   d.q_dtype = a.q_dtype;
   d.scratch_dtype = a.scratch_dtype;
   d.out_dtype = a.out_dtype;

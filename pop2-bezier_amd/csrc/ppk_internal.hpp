@@ -178,6 +178,7 @@ struct AttentionPlan {
   // row's length arrives (off when 1/16 or more of the waves are known to
   // have no history).
   bool speculate = true;
+  Turns turn{};          // per-row int8 plan: how a row's waves take its batches
   uint32_t blocks = 0;   // flat: blocks launched
   uint32_t span = 0;     // flat: rows with past beyond it give NaN
   FlatTable table{};

@@ -84,9 +84,19 @@ constexpr uint32_t kWaveClockDecode = 1;  // 0 entry, 1 first loads issued, 2 pa
                                           // 4 stream done, 5 block joined, 6 output / record stored
 constexpr uint32_t kWaveClockMerge = 2;   // 0 entry, 1 records combined, 2 output stored
 
+// How the ngroups * W waves of a row of the per-row int8 plan take its batches
+// (four load tiles each): chunks of chunk = 2^shift batches in turn, or, with
+// shift 31, one contiguous range of `chunk` batches per wave.
+struct Turns {
+  uint32_t shift, chunk;
+  uint32_t tokens;          // the most tokens of one wave's batches
+  FastDiv div;              // by the waves of a row
+};
+
 // Decode attention: block (group g, row r), blockIdx.x = g * rows + r, of
-// W = blockDim.x / 64 waves covers history tokens [g*W*S, (g+1)*W*S) of row r,
-// S = split_tokens per wave.
+// W = blockDim.x / 64 waves; the ngroups * W waves of row r, S = split_tokens
+// each, cover its first ngroups * W * S history tokens and take its batches of
+// four load tiles in turn.
 // ngroups == 1: the block writes the final output row (current token included).
 // ngroups > 1: it writes a partial record for the merge kernel:
 //   y[D] floats at part_y + (row * ngroups + g) * D
@@ -115,6 +125,7 @@ struct DecodeArgs {
                             // plan, a past[b] <= span past the plan's coverage flags stale host lengths
   uint32_t speculate;       // per-row plan: request each wave's first K batches before past[] arrives
   FastDiv row_div, head_div;  // by rows, by heads
+  Turns turn;               // per-row plan
   uint32_t clock_seq;       // wave-clock builds only: the launch's sequence number in the records
   uint32_t clock_cap;       // wave-clock builds only: records the buffer holds (from its size on the host)
   uint64_t* clock;          // wave-clock builds only (kWaveClock*): record buffer, or null

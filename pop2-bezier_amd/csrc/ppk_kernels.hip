@@ -131,6 +131,15 @@ __device__ __forceinline__ void load_raw(const void* p, size_t i, uint32_t dtype
     __builtin_memcpy(r.w, __builtin_assume_aligned(static_cast<const uint16_t*>(p) + i, 2), 2 * N);
   }
 }
+// Waits for r's loads here. A kernel that loads an operand on some of its
+// paths only settles it before its streaming loop: the compiler would
+// otherwise keep those loads pending into the loop and, when it reuses their
+// registers there, wait for everything in flight.
+template <int N>
+__device__ __forceinline__ void settle(const RawVec<N>& r) {
+#pragma unroll
+  for (int e = 0; e < N; ++e) __asm__ volatile("" ::"v"(r.w[e]));
+}
 template <int N>
 __device__ __forceinline__ void widen(const RawVec<N>& r, uint32_t dtype, float (&x)[N]) {
 #pragma unroll
@@ -146,10 +155,9 @@ __device__ __forceinline__ void widen(const RawVec<N>& r, uint32_t dtype, float 
 // Round-to-nearest-even to bfloat16, returned as the 16 stored bits. NaN stays
 // a quiet NaN (the carry trick alone could turn some NaN payloads into Inf).
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float x) {
-  if (x != x) return 0x7fc0u;
-  uint32_t u = __float_as_uint(x);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return uint16_t(u >> 16);
+  const uint32_t u = __float_as_uint(x);
+  const uint32_t rounded = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+  return uint16_t(x != x ? 0x7fc0u : rounded);
 }
 // The same rounding kept in fp32 (the value a bf16 tensor would hold).
 __device__ __forceinline__ float round_bf16(float x) {
@@ -180,6 +188,12 @@ __device__ __forceinline__ void store_elem(void* p, size_t i, uint32_t dtype, fl
   else static_cast<uint16_t*>(p)[i] = dtype == kBF16 ? f32_to_bf16_bits(x) : f32_to_f16_bits(x);
 }
 
+// Loads above this line are issued before anything below it (both the
+// optimiser and the scheduler would otherwise move them down to their use).
+__device__ __forceinline__ void issue_here() {
+  __asm__ volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
 // x / d for x < 2^31 by the host's precomputed FastDiv of d (scalar: one
 // multiply-high and a shift, where the compiler's division takes ~30
 // dependent instructions, on the path of every wave's first load).
@@ -366,12 +380,23 @@ __device__ __forceinline__ float lane_absmax(const float (&x)[N]) {
 // NaN quotients become code 0 (as a float->int conversion of NaN does on
 // the reference GPU path); the absmax ignores NaN like fmaxf / f32::max.
 // ---------------------------------------------------------------------------
+// ORs `bits` (PPK_FLAG_*, uniform) into *flags, if there is one and any bit is
+// set. Every lane issues the atomic (the same bits; a rare path): see
+// quantize_values on branches on the lane, which the compiler's own atomic
+// would bring back.
+__device__ __forceinline__ void raise_flags(uint32_t* flags, uint32_t bits) {
+  if (flags && bits) __asm__ volatile("global_atomic_or %0, %1, off" ::"v"(flags), "v"(bits) : "memory");
+}
+
 // Quantise one row of D values into codes[0..D) and *scale; the whole wave
 // participates, lane l holding elements l*D/64 ... (l+1)*D/64 - 1 of the
-// row. A non-finite value is reported through flags when given.
+// row. Returns whether any value was non-finite. Every lane stores the scale
+// (one value at one address): a lane-0 branch here would make the compiler
+// restructure the control flow around it, and the decode kernels' streaming
+// loops then wait for loads of paths that never reach them.
 template <int D>
-__device__ __forceinline__ void quantize_values(const float (&x)[D / ppk::kWave], uint8_t* codes, float* scale,
-                                                uint32_t* flags, int lane) {
+__device__ __forceinline__ bool quantize_values(const float (&x)[D / ppk::kWave], uint8_t* codes, float* scale,
+                                                int lane) {
 #pragma clang fp contract(off)
   constexpr int EPL = D / ppk::kWave;
   bool finite = true;
@@ -390,11 +415,8 @@ __device__ __forceinline__ void quantize_values(const float (&x)[D / ppk::kWave]
   if constexpr (EPL == 1) *out = uint8_t(packed);
   else if constexpr (EPL == 2) *reinterpret_cast<uint16_t*>(out) = uint16_t(packed);
   else *reinterpret_cast<uint32_t*>(out) = packed;
-  if (lane == 0) *scale = s;
-  if (flags) {
-    const bool any_bad = __any(!finite);
-    if (any_bad && lane == 0) atomicOr(flags, 1u);
-  }
+  *scale = s;
+  return __any(!finite);
 }
 
 // The same for row src_row of src[rows, D] in dtype.
@@ -404,7 +426,7 @@ __device__ __forceinline__ void quantize_row(const void* src, size_t src_row, ui
   constexpr int EPL = D / ppk::kWave;
   float x[EPL];
   load_vec<EPL>(src, src_row * D + size_t(lane) * EPL, dtype, x);
-  quantize_values<D>(x, codes, scale, flags, lane);
+  if (quantize_values<D>(x, codes, scale, lane) && flags && lane == 0) atomicOr(flags, 1u);
 }
 
 template <int D>
@@ -516,9 +538,9 @@ __device__ __forceinline__ void dequantize_body(const ppk::DequantizeArgs& a) {
 }
 
 // ---------------------------------------------------------------------------
-// Kernel 2a: decode attention. A block of W waves covers W*S consecutive
-// history tokens of one row (group g of the row); each wave streams its own S
-// tokens, the block combines its waves through LDS. With one group per row
+// Kernel 2a: decode attention. A row is covered by G blocks (groups) of W waves
+// of S tokens each; its waves take its batches in turn (Batches below), the
+// block combines its waves through LDS. With one group per row
 // the block also scores the current token and writes the final output, so a
 // decode step is a single launch; otherwise it writes a partial (m, z, y)
 // record for the merge kernel. Optionally the block first quantises the new
@@ -902,20 +924,29 @@ __device__ __forceinline__ void tile_accumulate(const u4& raw, float p, float vs
   }
 }
 
-// Phase K for one batch of U tiles: scores (log2 domain) into LDS, running max.
+// Phase K for one batch of U tiles: scores (log2 domain) into LDS, running
+// max. The tiles' scales are fetched together and the lanes of chunk c store
+// tile c % 4's scores, one unmasked write for the batch: with a fetch and a
+// masked write per tile, each tile waited for its own LDS round trip, and the
+// branch on the lane made the compiler restructure the kernel (see
+// quantize_values).
 template <int D, bool BF16H, int U>
 __device__ __forceinline__ float score_batch(const u4 (&raw)[U], float scale_lane, uint32_t t0, uint32_t n, int j,
-                                             int c, const Query<BF16H>& q, float* s_lds, float mloc) {
+                                             int c, const Query<BF16H>& q, float* s_batch, float mloc) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
+  static_assert(U == 4 && LPT >= U, "a lane of each token per tile");
+  float kscale[U], s[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) kscale[u] = __shfl(scale_lane, u * TPL + j);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const uint32_t tok = (t0 + u) * TPL + j;
-    float sc = tile_score<D, BF16H>(raw[u], __shfl(scale_lane, u * TPL + j), q);
-    sc = tok < n ? sc : -INFINITY;
-    mloc = fmaxf(mloc, sc);
-    if (c == 0 && tok < n) s_lds[tok] = sc;
+    const float x = tile_score<D, BF16H>(raw[u], kscale[u], q);
+    s[u] = (t0 + u) * TPL + j < n ? x : -INFINITY;
+    mloc = fmaxf(mloc, s[u]);
   }
+  const float lo = (c & 1) ? s[1] : s[0], hi = (c & 1) ? s[3] : s[2];
+  s_batch[(c & 3) * TPL + j] = (c & 2) ? hi : lo;
   return mloc;
 }
 
@@ -925,42 +956,83 @@ __device__ __forceinline__ float score_batch(const u4 (&raw)[U], float scale_lan
 // token's weight with one cross-lane read and accumulate weight * code.
 template <int D, bool BF16H, int U>
 __device__ __forceinline__ void accumulate_batch(const u4 (&raw)[U], float scale_lane, uint32_t t0, uint32_t n, int j,
-                                                 int lane, float m, const float* s_lds, float& z, float (&acc)[16]) {
+                                                 int lane, float m, const float* s_batch, float& z,
+                                                 float (&acc)[16]) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
   constexpr int TPB = U * TPL;  // tokens per batch (<= 64)
   static_assert(TPB <= ppk::kWave, "one scale per lane per batch");
-  const uint32_t tl = t0 * TPL + uint32_t(lane % TPB);
-  const float e = __builtin_amdgcn_exp2f(s_lds[min(tl, n - 1)] - m);
-  const float pr = (tl < n && lane < TPB) ? e : 0.f;
+  const float e = __builtin_amdgcn_exp2f(s_batch[lane % TPB] - m);
+  const float pr = (t0 * TPL + uint32_t(lane % TPB) < n && lane < TPB) ? e : 0.f;
   z += pr;
   const float w_lane = BF16H ? pr : pr * scale_lane;
+  float wgt[U], vscale[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const float wgt = __shfl(w_lane, u * TPL + j);
-    const float vscale = BF16H ? __shfl(scale_lane, u * TPL + j) : 1.f;
-    tile_accumulate<BF16H>(raw[u], wgt, vscale, acc);
+  for (int u = 0; u < U; ++u) {  // all four fetched before the first is used
+    wgt[u] = __shfl(w_lane, u * TPL + j);
+    vscale[u] = BF16H ? __shfl(scale_lane, u * TPL + j) : 1.f;
   }
+#pragma unroll
+  for (int u = 0; u < U; ++u) tile_accumulate<BF16H>(raw[u], wgt[u], vscale[u], acc);
+}
+
+// The wave's batches of a row of n tokens (DecodeArgs::turn): chunks of 2^shift
+// batches, the row's waves taking the row's chunks in turn. Every wave of every
+// block of the row then has the same share whatever the row's length (a short
+// row of a ragged batch no longer fills its first waves and leaves the others
+// idle until the block's join), and at any time a block's waves read one
+// contiguous stretch, where ranges of a power of two bytes per wave moved
+// through the same memory channels in step. One chunk per wave (shift 31)
+// gives each wave a contiguous range of `chunk` batches. The host picks by
+// the waves' share, see plan_attention.
+struct Batches {
+  uint32_t first, step, shift;  // chunk k starts at batch first + k * step
+  uint32_t count;               // batches of this wave
+  uint32_t end;                 // batches of the row: the place past the last one
+  // The first tile of batch i; past this wave's last one, the first tile past the row's end.
+  __device__ __forceinline__ uint32_t tile(uint32_t i) const {
+    const uint32_t k = i >> shift;
+    return 4 * (i < count ? first + k * step + (i - (k << shift)) : end);
+  }
+};
+template <int TPB>
+__device__ __forceinline__ Batches row_batches(const ppk::DecodeArgs& a, uint32_t n, uint32_t place, uint32_t turns) {
+  const uint32_t end = n / TPB + (n % TPB != 0 ? 1u : 0u);
+  if (a.turn.shift == 31) {
+    const uint32_t first = place * a.turn.chunk;
+    return Batches{first, 0, 31, end > first ? min(end - first, a.turn.chunk) : 0u, end};
+  }
+  const uint32_t chunks = (end + a.turn.chunk - 1) >> a.turn.shift;
+  uint32_t count = 0;
+  if (chunks > place) {
+    const uint32_t last = fast_div(chunks - place - 1, a.turn.div);  // this wave's last chunk
+    count = (last + 1) << a.turn.shift;
+    if (place + last * turns == chunks - 1) count -= (chunks << a.turn.shift) - end;  // the row's last, cut short
+  }
+  return Batches{place << a.turn.shift, turns << a.turn.shift, a.turn.shift, count, end};
 }
 
 // A stream of at most NBATCH batches per phase, K and V already requested:
 // scores, weights and sums stay in the registers of the token groups (no LDS
-// round trip between the phases). Tokens at or past n may hold anything: their
-// scores are masked and their V scales zeroed.
+// round trip between the phases). Tokens at or past the row's length n may
+// hold anything: their scores are masked and their V scales zeroed.
 template <int D, bool BF16H, int NBATCH, int NB>
 __device__ __forceinline__ void short_attention(const u4 (&k)[NB][4], const float (&ks)[NB], const u4 (&v)[2][4],
-                                                const float (&vs)[2], uint32_t n, int lane, const Query<BF16H>& q,
-                                                WavePartial& out) {
+                                                const float (&vs)[2], const Batches& bt, uint32_t n, int lane,
+                                                const Query<BF16H>& q, WavePartial& out) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
   constexpr int TPB = 4 * TPL;
   const int j = lane / LPT;
   PPK_CLK_AT(out.t_first, k[0][0][0]);
+  uint32_t tok[NBATCH];  // the batches' first tokens
+#pragma unroll
+  for (int b = 0; b < NBATCH; ++b) tok[b] = bt.tile(uint32_t(b)) * TPL;
   float sc[NBATCH][4], vsc[NBATCH][4];
   float m = -INFINITY;
 #pragma unroll
   for (int b = 0; b < NBATCH; ++b) {
-    const float vl = uint32_t(b * TPB + lane % TPB) < n ? vs[b] : 0.f;
+    const float vl = tok[b] + uint32_t(lane % TPB) < n ? vs[b] : 0.f;
 #pragma unroll
     for (int u = 0; u < 4; ++u) vsc[b][u] = __shfl(vl, u * TPL + j);
   }
@@ -972,7 +1044,7 @@ __device__ __forceinline__ void short_attention(const u4 (&k)[NB][4], const floa
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const float x = tile_score<D, BF16H>(k[b][u], kscale[u], q);
-      sc[b][u] = uint32_t((b * 4 + u) * TPL + j) < n ? x : -INFINITY;
+      sc[b][u] = tok[b] + uint32_t(u * TPL + j) < n ? x : -INFINITY;
       m = fmaxf(m, sc[b][u]);
     }
   }
@@ -985,7 +1057,7 @@ __device__ __forceinline__ void short_attention(const u4 (&k)[NB][4], const floa
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const float e = __builtin_amdgcn_exp2f(sc[b][u] - m);
-      const float p = uint32_t((b * 4 + u) * TPL + j) < n ? e : 0.f;
+      const float p = tok[b] + uint32_t(u * TPL + j) < n ? e : 0.f;
       z += p;
       tile_accumulate<BF16H>(v[b][u], p, vsc[b][u], out.acc);
     }
@@ -994,7 +1066,7 @@ __device__ __forceinline__ void short_attention(const u4 (&k)[NB][4], const floa
   reduce_scatter_groups<LPT, 16>(out.acc, lane);
 }
 
-// Streams this wave's n tokens (n beyond two batches per phase): phase K
+// Streams this wave's batches (more than two) of a row of n tokens: phase K
 // scores, phase V accumulation. A ring of NB batches (rr[b], rs[b]) keeps NB -
 // 1 batches' loads in flight while one is consumed: batch i of the sequence
 // K_0 .. K_{nb-1}, (padding to a whole ring), V_0 .. V_{nb-1} lives in slot
@@ -1010,28 +1082,31 @@ __device__ __forceinline__ void short_attention(const u4 (&k)[NB][4], const floa
 // arithmetic of batches past the end is skipped (uniform branches).
 template <int D, bool BF16H, int NB>
 __device__ __forceinline__ void ring_attention(const uint8_t* kb, const uint8_t* vb, const float* ksb,
-                                               const float* vsb, uint32_t n, const Query<BF16H>& q, float* s_lds,
-                                               int lane, WavePartial& out, u4 (&rr)[NB][4], float (&rs)[NB]) {
+                                               const float* vsb, const Batches& bt, uint32_t n,
+                                               const Query<BF16H>& q, float* s_lds, int lane, WavePartial& out,
+                                               u4 (&rr)[NB][4], float (&rs)[NB]) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
   constexpr int U = 4;  // tiles per batch
+  constexpr int TPB = U * TPL;
   const int j = lane / LPT;  // token within a load tile
   const int c = lane % LPT;  // 16-channel chunk
 #pragma unroll
   for (int i = 0; i < 16; ++i) out.acc[i] = 0.f;
   float mloc = -INFINITY, z = 0.f;
-  const uint32_t nb = ((n + TPL - 1) / TPL + U - 1) / U;  // K batches (and V batches)
-  const uint32_t nbp = (nb + NB - 1) / NB * NB;           // rounded up to whole rings
+  const uint32_t nb = bt.count;                  // K batches (and V batches)
+  const uint32_t nbp = (nb + NB - 1) / NB * NB;  // rounded up to whole rings
   PPK_CLK_AT(out.t_first, rr[0][0][0]);
   for (uint32_t k0 = 0; k0 < nbp; k0 += NB) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const uint32_t i = k0 + uint32_t(b);
-      if (i < nb) mloc = score_batch<D, BF16H, U>(rr[b], rs[b], i * U, n, j, c, q, s_lds, mloc);
+      if (i < nb) mloc = score_batch<D, BF16H, U>(rr[b], rs[b], bt.tile(i), n, j, c, q, s_lds + i * TPB, mloc);
       // Refill slot b with item i + NB: K batch i + NB, or V batch i + NB - nbp.
       const bool isv = i + NB >= nbp;
-      load_batch<D, U>(isv ? vb : kb, isv ? vsb : ksb, (isv ? i + NB - nbp : i + NB) * U, n, j, lane, rr[b],
+      load_batch<D, U>(isv ? vb : kb, isv ? vsb : ksb, bt.tile(isv ? i + NB - nbp : i + NB), n, j, lane, rr[b],
                        rs[b]);
+      issue_here();  // the refill goes out before the next batch is used
     }
   }
   const float m = groups_max<LPT>(mloc);
@@ -1040,8 +1115,9 @@ __device__ __forceinline__ void ring_attention(const uint8_t* kb, const uint8_t*
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const uint32_t i = v0 + uint32_t(b);
-      if (i < nb) accumulate_batch<D, BF16H, U>(rr[b], rs[b], i * U, n, j, lane, m, s_lds, z, out.acc);
-      load_batch<D, U>(vb, vsb, (i + NB) * U, n, j, lane, rr[b], rs[b]);  // past the end on the last ring
+      if (i < nb) accumulate_batch<D, BF16H, U>(rr[b], rs[b], bt.tile(i), n, j, lane, m, s_lds + i * TPB, z, out.acc);
+      load_batch<D, U>(vb, vsb, bt.tile(i + NB), n, j, lane, rr[b], rs[b]);  // past the end on the last ring
+      issue_here();
     }
   }
   // Each token's p was added once, by its owning lane: sum over the wave.
@@ -1057,10 +1133,8 @@ __device__ __forceinline__ void write_block_record(float* rec, int ch, int lane,
                                                    const float (&acc)[N]) {
 #pragma unroll
   for (int e = 0; e < D / ppk::kWave; ++e) rec[4 + ch + e] = acc[e];
-  if (lane == 0) {
-    rec[0] = m;
-    rec[1] = z;
-  }
+  rec[0] = m;  // the same in every lane, as below wherever a wave's (m, z) is stored
+  rec[1] = z;
 }
 
 // Log-sum-exp combine of a block's W <= MAXW records (stride floats apart) and
@@ -1126,7 +1200,7 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
                    "s"(a.k_new), "s"(a.v_new), "s"(a.rows), "s"(a.capacity), "s"(a.split_tokens), "s"(a.ngroups),
                    "s"(a.q_dtype), "s"(a.scratch_dtype), "s"(a.new_dtype), "s"(a.append), "s"(a.speculate),
                    "s"(a.row_div.mul), "s"(a.row_div.shift), "s"(a.head_div.mul), "s"(a.head_div.shift),
-                   "s"(blockDim.x));
+                   "s"(a.turn.div.mul), "s"(a.turn.div.shift), "s"(a.turn.shift), "s"(a.turn.chunk), "s"(blockDim.x));
   const int lane = threadIdx.x & 63;
   // The wave index is uniform: in a scalar register, every quantity derived
   // from it (the wave's range, its length, its batch counts) is too, and the
@@ -1175,34 +1249,50 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   if (kw) load_raw<EPL>(a.k_new, first, a.new_dtype, kn_raw);
   if (vw) load_raw<EPL>(a.v_new, first, a.new_dtype, vn_raw);
 
-  const uint32_t begin = (group * W + wave) * S;
-  const uint32_t nspec = (a.speculate && begin < a.capacity) ? min(S, a.capacity - begin) : 0u;
-  const size_t tok0 = size_t(row) * a.capacity + begin;
+  // This wave's batches of the row: those of the longest row the plan covers,
+  // until the length is known.
+  constexpr int TPB = U * TPL;
+  const uint32_t place = group * W + wave, turns = a.ngroups * W;
+  const uint64_t cover = uint64_t(turns) * S;
+  const uint32_t nspec = a.speculate ? uint32_t(min(uint64_t(a.capacity), cover)) : 0u;
+  const Batches early = row_batches<TPB>(a, nspec, place, turns);
+  const size_t tok0 = size_t(row) * a.capacity;
   const uint8_t* kb = a.k + tok0 * D + size_t(c) * 16;
   const uint8_t* vb = a.v + tok0 * D + size_t(c) * 16;
   const float* ksb = a.ks + tok0;
   const float* vsb = a.vs + tok0;
   // LDS of this wave alone: the query's exchange, then a score per token of
   // its range, at last its (m, z, pad, pad, y[D]) record.
-  const uint32_t lds_stride = max(S, uint32_t(D + 4));
+  const uint32_t lds_stride = max(a.turn.tokens, uint32_t(D + 4));
   float* s_lds = lds + size_t(wave) * lds_stride;
 
   float s_cur = -INFINITY, sv[EPL];
   bool valid = false;
-  uint32_t n = 0;
+  uint32_t n = 0;  // the row's live history
+  Batches bt{};
+  uint32_t raise = 0;  // PPK_FLAG_* bits, uniform; reported at the end (a branch on the lane here, see quantize_values)
   Query<BF16H> query;
+  auto settle_all = [&]() {
+    settle(q_raw);
+    settle(sk_raw);
+    settle(sv_raw);
+    settle(kn_raw);
+    settle(vn_raw);
+  };
   // Everything that waits for the small loads; runs with the stream's first
   // batches in flight.
   auto prologue = [&]() {
+    issue_here();
     PPK_CLK(1);
     const uint32_t p = __builtin_amdgcn_readfirstlane(p_raw);
     PPK_CLK_AFTER(2, p_raw);
-    const uint64_t cover = uint64_t(a.ngroups) * W * S;
+    settle_all();
     valid = p <= a.capacity && uint64_t(p) <= cover;
-    n = (valid && begin < p) ? min(S, p - begin) : 0u;
+    n = valid ? p : 0u;
+    bt = row_batches<TPB>(a, n, place, turns);
     float x[EPL];
     widen<EPL>(q_raw, a.q_dtype, x);
-    if (n > 0) make_query<D, BF16H>(x, a.scale_log2, s_lds, lane, query);
+    if (bt.count > 0) make_query<D, BF16H>(x, a.scale_log2, s_lds, lane, query);
     if (cur) {
       // Log2-domain score of the current token, which comes from the scratch copy, not the arena.
       float kv[EPL], d = 0.f;
@@ -1214,20 +1304,20 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
     }
     // A length within the caller's span that the plan does not cover: the plan
     // was sized from a stale host copy of the lengths (the row gives NaN).
-    if (kw && lane == 0 && a.flags && p <= a.capacity && p <= a.span && uint64_t(p) > cover) atomicOr(a.flags, 4u);
+    if (kw && p <= a.capacity && p <= a.span && uint64_t(p) > cover) raise |= 4u;
     if (kw || vw) {
       if (p >= a.capacity) {
-        if (lane == 0 && a.flags) atomicOr(a.flags, 2u);
+        raise |= 2u;
       } else {
         const size_t slot = size_t(row) * a.capacity + p;
         float t[EPL];
         if (kw) {
           widen<EPL>(kn_raw, a.new_dtype, t);
-          quantize_values<D>(t, a.k + slot * D, a.ks + slot, a.flags, lane);
+          if (quantize_values<D>(t, a.k + slot * D, a.ks + slot, lane)) raise |= 1u;
         }
         if (vw) {
           widen<EPL>(vn_raw, a.new_dtype, t);
-          quantize_values<D>(t, a.v + slot * D, a.vs + slot, a.flags, lane);
+          if (quantize_values<D>(t, a.v + slot * D, a.vs + slot, lane)) raise |= 1u;
         }
       }
     }
@@ -1240,39 +1330,46 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   for (int i = 0; i < 16; ++i) part.acc[i] = 0.f;
   u4 rr[NB][U], va[2][U];
   float rs[NB], vsa[2];
+  auto load_k = [&](int b, const Batches& of, uint32_t limit) {
+    load_batch<D, U>(kb, ksb, of.tile(uint32_t(b)), limit, j, lane, rr[b], rs[b]);
+  };
+  auto load_v = [&](int b, const Batches& of, uint32_t limit) {
+    load_batch<D, U>(vb, vsb, of.tile(uint32_t(b)), limit, j, lane, va[b], vsa[b]);
+  };
   // The paths differ in what is in flight when the prologue runs; each runs
   // its own copy of it, so that its waits count that path's loads only.
-  if (nspec > 0 && nspec <= uint32_t(U * TPL)) {
-    // A window of one batch: K and V at once, one memory round trip in all.
-    load_batch<D, U>(kb, ksb, 0, nspec, j, lane, rr[0], rs[0]);
-    load_batch<D, U>(vb, vsb, 0, nspec, j, lane, va[0], vsa[0]);
+  if (early.count == 1) {
+    // At most one batch: K and V at once, one memory round trip in all.
+    load_k(0, early, nspec);
+    load_v(0, early, nspec);
     prologue();
-    if (n > 0) short_attention<D, BF16H, 1>(rr, rs, va, vsa, n, lane, query, part);
-  } else if (nspec > 0 && nspec <= uint32_t(2 * U * TPL)) {
-    load_batch<D, U>(kb, ksb, 0, nspec, j, lane, rr[0], rs[0]);
-    load_batch<D, U>(kb, ksb, U, nspec, j, lane, rr[1], rs[1]);
-    load_batch<D, U>(vb, vsb, 0, nspec, j, lane, va[0], vsa[0]);
-    load_batch<D, U>(vb, vsb, U, nspec, j, lane, va[1], vsa[1]);
+    if (bt.count > 0) short_attention<D, BF16H, 1>(rr, rs, va, vsa, early, n, lane, query, part);
+  } else if (early.count == 2) {
+    load_k(0, early, nspec);
+    load_k(1, early, nspec);
+    load_v(0, early, nspec);
+    load_v(1, early, nspec);
     prologue();
-    if (n > 0) short_attention<D, BF16H, 2>(rr, rs, va, vsa, n, lane, query, part);
+    if (bt.count > 0) short_attention<D, BF16H, 2>(rr, rs, va, vsa, early, n, lane, query, part);
   } else {
-    if (nspec > 0) {
+    if (early.count > 0) {
 #pragma unroll
-      for (int b = 0; b < NB; ++b) load_batch<D, U>(kb, ksb, uint32_t(b) * U, nspec, j, lane, rr[b], rs[b]);
+      for (int b = 0; b < NB; ++b) load_k(b, early, nspec);
       prologue();
     } else {
       prologue();
-      if (n > 0) {
+      if (bt.count > 0) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) load_batch<D, U>(kb, ksb, uint32_t(b) * U, n, j, lane, rr[b], rs[b]);
+        for (int b = 0; b < NB; ++b) load_k(b, bt, n);
       }
     }
-    if (n > uint32_t(2 * U * TPL)) {
-      ring_attention<D, BF16H, NB>(kb, vb, ksb, vsb, n, query, s_lds, lane, part, rr, rs);
-    } else if (n > 0) {
-      load_batch<D, U>(vb, vsb, 0, n, j, lane, va[0], vsa[0]);
-      load_batch<D, U>(vb, vsb, U, n, j, lane, va[1], vsa[1]);
-      short_attention<D, BF16H, 2>(rr, rs, va, vsa, n, lane, query, part);
+    if (bt.count > 2) {
+      settle_all();  // long done, but not on every edge the compiler gives this block
+      ring_attention<D, BF16H, NB>(kb, vb, ksb, vsb, bt, n, query, s_lds, lane, part, rr, rs);
+    } else if (bt.count > 0) {
+      load_v(0, bt, n);
+      load_v(1, bt, n);
+      short_attention<D, BF16H, 2>(rr, rs, va, vsa, bt, n, lane, query, part);
     }
   }
   PPK_CLK(4);
@@ -1283,6 +1380,7 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   // Combine the block's waves through LDS: each wave's record replaces its
   // scores (its own LDS, so no barrier is needed before).
   write_block_record<D>(s_lds, c * 16 + scatter_base<LPT, 16>(lane), lane, part.m, part.z, part.acc);
+  raise_flags(a.flags, raise);
   __syncthreads();
   PPK_CLK(5);
   if (wave != 0) {
@@ -1304,10 +1402,8 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
     const size_t rec = size_t(row) * a.ngroups + group;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a.part_y[rec * D + size_t(lane) * EPL + e] = y[e];
-    if (lane == 0) {
-      a.part_mz[rec * 2] = m;
-      a.part_mz[rec * 2 + 1] = zsum;
-    }
+    a.part_mz[rec * 2] = m;
+    a.part_mz[rec * 2 + 1] = zsum;
   }
   PPK_CLK(6);
   PPK_CLK_RECORD(a, ppk::kWaveClockDecode, blockIdx.x, 0u);
@@ -1477,7 +1573,11 @@ __device__ __forceinline__ void attn_merge_body(const ppk::MergeArgs& a) {
 // every small operand travels as raw words beside the window's first pairs,
 // and the window's refills are unconditional (past the end they read the
 // unit's last token again), so that each wait is for the oldest pair only.
-// @MEASURED_FLAT@
+// Against a per-lane table search, loads widened one after another and
+// conditional refills (H = 16, host lengths): B = 8 of 256..4096 at D = 128
+// 24.5 -> 21.1 us, at D = 64 16.0 -> 14.1; B = 24 of 200..3000 at D = 64 25.0
+// -> 20.5; B = 32 of 256..4096 at D = 128 60.9 -> 56.5. Three or four pairs
+// were 1 and 5 % slower.
 // ---------------------------------------------------------------------------
 // One (K, V) batch pair of a unit under the online softmax. Token group j
 // (the LPT lanes holding one token of each tile) keeps its own running max m,
@@ -1548,6 +1648,7 @@ __device__ __forceinline__ void wave_attention_window(const uint8_t* kb, const u
       if (bi < nb) online_pair<D, BF16H>(kr[p], vr[p], ksl[p], vsl[p], bi * U, n, j, q, m, z, out.acc);
       load_batch<D, U>(kb, ksb, (bi + NP) * U, n, j, lane, kr[p], ksl[p]);
       load_batch<D, U>(vb, vsb, (bi + NP) * U, n, j, lane, vr[p], vsl[p]);
+      issue_here();
     }
   }
   // Join the token groups: common max, then sums across groups.
@@ -1622,21 +1723,24 @@ __device__ __forceinline__ void decode_flat_body(const ppk::DecodeFlatArgs& fa) 
     ap_raw = a.past[fast_div(arow, a.head_div) + lane_zero()];
     load_raw<EPL>((wid & 1u) ? a.v_new : a.k_new, size_t(arow) * D + size_t(lane) * EPL, a.new_dtype, new_raw);
   }
+  uint32_t raise = 0;  // PPK_FLAG_* bits, uniform; reported at the end
   auto commit = [&]() {
     if (!append) return;
     const uint32_t ap = __builtin_amdgcn_readfirstlane(ap_raw);
     if (ap >= a.capacity) {
-      if (lane == 0 && a.flags) atomicOr(a.flags, 2u);
+      raise |= 2u;
     } else {
       const size_t dst = size_t(arow) * a.capacity + ap;
+      const bool value = (wid & 1u) != 0;
       float x[EPL];
       widen<EPL>(new_raw, a.new_dtype, x);
-      if (wid & 1u) quantize_values<D>(x, a.v + dst * D, a.vs + dst, a.flags, lane);
-      else quantize_values<D>(x, a.k + dst * D, a.ks + dst, a.flags, lane);
+      if (quantize_values<D>(x, (value ? a.v : a.k) + dst * D, (value ? a.vs : a.ks) + dst, lane)) raise |= 1u;
     }
   };
+  auto report = [&]() { raise_flags(a.flags, raise); };
   if (wid >= t.units_total) {
     commit();
+    report();
     return;
   }
   const FlatUnit u = flat_unit(t, wid);
@@ -1662,6 +1766,10 @@ __device__ __forceinline__ void decode_flat_body(const ppk::DecodeFlatArgs& fa) 
     Query<BF16H> query;
     const size_t tok0 = size_t(row) * a.capacity + t0;
     auto early = [&]() {  // with the unit's first loads in flight
+      issue_here();
+      settle(new_raw);
+      settle(sk_raw);
+      settle(sv_raw);
       float x[EPL];
       widen<EPL>(q_raw, a.q_dtype, x);
       make_query<D, BF16H>(x, a.scale_log2, s_query[wave], lane, query);
@@ -1682,7 +1790,8 @@ __device__ __forceinline__ void decode_flat_body(const ppk::DecodeFlatArgs& fa) 
   // The row is valid when the host's length is in range and the device agrees.
   const bool host_ok = u.past <= a.capacity && u.past <= a.span;
   const bool fresh = __builtin_amdgcn_readfirstlane(p_raw) == u.past;
-  if (!fresh && lane == 0 && a.flags) atomicOr(a.flags, 4u);
+  if (!fresh) raise |= 4u;
+  report();
   if (whole) {
     const bool valid = fresh && host_ok;
     const float m = fmaxf(part.m, s_cur);
@@ -1700,10 +1809,8 @@ __device__ __forceinline__ void decode_flat_body(const ppk::DecodeFlatArgs& fa) 
     const size_t rec = size_t(row) * a.ngroups + u.slot;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a.part_y[rec * D + size_t(ch + e)] = part.acc[e];
-    if (lane == 0) {
-      a.part_mz[rec * 2] = part.m;
-      a.part_mz[rec * 2 + 1] = part.z;
-    }
+    a.part_mz[rec * 2] = part.m;
+    a.part_mz[rec * 2 + 1] = part.z;
   }
 }
 
@@ -1951,7 +2058,7 @@ template <int EPL, bool BF16KV>
 __device__ __forceinline__ void write_current(void* store, uint64_t stride, uint32_t row, uint32_t p, uint32_t size,
                                               const float (&x)[EPL], uint32_t* flags, int lane) {
   if (p >= size) {
-    if (lane == 0 && flags) atomicOr(flags, 2u);
+    raise_flags(flags, 2u);
     return;
   }
   const size_t base = size_t(row) * stride + size_t(p) * (EPL * ppk::kWave) + size_t(lane) * EPL;
@@ -1999,8 +2106,7 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
   if (cur) load_vec<EPL>(a.q, size_t(row) * a.q_stride + size_t(lane) * EPL, a.q_dtype, qcur);
   // A stored length within the span that the plan does not cover: the plan
   // was sized from a stale host copy of the lengths (the row gives NaN).
-  if (kw && lane == 0 && a.flags && len < a.size && len + 1 <= a.span && uint64_t(len) > uint64_t(a.ngroups) * W * S)
-    atomicOr(a.flags, 4u);
+  if (kw && len < a.size && len + 1 <= a.span && uint64_t(len) > uint64_t(a.ngroups) * W * S) raise_flags(a.flags, 4u);
   if (kw) write_current<EPL, BF16KV>(const_cast<void*>(a.k), a.k_stride, row, len, a.size, kcur, a.flags, lane);
   if (vw) write_current<EPL, BF16KV>(const_cast<void*>(a.v), a.v_stride, row, len, a.size, vcur, a.flags, lane);
   const uint32_t begin = (group * W + wave) * S;
@@ -2042,10 +2148,8 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
     const size_t rec = size_t(row) * a.ngroups + group;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a.part_y[rec * D + size_t(lane) * EPL + e] = y[e];
-    if (lane == 0) {
-      a.part_mz[rec * 2] = m;
-      a.part_mz[rec * 2 + 1] = zsum;
-    }
+    a.part_mz[rec * 2] = m;
+    a.part_mz[rec * 2 + 1] = zsum;
   }
 }
 
@@ -2209,6 +2313,7 @@ __device__ __forceinline__ void fwave_attention_window(const ppk::FloatDecodeArg
       if (bi < nb) fonline_pair<D, BF16KV>(kr[p], vr[p], bi * U, n, j, qr, a.scale_log2, m, z, acc);
       load_fbatch<D, BF16KV, U>(kb, (bi + NP) * U, n, j, kr[p]);
       load_fbatch<D, BF16KV, U>(vb, (bi + NP) * U, n, j, vr[p]);
+      issue_here();
     }
   }
   const float mm = groups_max<G::kLpt>(m);
@@ -2292,6 +2397,10 @@ __device__ __forceinline__ void fdecode_flat_body(const ppk::FloatDecodeFlatArgs
   for (int e = 0; e < G::kEpc; ++e) part.acc[e] = 0.f;
   float qr[G::kEpc];
   auto early = [&]() {
+    issue_here();
+    settle(new_raw);
+    settle(kx_raw);
+    settle(vx_raw);
     widen<G::kEpc>(q_raw, a.q_dtype, qr);
     write();
   };
@@ -2303,7 +2412,7 @@ __device__ __forceinline__ void fdecode_flat_body(const ppk::FloatDecodeFlatArgs
     valid = ldev == u.past && u.past < a.size && u.past + 1 <= a.span;
     // A device length that differs from the host copy the table was built
     // from: the row gives NaN, and a decode step says why in its flags.
-    if (ldev != u.past && lane == 0 && a.flags) atomicOr(a.flags, 4u);
+    if (ldev != u.past) raise_flags(a.flags, 4u);
   } else {
     valid = u.len > 0 && ldev == u.past;
   }
@@ -2337,10 +2446,8 @@ __device__ __forceinline__ void fdecode_flat_body(const ppk::FloatDecodeFlatArgs
     const size_t rec = size_t(row) * a.ngroups + u.slot;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a.part_y[rec * D + size_t(ch + e)] = part.acc[e];
-    if (lane == 0) {
-      a.part_mz[rec * 2] = part.m;
-      a.part_mz[rec * 2 + 1] = part.z;
-    }
+    a.part_mz[rec * 2] = part.m;
+    a.part_mz[rec * 2 + 1] = part.z;
   }
 }
 
