@@ -156,7 +156,8 @@ static uint32_t score_tokens(uint32_t split, uint32_t batch) {
 
 // How a row's waves take its batches, by the batches of one wave's share
 // (q = ceil(split / batch)). Shares of six batches or more within 1/16 of
-// whole pairs: two batches at a time in turn. Shares of three, at least 2.5
+// whole pairs: two batches at a time in turn (one where a block covers its
+// row and rows start on 4 KiB boundaries: every batch is then a whole page). Shares of three, at least 2.5
 // batches: one contiguous range per wave (the whole of K is in flight at
 // once, and turns only mix the waves' pages). Others: one batch at a time.
 // Same-box A/B, H = 16, us per step, contiguous ranges / turns of one / turns
@@ -165,12 +166,16 @@ static uint32_t score_tokens(uint32_t split, uint32_t batch) {
 // 43.9 / 44.5, x 3000 32.8 / 35.1 / 32.9 / 33.5, x 1500 18.3 / 19.7 / 18.3 / -,
 // x 1400 (5.5 batches) 17.3 / 16.9 / 17.7 / -; B = 32 x 1100 (9 batches) 25.0
 // / 24.3 / 26.1 / -; D = 64, B = 16 x 1500 (three batches) 10.8 / 11.3 / - /
-// -, x 1600 (3.25) 13.2 / 11.5 / - / -, x 300..700 7.4 / 6.8 / - / -.
-static Turns plan_turns(const AttentionPlan& p, uint32_t batch) {
+// -, x 1600 (3.25) 13.2 / 11.5 / - / -, x 300..700 7.4 / 6.8 / - / -. Rows on 4
+// KiB boundaries: B = 32 x 4000 D = 64 in 4096 slots 47.2 / 44.7 / 46.6 / -, x
+// 3500 41.0 / 39.5 / 41.1 / -, x 2000 D = 128 in 2048 46.5 / 44.7 / 46.0 / -;
+// in two blocks a row, B = 8 x 8000 D = 64 in 8192 29.6 / 29.6 / 26.4 / -.
+static Turns plan_turns(const AttentionPlan& p, uint32_t batch, uint64_t row_bytes) {
   Turns t;
   const uint32_t q = (p.split + batch - 1) / batch;
   const uint32_t pairs = (p.split + 2 * batch - 1) / (2 * batch) * 2 * batch;
-  t.shift = q >= 6 && 16 * (pairs - p.split) <= p.split ? 1 : q == 3 && 2 * p.split >= 5 * batch ? 31 : 0;
+  const bool pages = p.ngroups == 1 && row_bytes % 4096 == 0;
+  t.shift = q >= 6 && 16 * (pairs - p.split) <= p.split && !pages ? 1 : q == 3 && 2 * p.split >= 5 * batch ? 31 : 0;
   t.chunk = t.shift == 31 ? 3 : 1u << t.shift;
   t.tokens = score_tokens(p.split, batch);
   t.div = fast_divisor(p.ngroups * p.waves);
@@ -491,8 +496,8 @@ AttentionPlan plan_attention(const ppk_context* ctx, const PpkAttentionArgs& a) 
     }
   }
   if (!plan.flat) {
-    plan.turn = plan_turns(plan, 4 * tpl);
-    plan.speculate = per_row_speculates(plan, a.rows, a.heads, host, cover, limit);
+    plan.turn = plan_turns(plan, 4 * tpl, uint64_t(a.capacity) * a.head_dim);
+    plan.speculate = per_row_speculates(plan, a.rows, a.heads, host, cover, limit, 4 * tpl);
     plan.span = uint32_t(span);
   }
   return plan;
@@ -503,8 +508,8 @@ uint64_t row_cover(const uint32_t* host, uint32_t batch, uint64_t limit) {
 }
 
 bool per_row_speculates(const AttentionPlan& p, uint32_t rows, uint32_t heads, const uint32_t* host, uint64_t span,
-                        uint64_t limit) {
-  const uint64_t per_row = uint64_t(p.ngroups) * p.waves, batch = 4096 / p.head_dim;
+                        uint64_t limit, uint32_t batch) {
+  const uint64_t per_row = uint64_t(p.ngroups) * p.waves;
   uint64_t live = 0;
   for (uint32_t b = 0; b < rows / heads; ++b) {
     const uint64_t len = host ? (host[b] <= limit ? host[b] : 0) : span;
@@ -1034,6 +1039,21 @@ AttentionPlan plan_float_attention(const ppk_context* ctx, const PpkFloatAttenti
              per_row_waves_uneven(batch, host, span, plan.split)) {
     plan = plan_flat(ctx, a.rows, a.heads, host, span, a.head_dim);
   }
+  if (!plan.flat) {
+    // Shares of 16 batches or more: the row's waves take its batches in turn,
+    // as on the int8 path. Shorter shares: one contiguous range per wave, each
+    // wave starting at a batch of its own (turns would have the waves of rows
+    // a power of two apart meet in the same memory banks). Same-box A/B, bf16,
+    // H = 16, us per step, contiguous / turns: B = 32 x 8192 D = 128 310.0 /
+    // 302.5, x 1024 in 1024 slots 42.3 / 41.3, B = 16 x 4096 in 4096 81.8 /
+    // 79.0, B = 32 x 4000 D = 64 79.0 / 76.4; shares of eight batches, B = 8 x
+    // 4000 D = 64 23.4 / 23.9, B = 16 x 2000 21.1 / 21.5, of four, x 1000 11.9
+    // / 12.4.
+    const uint32_t batch = 4 * std::max<uint32_t>(tpl, 1u);
+    plan.turn = plan_turns(plan, batch, 4096);
+    plan.turn.shift = plan.split > 15 * batch ? 0 : 31;
+    plan.turn.chunk = 1;
+  }
   plan.span = uint32_t(span);
   return plan;
 }
@@ -1085,6 +1105,7 @@ void run_float_attention(ppk_context* ctx, hipStream_t stream, const PpkFloatAtt
   d.size = a.size;
   d.split_tokens = plan.split;
   d.ngroups = plan.ngroups;
+  d.turn = plan.turn;
   d.q_dtype = a.q_dtype;
   d.out_dtype = a.out_dtype;
   d.scale_log2 = scale * 1.4426950408889634f;

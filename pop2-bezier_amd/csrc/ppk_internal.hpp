@@ -178,7 +178,7 @@ struct AttentionPlan {
   // row's length arrives (off when 1/16 or more of the waves are known to
   // have no history).
   bool speculate = true;
-  Turns turn{};          // per-row int8 plan: how a row's waves take its batches
+  Turns turn{};          // per-row plan: how a row's waves take its batches
   uint32_t blocks = 0;   // flat: blocks launched
   uint32_t span = 0;     // flat: rows with past beyond it give NaN
   FlatTable table{};
@@ -226,7 +226,7 @@ uint64_t flat_cu_peak(const AttentionPlan& p, uint32_t heads, uint32_t cus);
 // fewer than 1/16 of its waves lie wholly past their row's live history (the
 // host lengths, or every row at `span` without them).
 bool per_row_speculates(const AttentionPlan& p, uint32_t rows, uint32_t heads, const uint32_t* host, uint64_t span,
-                        uint64_t limit);
+                        uint64_t limit, uint32_t batch);
 bool balanced_pays(const ppk_context* ctx, const AttentionPlan& per_row, const AttentionPlan& flat, uint32_t rows,
                    uint32_t heads, const uint32_t* host, uint64_t limit, uint64_t token_bytes);
 // Whether the per-row plan's waves of `split` tokens are uneven: the most

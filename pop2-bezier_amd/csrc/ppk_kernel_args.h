@@ -84,7 +84,7 @@ constexpr uint32_t kWaveClockDecode = 1;  // 0 entry, 1 first loads issued, 2 pa
                                           // 4 stream done, 5 block joined, 6 output / record stored
 constexpr uint32_t kWaveClockMerge = 2;   // 0 entry, 1 records combined, 2 output stored
 
-// How the ngroups * W waves of a row of the per-row int8 plan take its batches
+// How the ngroups * W waves of a row of a per-row plan take its batches
 // (four load tiles each): chunks of chunk = 2^shift batches in turn, or, with
 // shift 31, one contiguous range of `chunk` batches per wave.
 struct Turns {
@@ -214,6 +214,7 @@ struct FloatDecodeArgs {
   uint32_t span;            // most tokens a row may attend (<= size)
   uint32_t new_dtype;
   FastDiv row_div, head_div;  // by rows, by heads
+  Turns turn;               // per-row plan: shift 0, turns of one batch; else contiguous ranges of split_tokens
 };
 
 struct FloatMergeArgs {

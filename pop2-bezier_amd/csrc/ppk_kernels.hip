@@ -996,20 +996,20 @@ struct Batches {
   }
 };
 template <int TPB>
-__device__ __forceinline__ Batches row_batches(const ppk::DecodeArgs& a, uint32_t n, uint32_t place, uint32_t turns) {
+__device__ __forceinline__ Batches row_batches(const ppk::Turns& t, uint32_t n, uint32_t place, uint32_t turns) {
   const uint32_t end = n / TPB + (n % TPB != 0 ? 1u : 0u);
-  if (a.turn.shift == 31) {
-    const uint32_t first = place * a.turn.chunk;
-    return Batches{first, 0, 31, end > first ? min(end - first, a.turn.chunk) : 0u, end};
+  if (t.shift == 31) {
+    const uint32_t first = place * t.chunk;
+    return Batches{first, 0, 31, end > first ? min(end - first, t.chunk) : 0u, end};
   }
-  const uint32_t chunks = (end + a.turn.chunk - 1) >> a.turn.shift;
+  const uint32_t chunks = (end + t.chunk - 1) >> t.shift;
   uint32_t count = 0;
   if (chunks > place) {
-    const uint32_t last = fast_div(chunks - place - 1, a.turn.div);  // this wave's last chunk
-    count = (last + 1) << a.turn.shift;
-    if (place + last * turns == chunks - 1) count -= (chunks << a.turn.shift) - end;  // the row's last, cut short
+    const uint32_t last = fast_div(chunks - place - 1, t.div);  // this wave's last chunk
+    count = (last + 1) << t.shift;
+    if (place + last * turns == chunks - 1) count -= (chunks << t.shift) - end;  // the row's last, cut short
   }
-  return Batches{place << a.turn.shift, turns << a.turn.shift, a.turn.shift, count, end};
+  return Batches{place << t.shift, turns << t.shift, t.shift, count, end};
 }
 
 // A stream of at most NBATCH batches per phase, K and V already requested:
@@ -1255,7 +1255,7 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   const uint32_t place = group * W + wave, turns = a.ngroups * W;
   const uint64_t cover = uint64_t(turns) * S;
   const uint32_t nspec = a.speculate ? uint32_t(min(uint64_t(a.capacity), cover)) : 0u;
-  const Batches early = row_batches<TPB>(a, nspec, place, turns);
+  const Batches early = row_batches<TPB>(a.turn, nspec, place, turns);
   const size_t tok0 = size_t(row) * a.capacity;
   const uint8_t* kb = a.k + tok0 * D + size_t(c) * 16;
   const uint8_t* vb = a.v + tok0 * D + size_t(c) * 16;
@@ -1281,15 +1281,19 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   };
   // Everything that waits for the small loads; runs with the stream's first
   // batches in flight.
-  auto prologue = [&]() {
+  uint32_t p = 0;
+  auto length_here = [&]() {
     issue_here();
     PPK_CLK(1);
-    const uint32_t p = __builtin_amdgcn_readfirstlane(p_raw);
+    p = __builtin_amdgcn_readfirstlane(p_raw);
     PPK_CLK_AFTER(2, p_raw);
-    settle_all();
     valid = p <= a.capacity && uint64_t(p) <= cover;
     n = valid ? p : 0u;
-    bt = row_batches<TPB>(a, n, place, turns);
+    bt = row_batches<TPB>(a.turn, n, place, turns);
+  };
+  auto operands_here = [&]() {
+    issue_here();
+    settle_all();
     float x[EPL];
     widen<EPL>(q_raw, a.q_dtype, x);
     if (bt.count > 0) make_query<D, BF16H>(x, a.scale_log2, s_lds, lane, query);
@@ -1336,6 +1340,10 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   auto load_v = [&](int b, const Batches& of, uint32_t limit) {
     load_batch<D, U>(vb, vsb, of.tile(uint32_t(b)), limit, j, lane, va[b], vsa[b]);
   };
+  auto prologue = [&]() {
+    length_here();
+    operands_here();
+  };
   // The paths differ in what is in flight when the prologue runs; each runs
   // its own copy of it, so that its waits count that path's loads only.
   if (early.count == 1) {
@@ -1357,10 +1365,14 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
       for (int b = 0; b < NB; ++b) load_k(b, early, nspec);
       prologue();
     } else {
-      prologue();
+      // The length decides the first batches; the operands that came with it wait until those are on their way.
+      length_here();
       if (bt.count > 0) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) load_k(b, bt, n);
+        operands_here();
+      } else {
+        operands_here();
       }
     }
     if (bt.count > 2) {
@@ -1872,8 +1884,12 @@ __device__ __forceinline__ float token_sum(float x) {
     return group_sum<LPT>(x);
   } else {
     x = group_sum<16>(x);
-    x += __shfl_xor(x, 16);
-    if constexpr (LPT >= 64) x += __shfl_xor(x, 32);
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    if constexpr (LPT >= 64) {
+      r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+      x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
     return x;
   }
 }
@@ -1915,7 +1931,7 @@ __device__ __forceinline__ void load_fbatch(const char* base, uint32_t t0, uint3
 template <int D, bool BF16KV, int U>
 __device__ __forceinline__ float fscore_batch(const u4 (&raw)[U], uint32_t t0, uint32_t n, int j, int c,
                                               const float (&qr)[FloatGeom<D, BF16KV>::kEpc], float sl2,
-                                              float* s_lds, float mloc) {
+                                              float* s_batch, float mloc) {
   using G = FloatGeom<D, BF16KV>;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -1928,20 +1944,20 @@ __device__ __forceinline__ float fscore_batch(const u4 (&raw)[U], uint32_t t0, u
     float sc = token_sum<G::kLpt>(d) * sl2;
     sc = tok < n ? sc : -INFINITY;
     mloc = fmaxf(mloc, sc);
-    if (c == 0 && tok < n) s_lds[tok] = sc;
+    if (c == 0) s_batch[u * G::kTpl + j] = sc;
   }
   return mloc;
 }
 
 template <int D, bool BF16KV, int U>
 __device__ __forceinline__ void faccumulate_batch(const u4 (&raw)[U], uint32_t t0, uint32_t n, int j, int lane,
-                                                  float m, const float* s_lds, float& z,
+                                                  float m, const float* s_batch, float& z,
                                                   float (&acc)[FloatGeom<D, BF16KV>::kEpc]) {
   using G = FloatGeom<D, BF16KV>;
   constexpr int TPB = U * G::kTpl;  // tokens per batch (<= 64)
   static_assert(TPB <= ppk::kWave, "one token per lane per batch");
   const uint32_t tl = t0 * G::kTpl + uint32_t(lane % TPB);
-  const float e = __builtin_amdgcn_exp2f(s_lds[min(tl, n - 1)] - m);
+  const float e = __builtin_amdgcn_exp2f(s_batch[lane % TPB] - m);
   const float pr = (tl < n && lane < TPB) ? e : 0.f;
   z += pr;
 #pragma unroll
@@ -1962,30 +1978,39 @@ struct FloatWavePartial {
   float acc[FloatGeom<D, BF16KV>::kEpc];
 };
 
-// One wave streams n tokens of a row from `begin`: phase K scores into LDS,
-// phase V accumulation; A/B batches ping-pong, and the last phase-K
-// iteration already fetches the first V batch.
-template <int D, bool BF16KV>
+// One wave streams its share of a row: phase K scores into LDS, phase V
+// accumulation; A/B batches ping-pong, and the last phase-K iteration already
+// fetches the first V batch. The share is the n tokens from `begin`, or, when
+// the row's waves take its batches in turn (a.turn.shift == 0), the batches
+// bt of the row's n tokens. early() leaves the query chunk in qr, with the
+// first batch in flight.
+template <int D, bool BF16KV, class Early>
 __device__ __forceinline__ void fwave_attention(const ppk::FloatDecodeArgs& a, uint32_t row, uint32_t begin,
-                                                uint32_t n, const float (&qr)[FloatGeom<D, BF16KV>::kEpc],
-                                                float* s_lds, int lane, FloatWavePartial<D, BF16KV>& out) {
+                                                uint32_t n, const Batches& bt,
+                                                const float (&qr)[FloatGeom<D, BF16KV>::kEpc], float* s_lds, int lane,
+                                                FloatWavePartial<D, BF16KV>& out, Early early) {
   using G = FloatGeom<D, BF16KV>;
   constexpr int U = 4;
+  constexpr int TPB = U * G::kTpl;
   const int j = lane / G::kLpt;
   const int c = lane % G::kLpt;
   out.m = -INFINITY;
   out.z = 0.f;
 #pragma unroll
   for (int i = 0; i < G::kEpc; ++i) out.acc[i] = 0.f;
-  if (n == 0) return;  // uniform per wave
+  const bool turns = a.turn.shift == 0;
+  const uint32_t nb = turns ? bt.count : (n + TPB - 1) / TPB;
+  if (nb == 0) {  // uniform per wave
+    early();
+    return;
+  }
 
   const char* kb = static_cast<const char*>(a.k) +
                    (size_t(row) * a.k_stride + size_t(begin) * D) * G::kElemBytes + size_t(c) * ppk::kLaneBytes;
   const char* vb = static_cast<const char*>(a.v) +
                    (size_t(row) * a.v_stride + size_t(begin) * D) * G::kElemBytes + size_t(c) * ppk::kLaneBytes;
-  const uint32_t ntiles = (n + G::kTpl - 1) / G::kTpl;
   const float sl2 = a.scale_log2;
-  // Each wave takes its batches in a rotated order: it starts at batch rot of
+  // A contiguous range is taken in a rotated order: the wave starts at batch rot of
   // its nb batches and wraps, and phase V follows the same order. Waves that
   // start at the same offset of rows a power of two apart (a store of 4096 or
   // 8192 tokens) otherwise move through the same HBM channels in step. rot is
@@ -2000,34 +2025,42 @@ __device__ __forceinline__ void fwave_attention(const ppk::FloatDecodeArgs& a, u
   // 8192 D=128 310.5 -> 309.0 us. It costs where a few long rows stream one
   // wave per CU: 4 x 8192 + 28 x 512 tokens on the per-row plan 112.2 ->
   // 115.7 us (the balanced plan, which host lengths select, does not rotate).
-  const uint32_t nb = (ntiles + U - 1) / U;
   const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
-  const uint32_t rot = ((wave_id * 0x9E37u & 0xFFFFu) * nb) >> 16;
-  auto ph = [&](uint32_t t) {  // logical first tile of a batch -> the tile it reads
-    const uint32_t b = t / U;
-    return b < nb ? (b + rot >= nb ? b + rot - nb : b + rot) * U : t;
-  };
+  const uint32_t rot = turns ? 0u : ((wave_id * 0x9E37u & 0xFFFFu) * nb) >> 16;
+  // Logical batch b: its place among the wave's batches (its scores' place in
+  // LDS) and its first tile. Past the end: a tile past the row's or range's.
+  auto place = [&](uint32_t b) { return b < nb ? (b + rot >= nb ? b + rot - nb : b + rot) : nb; };
+  auto tile = [&](uint32_t b) { return turns ? bt.tile(b) : (b < nb ? place(b) : b) * U; };
 
   u4 ra[U], rb[U];
   float mloc = -INFINITY;
-  load_fbatch<D, BF16KV, U>(kb, ph(0), n, j, ra);
-  for (uint32_t t0 = 0; t0 < ntiles; t0 += 2 * U) {
-    load_fbatch<D, BF16KV, U>(kb, ph(t0 + U), n, j, rb);
-    mloc = fscore_batch<D, BF16KV, U>(ra, ph(t0), n, j, c, qr, sl2, s_lds, mloc);
-    const bool last = t0 + 2 * U >= ntiles;
-    load_fbatch<D, BF16KV, U>(last ? vb : kb, last ? ph(0) : ph(t0 + 2 * U), n, j, ra);
-    mloc = fscore_batch<D, BF16KV, U>(rb, ph(t0 + U), n, j, c, qr, sl2, s_lds, mloc);
+  auto score = [&](const u4 (&r)[U], uint32_t b) {
+    if (b < nb) mloc = fscore_batch<D, BF16KV, U>(r, tile(b), n, j, c, qr, sl2, s_lds + place(b) * TPB, mloc);
+  };
+  load_fbatch<D, BF16KV, U>(kb, tile(0), n, j, ra);
+  issue_here();
+  early();
+  for (uint32_t b = 0; b < nb; b += 2) {
+    load_fbatch<D, BF16KV, U>(kb, tile(b + 1), n, j, rb);
+    score(ra, b);
+    const bool last = b + 2 >= nb;
+    load_fbatch<D, BF16KV, U>(last ? vb : kb, tile(last ? 0 : b + 2), n, j, ra);
+    score(rb, b + 1);
   }
   float m = mloc;
   m = groups_max<G::kLpt>(m);
   __builtin_amdgcn_wave_barrier();
 
   float z = 0.f;
-  for (uint32_t t0 = 0; t0 < ntiles; t0 += 2 * U) {
-    load_fbatch<D, BF16KV, U>(vb, ph(t0 + U), n, j, rb);
-    faccumulate_batch<D, BF16KV, U>(ra, ph(t0), n, j, lane, m, s_lds, z, out.acc);
-    load_fbatch<D, BF16KV, U>(vb, ph(t0 + 2 * U), n, j, ra);
-    faccumulate_batch<D, BF16KV, U>(rb, ph(t0 + U), n, j, lane, m, s_lds, z, out.acc);
+  auto accumulate = [&](const u4 (&r)[U], uint32_t b) {
+    if (b < nb)
+      faccumulate_batch<D, BF16KV, U>(r, tile(b), n, j, lane, m, s_lds + place(b) * TPB, z, out.acc);
+  };
+  for (uint32_t b = 0; b < nb; b += 2) {
+    load_fbatch<D, BF16KV, U>(vb, tile(b + 1), n, j, rb);
+    accumulate(ra, b);
+    load_fbatch<D, BF16KV, U>(vb, tile(b + 2), n, j, ra);
+    accumulate(rb, b + 1);
   }
   z = wave_sum(z);
   reduce_scatter_groups<G::kLpt, G::kEpc>(out.acc, lane);
@@ -2035,35 +2068,27 @@ __device__ __forceinline__ void fwave_attention(const ppk::FloatDecodeArgs& a, u
   out.z = z;
 }
 
-__device__ __forceinline__ uint32_t float_row_length(const uint32_t* lengths, uint32_t row, uint32_t heads,
-                                                     uint32_t size) {
-  return lengths ? lengths[row / heads] : size;
-}
-
-// The fused step's current token of row `row`, channels lane * EPL .. + EPL,
-// rounded to the store's dtype (the value a stored token would hold).
-template <int EPL, bool BF16KV>
-__device__ __forceinline__ void load_current(const void* src, uint32_t row, uint32_t dtype, int lane,
-                                             float (&x)[EPL]) {
-  load_vec<EPL>(src, size_t(row) * (EPL * ppk::kWave) + size_t(lane) * EPL, dtype, x);
+// The fused step's current token, widened from its raw words and rounded to
+// the store's dtype (the value a stored token would hold).
+template <int N, bool BF16KV>
+__device__ __forceinline__ void widen_current(const RawVec<N>& raw, uint32_t dtype, float (&x)[N]) {
+  widen<N>(raw, dtype, x);
   if constexpr (BF16KV) {
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) x[e] = bf16_to_f32(f32_to_bf16_bits(x[e]));
+    for (int e = 0; e < N; ++e) x[e] = bf16_to_f32(f32_to_bf16_bits(x[e]));
   }
 }
 
 // The fused step's write of one current-token tensor of `row` at slot p of
-// the store (or the overflow flag when the slot is past the store).
+// the store; returns PPK_FLAG_OVERFLOW when the slot is past the store.
 template <int EPL, bool BF16KV>
-__device__ __forceinline__ void write_current(void* store, uint64_t stride, uint32_t row, uint32_t p, uint32_t size,
-                                              const float (&x)[EPL], uint32_t* flags, int lane) {
-  if (p >= size) {
-    raise_flags(flags, 2u);
-    return;
-  }
+__device__ __forceinline__ uint32_t write_current(void* store, uint64_t stride, uint32_t row, uint32_t p,
+                                                  uint32_t size, const float (&x)[EPL], int lane) {
+  if (p >= size) return 2u;
   const size_t base = size_t(row) * stride + size_t(p) * (EPL * ppk::kWave) + size_t(lane) * EPL;
 #pragma unroll
   for (int e = 0; e < EPL; ++e) store_elem(store, base + e, BF16KV ? kBF16 : kF32, x[e]);
+  return 0;
 }
 
 template <int D, bool BF16KV, bool STEP>
@@ -2074,62 +2099,89 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
   const int lane = threadIdx.x & 63;
   // Uniform: the wave's range, length and loop bounds stay in scalar registers.
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int W = blockDim.x >> 6;
   const int c = lane % G::kLpt;
   // Blocks are numbered group-major: consecutive blocks belong to different
   // rows, so the empty tail groups of short rows (ragged batches) spread over
   // the CUs instead of leaving some CUs with only live blocks.
-  const uint32_t row = blockIdx.x % a.rows;
-  const uint32_t group = blockIdx.x / a.rows;
-  const uint32_t S = a.split_tokens;
+  const uint32_t group = fast_div(blockIdx.x, a.row_div);
+  const uint32_t row = blockIdx.x - group * a.rows;
   // The stored tokens a row streams: lengths[b] (the step's current token
-  // comes from k_new / v_new instead).
-  const uint32_t len = float_row_length(a.lengths, row, a.heads, a.size);
+  // comes from k_new / v_new instead). The wave's first loads wait for it: the
+  // other arguments they need are requested beside it (the compiler would
+  // load each where it is first used, one scalar round trip after another).
+  const uint32_t seq = fast_div(row, a.head_div);
+  const uint32_t len = a.lengths ? a.lengths[seq] : a.size;
+  __asm__ volatile("" ::"s"(seq), "s"(a.q), "s"(a.k), "s"(a.v), "s"(a.k_new), "s"(a.v_new), "s"(a.q_stride), "s"(a.k_stride),
+                   "s"(a.v_stride), "s"(a.size), "s"(a.split_tokens), "s"(a.ngroups), "s"(a.q_dtype),
+                   "s"(a.new_dtype), "s"(a.scale_log2), "s"(a.span), "s"(a.turn.div.mul), "s"(a.turn.div.shift),
+                   "s"(a.turn.shift), "s"(a.turn.chunk), "s"(a.turn.tokens), "s"(blockDim.x));
+  const int W = blockDim.x >> 6;
+  const uint32_t S = a.split_tokens;
   bool valid;
   if constexpr (STEP)
     valid = len < a.size && len + 1 <= a.span && uint64_t(len) <= uint64_t(a.ngroups) * W * S;
   else
     valid = len > 0 && len <= a.span && len <= a.size && uint64_t(len) <= uint64_t(a.ngroups) * W * S;
 
-  float qr[G::kEpc];
-  load_vec<G::kEpc>(a.q, size_t(row) * a.q_stride + size_t(c) * G::kEpc, a.q_dtype, qr);
   // The step: group 0's waves 0 and 1 write the current key and value at slot
   // len (never read here: every stream stops before it); wave 0 of a block
-  // that finishes its row also folds the current token into the result.
+  // that finishes its row also folds the current token into the result. The
+  // operands travel as raw words beside the stream's first batch.
   const bool final_out = a.ngroups == 1;
   const bool kw = STEP && group == 0 && wave == 0;
   const bool vw = STEP && group == 0 && wave == (W > 1 ? 1 : 0);
   const bool cur = STEP && final_out && wave == 0;
-  float kcur[EPL], vcur[EPL], qcur[EPL];
-  if (kw || cur) load_current<EPL, BF16KV>(a.k_new, row, a.new_dtype, lane, kcur);
-  if (vw || cur) load_current<EPL, BF16KV>(a.v_new, row, a.new_dtype, lane, vcur);
-  if (cur) load_vec<EPL>(a.q, size_t(row) * a.q_stride + size_t(lane) * EPL, a.q_dtype, qcur);
-  // A stored length within the span that the plan does not cover: the plan
-  // was sized from a stale host copy of the lengths (the row gives NaN).
-  if (kw && len < a.size && len + 1 <= a.span && uint64_t(len) > uint64_t(a.ngroups) * W * S) raise_flags(a.flags, 4u);
-  if (kw) write_current<EPL, BF16KV>(const_cast<void*>(a.k), a.k_stride, row, len, a.size, kcur, a.flags, lane);
-  if (vw) write_current<EPL, BF16KV>(const_cast<void*>(a.v), a.v_stride, row, len, a.size, vcur, a.flags, lane);
-  const uint32_t begin = (group * W + wave) * S;
-  const uint32_t n = (valid && begin < len) ? min(S, len - begin) : 0u;
+  RawVec<G::kEpc> q_raw;
+  RawVec<EPL> qc_raw, kn_raw, vn_raw;
+  load_raw<G::kEpc>(a.q, size_t(row) * a.q_stride + size_t(c) * G::kEpc, a.q_dtype, q_raw);
+  const size_t own = size_t(row) * D + size_t(lane) * EPL;
+  if (kw || cur) load_raw<EPL>(a.k_new, own, a.new_dtype, kn_raw);
+  if (vw || cur) load_raw<EPL>(a.v_new, own, a.new_dtype, vn_raw);
+  if (cur) load_raw<EPL>(a.q, size_t(row) * a.q_stride + size_t(lane) * EPL, a.q_dtype, qc_raw);
+  // This wave's share: a contiguous range of S tokens, or (a.turn) its turns of the row.
+  const bool turns = a.turn.shift == 0;
+  const uint32_t place = group * W + wave;
+  const uint32_t begin = turns ? 0u : place * S;
+  const uint32_t n = !valid || begin >= len ? 0u : turns ? len : min(S, len - begin);
+  const Batches bt = row_batches<4 * G::kTpl>(a.turn, turns ? n : 0u, place, a.ngroups * W);
+
+  float qr[G::kEpc], kcur[EPL], vcur[EPL];
+  float s_cur = -INFINITY;
+  uint32_t raise = 0;
+  auto early = [&]() {
+    settle(q_raw);
+    settle(kn_raw);
+    settle(vn_raw);
+    settle(qc_raw);
+    widen<G::kEpc>(q_raw, a.q_dtype, qr);
+    if (kw || cur) widen_current<EPL, BF16KV>(kn_raw, a.new_dtype, kcur);
+    if (vw || cur) widen_current<EPL, BF16KV>(vn_raw, a.new_dtype, vcur);
+    if (cur) {
+      float qcur[EPL], d = 0.f;
+      widen<EPL>(qc_raw, a.q_dtype, qcur);
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) d = fmaf(qcur[e], kcur[e], d);
+      s_cur = wave_sum(d) * a.scale_log2;
+    }
+    // A stored length within the span that the plan does not cover: the plan
+    // was sized from a stale host copy of the lengths (the row gives NaN).
+    if (kw && len < a.size && len + 1 <= a.span && uint64_t(len) > uint64_t(a.ngroups) * W * S) raise |= 4u;
+    if (kw) raise |= write_current<EPL, BF16KV>(const_cast<void*>(a.k), a.k_stride, row, len, a.size, kcur, lane);
+    if (vw) raise |= write_current<EPL, BF16KV>(const_cast<void*>(a.v), a.v_stride, row, len, a.size, vcur, lane);
+  };
   FloatWavePartial<D, BF16KV> part;
-  // LDS of this wave alone: a score per token of its range, then its record.
-  const uint32_t lds_stride = max(S, uint32_t(D + 4));
+  // LDS of this wave alone: a score per token of its share, then its record.
+  const uint32_t lds_stride = max(a.turn.tokens, uint32_t(D + 4));
   float* s_lds = lds + size_t(wave) * lds_stride;
-  fwave_attention<D, BF16KV>(a, row, begin, n, qr, s_lds, lane, part);
+  fwave_attention<D, BF16KV>(a, row, begin, n, bt, qr, s_lds, lane, part, early);
 
   // Combine the block's waves through LDS: each wave's record replaces its
   // scores (its own LDS, so no barrier is needed before).
   write_block_record<D>(s_lds, c * G::kEpc + scatter_base<G::kLpt, G::kEpc>(lane), lane, part.m, part.z, part.acc);
+  raise_flags(a.flags, raise);
   __syncthreads();
   if (wave != 0) return;
 
-  float s_cur = -INFINITY;
-  if (cur) {
-    float d = 0.f;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) d = fmaf(qcur[e], kcur[e], d);
-    s_cur = wave_sum(d) * a.scale_log2;
-  }
   float m, y[EPL], zsum;
   combine_block<D, 16>(lds, lds_stride, uint32_t(W), lane, s_cur, m, zsum, y);
   if (cur) {
@@ -2365,8 +2417,9 @@ __device__ __forceinline__ void fdecode_flat_body(const ppk::FloatDecodeFlatArgs
     if (!put) return;
     float x[EPL];
     widen<EPL>(new_raw, a.new_dtype, x);
-    write_current<EPL, BF16KV>(const_cast<void*>(value ? a.v : a.k), value ? a.v_stride : a.k_stride, arow,
-                               __builtin_amdgcn_readfirstlane(slot_raw), a.size, x, a.flags, lane);
+    raise_flags(a.flags, write_current<EPL, BF16KV>(const_cast<void*>(value ? a.v : a.k),
+                                                    value ? a.v_stride : a.k_stride, arow,
+                                                    __builtin_amdgcn_readfirstlane(slot_raw), a.size, x, lane));
   };
   if (wid >= t.units_total) {
     write();
