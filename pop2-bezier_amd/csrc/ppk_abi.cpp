@@ -156,8 +156,7 @@ static uint32_t score_tokens(uint32_t split, uint32_t batch) {
 
 // How a row's waves take its batches, by the batches of one wave's share
 // (q = ceil(split / batch)). Shares of six batches or more within 1/16 of
-// whole pairs: two batches at a time in turn (one where a block covers its
-// row and rows start on 4 KiB boundaries: every batch is then a whole page). Shares of three, at least 2.5
+// whole pairs, and below 32: two batches at a time in turn. Shares of three, at least 2.5
 // batches: one contiguous range per wave (the whole of K is in flight at
 // once, and turns only mix the waves' pages). Others: one batch at a time.
 // Same-box A/B, H = 16, us per step, contiguous ranges / turns of one / turns
@@ -166,16 +165,15 @@ static uint32_t score_tokens(uint32_t split, uint32_t batch) {
 // 43.9 / 44.5, x 3000 32.8 / 35.1 / 32.9 / 33.5, x 1500 18.3 / 19.7 / 18.3 / -,
 // x 1400 (5.5 batches) 17.3 / 16.9 / 17.7 / -; B = 32 x 1100 (9 batches) 25.0
 // / 24.3 / 26.1 / -; D = 64, B = 16 x 1500 (three batches) 10.8 / 11.3 / - /
-// -, x 1600 (3.25) 13.2 / 11.5 / - / -, x 300..700 7.4 / 6.8 / - / -. Rows on 4
-// KiB boundaries: B = 32 x 4000 D = 64 in 4096 slots 47.2 / 44.7 / 46.6 / -, x
-// 3500 41.0 / 39.5 / 41.1 / -, x 2000 D = 128 in 2048 46.5 / 44.7 / 46.0 / -;
-// in two blocks a row, B = 8 x 8000 D = 64 in 8192 29.6 / 29.6 / 26.4 / -.
-static Turns plan_turns(const AttentionPlan& p, uint32_t batch, uint64_t row_bytes) {
+// -, x 1600 (3.25) 13.2 / 11.5 / - / -, x 300..700 7.4 / 6.8 / - / -. (The
+// arena's capacity has no say: a row's result does not depend on it. Where rows
+// start on 4 KiB boundaries turns of one would be up to 4 % faster: B = 32 x
+// 4000 D = 64 in 4096 slots 47.2 / 44.7 / 46.6 / -.)
+static Turns plan_turns(const AttentionPlan& p, uint32_t batch) {
   Turns t;
   const uint32_t q = (p.split + batch - 1) / batch;
   const uint32_t pairs = (p.split + 2 * batch - 1) / (2 * batch) * 2 * batch;
-  const bool pages = p.ngroups == 1 && row_bytes % 4096 == 0;
-  t.shift = q >= 6 && 16 * (pairs - p.split) <= p.split && !pages ? 1 : q == 3 && 2 * p.split >= 5 * batch ? 31 : 0;
+  t.shift = q >= 6 && q < 32 && 16 * (pairs - p.split) <= p.split ? 1 : q == 3 && 2 * p.split >= 5 * batch ? 31 : 0;
   t.chunk = t.shift == 31 ? 3 : 1u << t.shift;
   t.tokens = score_tokens(p.split, batch);
   t.div = fast_divisor(p.ngroups * p.waves);
@@ -496,7 +494,7 @@ AttentionPlan plan_attention(const ppk_context* ctx, const PpkAttentionArgs& a) 
     }
   }
   if (!plan.flat) {
-    plan.turn = plan_turns(plan, 4 * tpl, uint64_t(a.capacity) * a.head_dim);
+    plan.turn = plan_turns(plan, 4 * tpl);
     plan.speculate = per_row_speculates(plan, a.rows, a.heads, host, cover, limit, 4 * tpl);
     plan.span = uint32_t(span);
   }
@@ -1050,7 +1048,7 @@ AttentionPlan plan_float_attention(const ppk_context* ctx, const PpkFloatAttenti
     // 4000 D = 64 23.4 / 23.9, B = 16 x 2000 21.1 / 21.5, of four, x 1000 11.9
     // / 12.4.
     const uint32_t batch = 4 * std::max<uint32_t>(tpl, 1u);
-    plan.turn = plan_turns(plan, batch, 4096);
+    plan.turn = plan_turns(plan, batch);
     plan.turn.shift = plan.split > 15 * batch ? 0 : 31;
     plan.turn.chunk = 1;
   }
