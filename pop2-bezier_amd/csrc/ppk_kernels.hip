@@ -2556,13 +2556,20 @@ __device__ __forceinline__ void fmerge_flat_body(const ppk::FloatMergeFlatArgs& 
 //
 // The arithmetic that decides support keeps the reference's order: 256
 // strided partial sums of exp(v - m) and exp(alpha (v - m)) in candidate
-// order, then the halving tree (steps 128, 64 through LDS, 32..1 by
-// shuffles within one wave: the same pairs added in the same order), with
+// order, then the halving tree (steps 128, 64 through LDS, 32..1 by lane
+// swaps within each wave: the same pairs added in the same order), with
 // the device expf/logf. The candidate selection is this file's own: the
 // reference sorts the whole legal range (a bitonic network of ~66 barrier
-// phases at 2048 candidates); here a 4-pass radix select over a 32-bit
-// order-preserving key of the value finds the selected value and a ballot
-// count orders equal values by index, which names the same candidate.
+// phases at 2048 candidates); here the values are counted into 512 equal bins
+// beside the sums, and the few candidates of the bin that holds the rank are
+// ordered by comparison. Where that bin is crowded, a 4-pass radix select over
+// a 32-bit order-preserving key of the value finds the selected value and a
+// ballot count orders equal values by index. All name the same candidate.
+// The kernel is a chain of barriers and round trips (one block per row, one
+// wave per SIMD): three barriers now, where four radix passes took twenty and
+// the support two more: 32 rows x 2048 choices with guidance 10.3 -> 6.3 us,
+// 1024 rows 14.3 -> 9.1, 64 rows x 37 choices 8.1 -> 4.3 (one launch in a
+// captured sequence of 50).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ bool finite_bits(float x) { return (__float_as_uint(x) & 0x7fffffffu) < 0x7f800000u; }
 __device__ __forceinline__ bool sample_before(float a, uint32_t ai, float b, uint32_t bi) {
@@ -2583,6 +2590,31 @@ __device__ __forceinline__ void write_sample(const ppk::RenyiArgs& a, uint32_t r
   a.out[2 * size_t(a.batch) + row] = support;
 }
 
+// Inclusive prefix sum over the wave's lanes (DPP, no LDS).
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
+  int x = int(v);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return uint32_t(x);
+}
+// Lane 0 receives the sum over the wave in the halving order x[i] += x[i + o],
+// o = 32, 16, ... 1 (the other lanes: partial sums).
+__device__ __forceinline__ float halving_sum(float x) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  x += dpp_f32<0x108>(x);  // row_shl:8
+  x += dpp_f32<0x104>(x);
+  x += dpp_f32<0x102>(x);
+  x += dpp_f32<0x101>(x);
+  return x;
+}
+
 __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
   // Every float operation rounds on its own, as the reference kernel is built
   // (-ffp-contract=off, app/src/model/hip_kernel.rs:46) and as its host oracle
@@ -2592,14 +2624,20 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
 #pragma clang fp contract(off)
   constexpr int T = ppk::kSamplerThreads;
   constexpr int PER = ppk::kSamplerMaxChoices / T;  // candidates per thread
+  constexpr int BINS = 512;                         // value bins of the selection, BINS / 64 per lane
+  constexpr uint32_t LIST = 64;                     // most candidates of the selected bin the fast path orders
   __shared__ float s_vals[ppk::kSamplerMaxChoices];
   __shared__ float s_sum[T], s_sum_a[T];
-  __shared__ float s_wmax[T / 64];
+  __shared__ float s_wmax[T / 64], s_wmin[T / 64];
   __shared__ uint32_t s_wid[T / 64], s_wbad[T / 64];
+  __shared__ __attribute__((aligned(16))) uint32_t s_bins[BINS];
+  __shared__ float s_list_v[LIST];
+  __shared__ uint32_t s_list_i[LIST];
+  __shared__ uint32_t s_listed;
   __shared__ uint32_t s_hist[256];
   __shared__ uint32_t s_wtotal[T / 64];
   __shared__ uint64_t s_ballot[PER][T / 64];
-  __shared__ uint32_t s_state[4];  // support, rank, invalid, selected bin / below
+  __shared__ uint32_t s_state[4];  // selected bin / below of the radix passes
 
   const uint32_t row = blockIdx.x;
   const int t = threadIdx.x;
@@ -2620,6 +2658,9 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
   const uint32_t start = a.bounds[2 * row];
   const uint32_t count = a.bounds[2 * row + 1];
   const float uniform = a.uniforms[row];
+#pragma unroll
+  for (int i = 0; i < BINS / T; ++i) s_bins[t + i * T] = 0;
+  if (t == 0) s_listed = 0;
   // Every thread evaluates the same metadata, so these exits are uniform.
   if (!finite_bits(uniform) || uniform < 0.f || uniform >= 1.f || start >= a.choices || count == 0 ||
       count > a.choices - start) {
@@ -2628,8 +2669,8 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
   }
 
   // Whole head, in column order: CFG combine and finiteness; legal values to
-  // LDS; arg-max.
-  float lmax = -INFINITY;
+  // LDS; arg-max (the lowest index of the largest value) and minimum.
+  float lmax = -INFINITY, lmin = INFINITY;
   uint32_t lid = 0xffffffffu, lbad = 0;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
@@ -2648,29 +2689,29 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
     if (!finite) value = 0.f;
     if (col >= start && col - start < count) {
       s_vals[col - start] = value;
+      lmin = fminf(lmin, value);
       if (sample_before(value, col, lmax, lid)) {
         lmax = value;
         lid = col;
       }
     }
   }
-#pragma unroll
-  for (int o = 32; o; o >>= 1) {
-    const float ov = __shfl_xor(lmax, o);
-    const uint32_t oi = __shfl_xor(lid, o);
-    if (sample_before(ov, oi, lmax, lid)) {
-      lmax = ov;
-      lid = oi;
+  {
+    const float wmax = wave_max(lmax);
+    const float wmin = wave_reduce(lmin, [](float x, float y) { return fminf(x, y); });
+    // The least index of the wave's maximum, on the bit patterns of indexes (below 2^24: exact as floats).
+    const float id = wave_reduce(lmax == wmax && lid != 0xffffffffu ? float(lid) : 16777216.f,
+                                 [](float x, float y) { return fminf(x, y); });
+    const bool wbad = __any(lbad != 0);
+    if (lane == 0) {
+      s_wmax[wave] = wmax;
+      s_wmin[wave] = wmin;
+      s_wid[wave] = uint32_t(id);
+      s_wbad[wave] = wbad ? 1u : 0u;
     }
-    lbad |= __shfl_xor(lbad, o);
-  }
-  if (lane == 0) {
-    s_wmax[wave] = lmax;
-    s_wid[wave] = lid;
-    s_wbad[wave] = lbad;
   }
   __syncthreads();
-  float maximum = s_wmax[0];
+  float maximum = s_wmax[0], minimum = s_wmin[0];
   uint32_t maximum_id = s_wid[0], bad = s_wbad[0];
 #pragma unroll
   for (int w = 1; w < T / 64; ++w) {
@@ -2678,6 +2719,7 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
       maximum = s_wmax[w];
       maximum_id = s_wid[w];
     }
+    minimum = fminf(minimum, s_wmin[w]);
     bad |= s_wbad[w];
   }
   if (bad) {
@@ -2685,69 +2727,131 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
     return;
   }
 
-  // Strided partial sums in candidate order, then the halving tree.
+  // Strided partial sums in candidate order, then the halving tree. The bins
+  // of the selection are counted beside them: bin = (maximum - v) scaled to
+  // BINS, a rounded subtraction and a rounded product, so a larger value never
+  // has a higher bin.
+  const float range = maximum - minimum;
+  const float bin_scale = float(BINS) / range;
+  const bool binned = range > 0.f && finite_bits(range) && finite_bits(bin_scale);
   float vals[PER];
+  uint32_t bins[PER];
   float sum = 0.f, sum_a = 0.f;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const uint32_t ci = uint32_t(t) + uint32_t(k) * T;
     vals[k] = ci < count ? s_vals[ci] : 0.f;
+    bins[k] = 0xffffffffu;
     if (ci < count) {
       const float shifted = vals[k] - maximum;
       sum += expf(shifted);
       sum_a += expf(a.alpha * shifted);
+      if (binned) {
+        bins[k] = min(uint32_t((maximum - vals[k]) * bin_scale), uint32_t(BINS - 1));
+        atomicAdd(&s_bins[bins[k]], 1u);
+      }
     }
   }
   s_sum[t] = sum;
   s_sum_a[t] = sum_a;
   __syncthreads();
-  if (t < 128) {
-    s_sum[t] += s_sum[t + 128];
-    s_sum_a[t] += s_sum_a[t + 128];
-  }
-  __syncthreads();
-  if (wave == 0) {
-    float z = s_sum[lane] + s_sum[lane + 64];
-    float za = s_sum_a[lane] + s_sum_a[lane + 64];
-#pragma unroll
-    for (int o = 32; o; o >>= 1) {
-      z += __shfl_down(z, o);
-      za += __shfl_down(za, o);
-    }
-    if (lane == 0) {
-      const float log_z = logf(z);
-      const float log_za = logf(za);
-      float correction = log_z - log_za;
-      if (correction < 0.0f) correction = 0.0f;
-      float entropy = log_z + correction / (a.alpha - 1.0f);
-      uint32_t invalid = !finite_bits(log_z) || !finite_bits(log_za) || !finite_bits(entropy);
-      uint32_t support = 1, rank = 0;
-      if (!invalid) {
-        const float maximum_entropy = logf((float)count);
-        if (entropy < 0.0f) entropy = 0.0f;
-        if (entropy > maximum_entropy) entropy = maximum_entropy;
-        const float rounded = expf(entropy) + 0.5f;
-        support = (uint32_t)rounded;
-        if (support < 1) support = 1;
-        if (support > count) support = count;
-        rank = (uint32_t)(uniform * (float)support);
-        if (rank >= support) rank = support - 1;
-      }
-      s_state[0] = support;
-      s_state[1] = rank;
-      s_state[2] = invalid;
+  // Every wave adds the tree's 256 partials (128 and 64 apart from LDS, then
+  // the halving steps across lanes, the same pairs in the same order) and
+  // evaluates the support, instead of one wave for all behind two barriers.
+  uint32_t support = 1, r = 0, invalid;
+  {
+    const float z = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(
+        halving_sum((s_sum[lane] + s_sum[lane + 128]) + (s_sum[lane + 64] + s_sum[lane + 192])))));
+    const float za = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(
+        halving_sum((s_sum_a[lane] + s_sum_a[lane + 128]) + (s_sum_a[lane + 64] + s_sum_a[lane + 192])))));
+    const float log_z = logf(z);
+    const float log_za = logf(za);
+    float correction = log_z - log_za;
+    if (correction < 0.0f) correction = 0.0f;
+    float entropy = log_z + correction / (a.alpha - 1.0f);
+    invalid = !finite_bits(log_z) || !finite_bits(log_za) || !finite_bits(entropy);
+    if (!invalid) {
+      const float maximum_entropy = logf((float)count);
+      if (entropy < 0.0f) entropy = 0.0f;
+      if (entropy > maximum_entropy) entropy = maximum_entropy;
+      const float rounded = expf(entropy) + 0.5f;
+      support = (uint32_t)rounded;
+      if (support < 1) support = 1;
+      if (support > count) support = count;
+      r = (uint32_t)(uniform * (float)support);
+      if (r >= support) r = support - 1;
     }
   }
-  __syncthreads();
-  const uint32_t support = s_state[0];
-  uint32_t r = s_state[1];
-  if (s_state[2]) {
+  support = __builtin_amdgcn_readfirstlane(support);
+  r = __builtin_amdgcn_readfirstlane(r);
+  if (__any(invalid != 0)) {
     if (t == 0) write_sample(a, row, a.token_offset + start, 0, 1);
     return;
   }
   if (r == 0) {
     if (t == 0) write_sample(a, row, a.token_offset + maximum_id, 1, support);
     return;
+  }
+  if (range == 0.f) {  // all candidates equal: ordered by index
+    if (t == 0) write_sample(a, row, a.token_offset + start + r, 1, support);
+    return;
+  }
+
+  // The bin that holds rank r (every wave finds it, from BINS / 64 bins per
+  // lane and a prefix sum over the lanes); its few candidates go to a list and
+  // are ordered by direct comparison. A bin of more than LIST candidates (heavy
+  // ties, or one outlier that stretches the range) is left to the radix passes.
+  if (binned) {
+    constexpr int PL = BINS / 64;
+    uint32_t h[PL], total = 0;
+#pragma unroll
+    for (int i = 0; i < PL; ++i) {
+      h[i] = s_bins[lane * PL + i];
+      total += h[i];
+    }
+    uint32_t below = wave_prefix(total) - total;
+    const uint64_t here = __ballot(below <= r && r < below + total);
+    uint32_t bin = 0, in_bin = 0;
+    bool found = false;
+#pragma unroll
+    for (int i = 0; i < PL; ++i) {
+      if (!found) {
+        if (r < below + h[i]) {
+          found = true;
+          bin = uint32_t(lane * PL + i);
+          in_bin = h[i];
+        } else {
+          below += h[i];
+        }
+      }
+    }
+    const int owner = __builtin_ctzll(here);  // one lane: the bins hold all `count` > r candidates
+    bin = __builtin_amdgcn_readlane(bin, owner);
+    in_bin = __builtin_amdgcn_readlane(in_bin, owner);
+    below = __builtin_amdgcn_readlane(below, owner);
+    if (in_bin <= LIST) {  // uniform
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        if (bins[k] == bin) {
+          const uint32_t at = atomicAdd(&s_listed, 1u);
+          s_list_v[at] = vals[k];
+          s_list_i[at] = uint32_t(t) + uint32_t(k) * T;
+        }
+      }
+      __syncthreads();
+      if (wave != 0) return;
+      const uint32_t mine = min(uint32_t(lane), in_bin - 1);
+      const float v = s_list_v[mine];
+      const uint32_t ci = s_list_i[mine];
+      uint32_t rank = below;
+      for (uint32_t i = 0; i < in_bin; ++i) {
+        const float ov = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), int(i)));
+        const uint32_t oi = __builtin_amdgcn_readlane(ci, int(i));
+        rank += sample_before(ov, oi, v, ci) ? 1u : 0u;
+      }
+      if (uint32_t(lane) < in_bin && rank == r) write_sample(a, row, a.token_offset + start + ci, 1, support);
+      return;
+    }
   }
 
   // Radix select, 8 key bits per pass from the top: after four passes the
