@@ -709,9 +709,10 @@ AttentionPlan plan_flat(const ppk_context* ctx, uint32_t rows, uint32_t heads, c
 // The streaming quantize kernel (dense or append): one 16-byte load per lane
 // covers 16 bytes of a source row, so every source must be 16-byte aligned
 // and every code array aligned to the 8 (4 for f32 sources) codes a lane
-// stores; rows of all tensors are indexed in 32 bits. Batches of 4 units per
-// lane, one batch per lane up to 128 blocks of 256 lanes per CU. Returns
-// false (nothing launched) when the operands do not fit these conditions.
+// stores; rows of all tensors are indexed in 32 bits. A wave takes a chunk of
+// 256 units of one tensor; one chunk per wave up to 128 blocks of 4 waves per
+// CU, beyond which waves loop. Returns false (nothing launched) when the
+// operands do not fit these conditions.
 bool launch_stream_quantize(ppk_context* ctx, hipStream_t stream, int prof_kernel, QuantizeArgs k,
                             uint32_t head_dim) {
   const uint32_t per_lane = k.src_dtype == PPK_F32 ? 4u : 8u;
@@ -719,11 +720,16 @@ bool launch_stream_quantize(ppk_context* ctx, hipStream_t stream, int prof_kerne
     if (!aligned(k.src[t], 16) || !aligned(k.codes[t], per_lane)) return false;
   if (uint64_t(k.rows) * k.ntensors >= (uint64_t(1) << 32)) return false;
   const uint64_t units = uint64_t(k.ntensors) * k.rows * (head_dim / per_lane);
-  // Below one full block per CU (e.g. a decode round's single-token appends)
-  // the one-wave-per-row kernel spreads the rows wider and finishes sooner.
+  // Few rows (e.g. a decode round's single-token appends) finish sooner on the
+  // one-wave-per-row kernel, which spreads them wider: 8192-8704 rows 3.9-4.4
+  // us against 4.7 here. It pays per row, so above 48 rows per CU (25600 rows
+  // of D = 64: 7.3 us against 5.0) or one block per CU here it is left.
   const uint64_t cus = uint64_t(std::max(ctx->cu_count, 1));
-  if (units < cus * 1024) return false;
-  const uint64_t grid = std::min<uint64_t>((units + 1023) / 1024, cus * 128);
+  if (units < cus * 1024 && uint64_t(k.rows) * k.ntensors < cus * 48) return false;
+  const uint64_t chunks = k.ntensors * ((units / k.ntensors + 255) / 256);
+  const uint64_t grid = std::min<uint64_t>((chunks + 3) / 4, cus * 128);
+  k.token_div = fast_divisor(k.tokens);
+  k.head_div = fast_divisor(k.heads);
   const Fn fn = Fn((k.capacity ? kQuantizeAppend64 : kQuantizeDense64) + dim_index(head_dim));
   launch(ctx, prof_kernel, fn, uint32_t(grid), 256, 0, stream, k);
   return true;

@@ -40,6 +40,8 @@ struct QuantizeArgs {
   uint32_t src_dtype;       // PPK_F32 / PPK_BF16 / PPK_F16
   uint32_t ntensors;        // 1 or 2
   uint32_t uniform_past;    // append mode with past == nullptr: slot of token 0 for every row
+  FastDiv token_div;        // streaming append: by tokens
+  FastDiv head_div;         // streaming append: by heads
 };
 
 // Float-store append: copy [rows, tokens, row_bytes] token records of K and V

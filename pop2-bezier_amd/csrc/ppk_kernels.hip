@@ -617,153 +617,200 @@ __device__ __forceinline__ float group_max_nonneg(float x) {
   return __uint_as_float(b);
 }
 
+// absmax / 127 correctly rounded for every finite absmax whose quotient is not
+// below the scale's floor: the product with the rounded reciprocal, corrected
+// once by its exact remainder (Markstein's division by a constant). With the
+// floor applied it equals the IEEE division for all finite non-negative floats
+// (checked over all 2^31 of them). 3 instructions instead of ~12.
+__device__ __forceinline__ float row_scale(float amax) {
+  constexpr float kInv = 1.0f / 127.0f;
+  const float q = amax * kInv;
+  return fmaxf(__builtin_fmaf(__builtin_fmaf(-127.0f, q, amax), kInv, q), 1e-12f);
+}
+
 // Quantization at streaming rates: dense (int8_kv_ops::quantize over [rows,
 // D]) and quantize-and-append into arenas (rows of K and V written at slot
 // past[b] + t). A row's D values are split over G = D / E lanes, 16 bytes (E
 // values) per lane, so one wave-wide load covers 64 / G whole rows and the
-// row's absmax is a G-lane reduction; each lane then forms its E codes with
-// the same arithmetic as quantize_row (IEEE division, ties-to-even, clamp,
-// NaN quotient -> 0). Lanes hold two batches of R units and issue the next
-// batch's loads (and, for appends, the sequences' past entries) before the
-// current batch's stores. Loop control is uniform per wave (rows never
-// straddle waves: G divides 64), so the cross-lane reductions always run
-// with every lane active; units past the end are clamped for loading and
-// masked for storing. The host sends rows * ntensors < 2^32 here.
+// row's absmax is a G-lane reduction; each lane then forms the E codes of
+// quantize_row's arithmetic (IEEE division, ties-to-even, clamp, NaN quotient
+// -> 0), see below. A wave takes chunks of R * 64 consecutive units of one
+// tensor: all its addresses are one scalar base plus the lane plus constants,
+// its loads cover 4 KiB and its code stores 2 KiB (1 KiB for f32 sources) in
+// one piece, and its R * 64 / G scales leave in one store. An append's chunk
+// that lies in one row of the arena and within its capacity (a scalar test)
+// stores like a dense one; others index per lane.
+//
+// Bound by vector instructions before this split (each unit paid 64-bit
+// addresses and three divisions by runtime sizes, an IEEE division, and five
+// to six instructions per value: ~230 per unit, now ~65). Appends of K and V, bf16 -> int8, 32 x 16 x 1000 tokens
+// of D = 128: 92.3 -> 65.0 us (6.1 TB/s), 8 x 16 x 3000 of D = 256: 133.6 ->
+// 90.9; dense 1 M rows of D = 128: 77 -> 70 us.
 template <int D, int E, uint32_t DT, bool ARENA>
 __device__ __forceinline__ void quantize_stream_units(const ppk::QuantizeArgs& a) {
 #pragma clang fp contract(off)
   constexpr int G = D / E;
   constexpr int R = 4;
-  static_assert(64 % G == 0, "a row's lanes stay inside one wave");
+  constexpr uint32_t RU = 64 / G;    // rows per wave-wide load
+  constexpr uint32_t ROWS = R * RU;  // rows per chunk
+  static_assert(64 % G == 0 && G >= R, "a row's lanes stay inside one wave");
   using Code = typename std::conditional<E == 8, u2, uint32_t>::type;
   const int lane = threadIdx.x & 63;
+  const uint32_t gl = uint32_t(lane) % G, gr = uint32_t(lane) / G;
   const uint32_t rows = uint32_t(a.rows);  // per tensor
-  const uint64_t units = uint64_t(a.ntensors) * rows * G;
-  const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-  uint64_t wave_base = uint64_t(blockIdx.x) * blockDim.x + (threadIdx.x & ~63u);
-  if (wave_base >= units) return;  // uniform per wave
-  u4 cur[R], nxt[R];
-  uint32_t pcur[R], pnxt[R];  // appends: past entry of the unit's sequence
-  auto load = [&](uint64_t wb, u4 (&raw)[R], uint32_t (&pv)[R]) {
+  const uint32_t per_tensor = (rows + ROWS - 1) / ROWS;  // chunks; one never crosses from K to V
+  const uint32_t chunks = per_tensor * a.ntensors;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  bool any_bad = false, any_over = false;
+  for (uint32_t chunk = blockIdx.x * 4 + wave; chunk < chunks; chunk += gridDim.x * 4) {
+    const bool second = chunk >= per_tensor;
+    const uint32_t row0 = (second ? chunk - per_tensor : chunk) * ROWS;
+    const uint32_t left = rows - row0;  // rows of the tensor from here on, at least one
+    const u4* src = static_cast<const u4*>(second ? a.src[1] : a.src[0]) + uint64_t(row0) * G;
+    u4 raw[R];
+    if (left >= ROWS) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const uint64_t u = min(wb + uint64_t(lane) + r * stride, units - 1);  // clamp: in bounds, masked later
-      if constexpr (ARENA) {
-        const uint32_t ri = uint32_t(u / G);
-        const uint32_t t = ri >= rows ? 1u : 0u;
-        const uint32_t row = ri - t * rows;
-        const u4* src = static_cast<const u4*>(t ? a.src[1] : a.src[0]);
-        raw[r] = __builtin_nontemporal_load(src + uint64_t(row) * G + uint32_t(u % G));
-        pv[r] = a.past ? a.past[(row / a.tokens) / a.heads] : a.uniform_past;
+      for (int r = 0; r < R; ++r) raw[r] = __builtin_nontemporal_load(src + (lane + r * 64));
+    } else {  // the tensor's last rows: clamped for loading, masked for storing
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        raw[r] = __builtin_nontemporal_load(src + min(uint32_t(lane + r * 64), left * G - 1));
+    }
+    // Appends: the arena row of the chunk's first row, and whether all the
+    // chunk's rows follow it there.
+    uint64_t dst0 = row0;
+    bool plain = left >= ROWS;
+    uint32_t past_of[R];
+    bool one_row = true;
+    if constexpr (ARENA) {
+      const uint32_t bh = fast_div(row0, a.token_div);
+      const uint32_t t0 = row0 - bh * a.tokens;
+      one_row = left >= ROWS && uint64_t(t0) + ROWS <= a.tokens;
+      if (one_row) {
+        const uint64_t slot = uint64_t(a.past ? a.past[fast_div(bh, a.head_div)] : a.uniform_past) + t0;
+        plain = slot + ROWS <= a.capacity;
+        dst0 = uint64_t(bh) * a.capacity + slot;
       } else {
-        raw[r] = __builtin_nontemporal_load(static_cast<const u4*>(a.src[0]) + u);
+        plain = false;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const uint32_t row = row0 + min(r * RU + gr, left - 1);
+          past_of[r] = a.past ? a.past[fast_div(fast_div(row, a.token_div), a.head_div)] : a.uniform_past;
+        }
       }
     }
-  };
-  load(wave_base, cur, pcur);
-  bool any_bad = false, any_over = false;
-  for (; wave_base < units; wave_base += R * stride) {
-    const bool more = wave_base + R * stride < units;  // uniform per wave
-    if (more) load(wave_base + R * stride, nxt, pnxt);
+    Code code[R];
+    float scale[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const uint64_t u = wave_base + uint64_t(lane) + r * stride;
-      const bool valid = u < units;
       float x[E];
       if constexpr (DT == kF32) {
 #pragma unroll
-        for (int k = 0; k < E; ++k) x[k] = __uint_as_float(cur[r][k]);
+        for (int k = 0; k < E; ++k) x[k] = __uint_as_float(raw[r][k]);
       } else {
 #pragma unroll
         for (int k = 0; k < E; ++k) {
-          const uint16_t h = uint16_t(cur[r][k / 2] >> (16 * (k % 2)));
+          const uint16_t h = uint16_t(raw[r][k / 2] >> (16 * (k % 2)));
           x[k] = DT == kBF16 ? bf16_to_f32(h) : f16_to_f32(h);
         }
       }
       // Fast row max: the float max chain is exact unless the lane holds a
-      // NaN (a signalling one can drop the values before it); such a lane
-      // then has a NaN product below, and the wave recomputes.
+      // NaN (a signalling one can drop the values before it); such a lane is
+      // seen below, and the wave recomputes.
       float m = 0.f;
 #pragma unroll
       for (int k = 0; k < E; ++k) m = fmaxf(m, fabsf(x[k]));
-      float sc = fmaxf(group_max_nonneg<G>(m) / 127.0f, 1e-12f);
-      // Rounded quotients from a product with the hardware reciprocal (at
-      // most 1 ulp off 1/sc): for finite x, |x·r - RN(x/sc)| <= 2.7e-5 since
-      // |x/sc| <= 127·(1 + 2^-24), so a product farther than 2^-14 from every
-      // half-integer rounds to the same integer as the correctly rounded
-      // quotient. A product within that band, or a non-finite one (x or sc
-      // non-finite), marks its lane for the division. A product outside the
-      // band is also below 127.5 in magnitude, so its rounded value needs no
-      // clamp; the division path keeps the clamp.
+      float sc = row_scale(group_max_nonneg<G>(m));
+      // Rounded quotients in fixed point: u = 384 + x / sc from one fused
+      // multiply-add with the hardware reciprocal (at most 1 ulp off 1/sc).
+      // |x/sc| <= 127 (1 + 2^-24), so u lies in [256, 512), where a float's
+      // grid is 2^-15 and its mantissa is the quotient + 128 in 8.15 bits; u
+      // is within 2^-16 (its rounding) + 1.52e-5 (the reciprocal) + 3.9e-6
+      // (the quotient's own rounding) < 1.2 grid steps of RN(x/sc). Half a
+      // unit and 2 steps are added and the word shifted one up: byte 2 then
+      // holds the rounded quotient + 128, and the low 16 bits, in half
+      // steps, the distance above the half-integer less 2 steps. At 9 or more
+      // the rounding is that of RN(x/sc) (and needs no clamp: the value is
+      // clear of 127.5); at 8 or less (5 steps of 2^15: one value in 6500) the
+      // value is divided. A NaN or infinite u is the largest word (u is
+      // positive otherwise).
       const float rcp = __builtin_amdgcn_rcpf(sc);
-      int qi[E];
-      bool near[E], any_near = false;
+      constexpr uint32_t kStep = 2, kNear = 8;
+      uint32_t w[E];
+      uint32_t top = 0;
+      uint16_t low = 0xffff;
 #pragma unroll
       for (int k = 0; k < E; ++k) {
-        const float p = x[k] * rcp;
-        const float n = rintf(p);
-        near[k] = !(fabsf(p - n) < 0.5f - 0x1p-14f);
-        any_near = any_near || near[k];
-        qi[k] = int(n);
+        const uint32_t u = __float_as_uint(__builtin_fmaf(x[k], rcp, 384.0f));
+        w[k] = (u + (0x4000u + kStep)) << 1;
+        top = max(top, u);
+        low = min(low, uint16_t(w[k]));
       }
-      auto exact = [&](int k) {
-        const float t = rintf(x[k] / sc);
-        qi[k] = t != t ? 0 : int(__builtin_amdgcn_fmed3f(t, -127.f, 127.f));  // NaN quotient -> code 0
-      };
-      bool finite = true;
-      if (__any(any_near)) {  // wave-uniform
+      uint32_t packed[E / 4];
+#pragma unroll
+      for (int i = 0; i < E / 4; ++i) {
+        // v_perm: bytes 2 of (a, b) and of (c, d), then the two byte pairs.
+        const uint32_t ab = __builtin_amdgcn_perm(w[4 * i + 1], w[4 * i], 0x0c0c0602u);
+        const uint32_t cd = __builtin_amdgcn_perm(w[4 * i + 3], w[4 * i + 2], 0x0c0c0602u);
+        packed[i] = __builtin_amdgcn_perm(cd, ab, 0x05040100u) ^ 0x80808080u;
+      }
+      if (__any(low <= kNear || top >= 0x7f800000u)) {  // wave-uniform
+        bool finite = true;
 #pragma unroll
         for (int k = 0; k < E; ++k) finite = finite && __builtin_isfinite(x[k]);
-        if (__any(!finite)) {
-          // A non-finite input may have spoilt the fast max of its row: the
-          // wave recomputes every row it holds with the NaN-skipping max and
-          // the division (the reduction needs all lanes).
-          sc = fmaxf(group_max_nonneg<G>(lane_absmax(x)) / 127.0f, 1e-12f);
+        // A non-finite input may have spoilt the fast max of its row: the
+        // wave then recomputes every row it holds with the NaN-skipping max
+        // and the division (the reduction needs all lanes). With finite rows
+        // the scale stands and only the flagged values divide.
+        const bool all = __any(!finite);
+        if (all) sc = fmaxf(group_max_nonneg<G>(lane_absmax(x)) / 127.0f, 1e-12f);
 #pragma unroll
-          for (int k = 0; k < E; ++k) exact(k);
-        } else {
-          // Finite rows: the scale stands; only the flagged values divide.
-#pragma unroll
-          for (int k = 0; k < E; ++k)
-            if (near[k]) exact(k);
+        for (int k = 0; k < E; ++k) {
+          if (all || uint16_t(w[k]) <= kNear) {
+            const float t = rintf(x[k] / sc);
+            const uint32_t q = t != t ? 0u : uint32_t(int(__builtin_amdgcn_fmed3f(t, -127.f, 127.f)));
+            const int at = 8 * (k % 4);
+            packed[k / 4] = (packed[k / 4] & ~(0xffu << at)) | ((q & 0xffu) << at);
+          }
         }
+        any_bad = any_bad || (!finite && r * RU + gr < left);
       }
-      uint32_t packed[(E + 3) / 4];
-#pragma unroll
-      for (int w = 0; w < E / 4; ++w) {
-        // v_perm: bytes 0 of (a, b) and of (c, d), then the two byte pairs.
-        const uint32_t ab = __builtin_amdgcn_perm(uint32_t(qi[4 * w + 1]), uint32_t(qi[4 * w]), 0x0c0c0400u);
-        const uint32_t cd = __builtin_amdgcn_perm(uint32_t(qi[4 * w + 3]), uint32_t(qi[4 * w + 2]), 0x0c0c0400u);
-        packed[w] = __builtin_amdgcn_perm(cd, ab, 0x05040100u);
-      }
-      Code c;
-      if constexpr (E == 8) c = u2{packed[0], packed[1]};
-      else c = packed[0];
-      bool in_arena = true;
-      if constexpr (ARENA) {
-        const uint32_t ri = uint32_t(min(u, units - 1) / G);
-        const uint32_t t = ri >= rows ? 1u : 0u;
-        const uint32_t row = ri - t * rows;
-        const uint32_t bh = row / a.tokens;
-        const uint64_t slot = uint64_t(pcur[r]) + (row - bh * a.tokens);
-        in_arena = slot < a.capacity;
-        const uint64_t dst = uint64_t(bh) * a.capacity + slot;
-        if (valid && in_arena) {
-          __builtin_nontemporal_store(c, reinterpret_cast<Code*>(a.codes[t] + dst * D) + uint32_t(u % G));
-          if (lane % G == 0) a.scales[t][dst] = sc;
-        }
-      } else if (valid) {
-        __builtin_nontemporal_store(c, reinterpret_cast<Code*>(a.codes[0]) + u);
-        if (lane % G == 0) a.scales[0][u / G] = sc;
-      }
-      any_bad = any_bad || (valid && !finite);
-      any_over = any_over || (valid && !in_arena);
+      scale[r] = sc;
+      if constexpr (E == 8) code[r] = u2{packed[0], packed[1]};
+      else code[r] = packed[0];
     }
-    if (!more) break;
+    uint8_t* codes = second ? a.codes[1] : a.codes[0];
+    float* scales = second ? a.scales[1] : a.scales[0];
+    if (plain) {
+      Code* out = reinterpret_cast<Code*>(codes + dst0 * D);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      cur[r] = nxt[r];
-      pcur[r] = pnxt[r];
+      for (int r = 0; r < R; ++r) __builtin_nontemporal_store(code[r], out + (lane + r * 64));
+      float s = scale[0];
+#pragma unroll
+      for (int r = 1; r < R; ++r) s = gl == r ? scale[r] : s;
+      if (gl < R) (scales + dst0)[gl * RU + gr] = s;
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const uint32_t in = r * RU + gr;
+        bool store = in < left;
+        uint64_t dst = dst0 + in;
+        if constexpr (ARENA) {
+          const uint32_t row = row0 + min(in, left - 1);
+          const uint32_t bh = fast_div(row, a.token_div);
+          uint64_t slot = dst - uint64_t(bh) * a.capacity;  // one arena row: from its first slot
+          if (!one_row) {
+            slot = uint64_t(past_of[r]) + (row - bh * a.tokens);
+            dst = uint64_t(bh) * a.capacity + slot;
+          }
+          any_over = any_over || (store && slot >= a.capacity);
+          store = store && slot < a.capacity;
+        }
+        if (store) {
+          __builtin_nontemporal_store(code[r], reinterpret_cast<Code*>(codes + dst * D) + gl);
+          if (gl == 0) scales[dst] = scale[r];
+        }
+      }
     }
   }
   if (a.flags) {
