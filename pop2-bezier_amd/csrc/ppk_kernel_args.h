@@ -57,6 +57,7 @@ struct ScatterArgs {
   uint32_t pad;
 };
 
+constexpr uint32_t kDequantizeUnits = 4;  // 16-byte output units per lane and chunk
 struct DequantizeArgs {
   const uint8_t* codes;     // [rows, D]
   const float* scales;      // [rows]

@@ -456,69 +456,70 @@ __device__ __forceinline__ void quantize_body(const ppk::QuantizeArgs& a) {
 // Dequantize: 16 codes per thread (one dwordx4), grid-stride.
 // ---------------------------------------------------------------------------
 // Dequantization in units of one 16-byte output chunk: E = 8 codes for a
-// 16-bit output, 4 for f32. Lane l of a wave handles units i, i + stride, ...
-// so every load instruction of a wave reads 64*E consecutive code bytes and
-// every store instruction writes 1 KiB of consecutive output. Each lane keeps
-// two batches of R units: the next batch's loads are issued before the
-// current batch's stores, so a load never waits behind the previous batch's
-// store acknowledgements (loads and stores share one in-order counter). The
-// host sizes the grid for one batch per lane up to 128 blocks per CU (the
-// measured optimum; the grid-stride loop covers larger inputs).
+// 16-bit output, 4 for f32. A wave takes chunks of R * 64 consecutive units,
+// all loads of a chunk before its first store: each load instruction reads
+// 64*E consecutive code bytes, each store instruction writes 1 KiB, and the
+// chunk's output is one piece of R KiB. Addresses are a scalar base, the lane
+// and constants. Bound by memory, mostly by its writes (two thirds of the
+// bytes for a 16-bit output): where a wave's units lay a grid apart (and the
+// next batch was loaded before the stores), 1 M rows of D = 128 to bf16 took
+// 77 us, now 64. Eight units per lane measured the same. The host sizes the
+// grid for one chunk per wave up to 128 blocks per CU.
 template <int E, uint32_t OUT, bool ROUND>
 __device__ __forceinline__ void dequantize_units(const ppk::DequantizeArgs& a) {
 #pragma clang fp contract(off)
-  constexpr int R = 8;
+  constexpr uint32_t R = ppk::kDequantizeUnits;
   using Raw = typename std::conditional<E == 8, u2, uint32_t>::type;
   const uint64_t units = a.rows * (a.head_dim / E);
-  const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-  const uint32_t row_shift = __builtin_ctz(a.head_dim / E);  // units per token row: a power of two
-  uint64_t base = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (base >= units) return;
-  Raw cur[R], nxt[R];
-  float cs[R], ns[R];
-  auto load = [&](uint64_t b, Raw (&raw)[R], float (&sc)[R]) {
+  const uint32_t row_shift = __builtin_ctz(a.head_dim / E);  // units per token row: a power of two up to 64
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  const uint64_t step = uint64_t(gridDim.x) * 4 * R * 64;
+  for (uint64_t u0 = (uint64_t(blockIdx.x) * 4 + wave) * R * 64; u0 < units; u0 += step) {
+    const uint32_t left = uint32_t(min(units - u0, uint64_t(R * 64)));
+    const bool full = left == R * 64;
+    const Raw* codes = reinterpret_cast<const Raw*>(a.codes) + u0;
+    const float* scales = a.scales + (u0 >> row_shift);
+    Raw raw[R];
+    float sc[R];
+    if (full) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const uint64_t u = min(b + r * stride, units - 1);  // clamp: always in bounds, extra units unused
-      raw[r] = __builtin_nontemporal_load(reinterpret_cast<const Raw*>(a.codes) + u);
-      sc[r] = a.scales[u >> row_shift];
+      for (uint32_t r = 0; r < R; ++r) raw[r] = __builtin_nontemporal_load(codes + (lane + r * 64));
+#pragma unroll
+      for (uint32_t r = 0; r < R; ++r) sc[r] = (scales + ((r * 64) >> row_shift))[lane >> row_shift];
+    } else {
+#pragma unroll
+      for (uint32_t r = 0; r < R; ++r) {
+        const uint32_t u = min(lane + r * 64, left - 1);  // clamped: in bounds, masked for storing
+        raw[r] = __builtin_nontemporal_load(codes + u);
+        sc[r] = scales[u >> row_shift];
+      }
     }
-  };
-  load(base, cur, cs);
-  for (; base < units; base += R * stride) {
-    const bool more = base + R * stride < units;
-    if (more) load(base + R * stride, nxt, ns);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const uint64_t u = base + r * stride;
-      if (u >= units) break;
+    for (uint32_t r = 0; r < R; ++r) {
       float f[E];
 #pragma unroll
       for (int k = 0; k < E; ++k) {
         uint32_t w;
-        if constexpr (E == 8) w = cur[r][k / 4];
-        else w = cur[r];
-        const float v = sbyte(w, k % 4) * cs[r];
+        if constexpr (E == 8) w = raw[r][k / 4];
+        else w = raw[r];
+        const float v = sbyte(w, k % 4) * sc[r];
         f[k] = ROUND ? round_bf16(v) : v;
       }
+      u4 out;
       if constexpr (E == 4) {
-        __builtin_nontemporal_store(f4{f[0], f[1], f[2], f[3]}, static_cast<f4*>(a.out) + u);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) out[k] = __float_as_uint(f[k]);
       } else {
-        uint32_t h[4];
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           const uint16_t lo = OUT == kBF16 ? f32_to_bf16_bits(f[2 * w]) : f32_to_f16_bits(f[2 * w]);
           const uint16_t hi = OUT == kBF16 ? f32_to_bf16_bits(f[2 * w + 1]) : f32_to_f16_bits(f[2 * w + 1]);
-          h[w] = uint32_t(lo) | (uint32_t(hi) << 16);
+          out[w] = uint32_t(lo) | (uint32_t(hi) << 16);
         }
-        __builtin_nontemporal_store(u4{h[0], h[1], h[2], h[3]}, static_cast<u4*>(a.out) + u);
       }
-    }
-    if (!more) break;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      cur[r] = nxt[r];
-      cs[r] = ns[r];
+      if (full || lane + r * 64 < left)
+        __builtin_nontemporal_store(out, static_cast<u4*>(a.out) + u0 + (lane + r * 64));
     }
   }
 }
