@@ -156,8 +156,8 @@ static uint32_t score_tokens(uint32_t split, uint32_t batch) {
 
 // How a row's waves take its batches, by the batches of one wave's share
 // (q = ceil(split / batch)). Shares of six batches or more within 1/16 of
-// whole pairs, and below 32: two batches at a time in turn. Shares of three, at least 2.5
-// batches: one contiguous range per wave (the whole of K is in flight at
+// whole pairs, and below 32: two batches at a time in turn. Shares of three, at
+// least 2.5 batches: one contiguous range per wave (the whole of K is in flight at
 // once, and turns only mix the waves' pages). Others: one batch at a time.
 // Same-box A/B, H = 16, us per step, contiguous ranges / turns of one / turns
 // of two / turns of four: B = 32 x 8192 D = 128 161.2 / 159.1 / 160.3 /
@@ -524,10 +524,25 @@ uint64_t per_row_cu_peak(const AttentionPlan& p, uint32_t rows, uint32_t heads, 
                          uint64_t limit, uint32_t cus) {
   std::vector<uint64_t> load(cus, 0);
   const uint64_t per_block = uint64_t(p.waves) * p.split;  // tokens of a row one block covers
-  for (uint32_t r = 0; r < rows; ++r) {
-    const uint64_t len = host[r / heads] <= limit ? host[r / heads] : 0;
-    for (uint64_t g = 0; g < p.ngroups && g * per_block < len; ++g)  // blocks numbered group-major
-      load[(g * rows + r) % cus] += std::min(per_block, len - g * per_block);
+  // Blocks are numbered group-major, so in that order the CU is a counter
+  // (divisions, per block here, per unit below and per sequence and step of
+  // plan_flat's search, were most of a plan's time: 24 ragged sequences of 16
+  // heads 7.9 -> 2.6 us of host time per plan, twice per decode step).
+  uint32_t cu = 0;
+  for (uint64_t g = 0; g < p.ngroups; ++g) {
+    const uint64_t t0 = g * per_block;
+    for (uint32_t b = 0; b < rows / heads; ++b) {
+      const uint64_t len = host[b] <= limit ? host[b] : 0;
+      if (len <= t0) {
+        cu = uint32_t((uint64_t(cu) + heads) % cus);
+        continue;
+      }
+      const uint64_t tokens = std::min(per_block, len - t0);
+      for (uint32_t h = 0; h < heads; ++h) {
+        load[cu] += tokens;
+        cu = cu + 1 == cus ? 0 : cu + 1;
+      }
+    }
   }
   return *std::max_element(load.begin(), load.end());
 }
@@ -535,14 +550,21 @@ uint64_t per_row_cu_peak(const AttentionPlan& p, uint32_t rows, uint32_t heads, 
 uint64_t flat_cu_peak(const AttentionPlan& p, uint32_t heads, uint32_t cus) {
   std::vector<uint64_t> load(cus, 0);
   const FlatTable& t = p.table;
-  uint64_t unit = 0;  // unit u on block u / waves (the int8 kernel's assignment)
+  uint32_t cu = 0, wave = 0;  // unit u on block u / waves (the int8 kernel's assignment), counted along
   for (uint32_t b = 0; b < t.batch; ++b) {
     const uint32_t len = t.seq[b].len, units = t.seq[b].units & 0xffffffu;
-    for (uint32_t h = 0; h < heads; ++h)
-      for (uint32_t s = 0; s < units; ++s, ++unit) {
-        const uint64_t t0 = uint64_t(s) * t.share;
-        if (len > t0) load[(unit / p.waves) % cus] += std::min<uint64_t>(t.share, len - t0);
+    for (uint32_t h = 0; h < heads; ++h) {
+      uint32_t left = len;
+      for (uint32_t s = 0; s < units; ++s) {
+        const uint32_t tokens = std::min(t.share, left);
+        load[cu] += tokens;
+        left -= tokens;
+        if (++wave == p.waves) {
+          wave = 0;
+          cu = cu + 1 == cus ? 0 : cu + 1;
+        }
       }
+    }
   }
   return *std::max_element(load.begin(), load.end());
 }
@@ -665,9 +687,11 @@ AttentionPlan plan_flat(const ppk_context* ctx, uint32_t rows, uint32_t heads, c
   // max(1, ceil(len / Q)) falls as Q grows, and Q = ceil(T / (waves - rows))
   // always fits (units <= T / Q + rows), so a binary search between 64 and it.
   auto units_for = [&](uint64_t q) {
+    // ceil(len / q) in 32 bits: (len - 1) / q + 1, and one unit for no tokens.
+    const uint32_t d = uint32_t(std::min<uint64_t>(q, 0xffffffffu));
     uint64_t u = 0;
-    for (uint32_t b = 0; b < t.batch; ++b) u += uint64_t(heads) * std::max<uint64_t>(1, (t.seq[b].len + q - 1) / q);
-    return u;
+    for (uint32_t b = 0; b < t.batch; ++b) u += t.seq[b].len ? (t.seq[b].len - 1) / d + 1 : 1;
+    return u * heads;
   };
   const uint64_t spare = waves - rows;
   uint64_t lo = kMinUnit, hi = std::max<uint64_t>((total + spare - 1) / spare, kMinUnit);

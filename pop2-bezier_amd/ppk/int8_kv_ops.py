@@ -49,7 +49,9 @@ def current_stream_handle(device: torch.device) -> ctypes.c_void_p:
 
 
 def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    if not t.is_cuda:  # torch's own error
+        return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return current_stream_handle(t.device)
 
 
 def _require(cond: bool, message: str) -> None:

@@ -17,7 +17,7 @@ import torch
 
 from . import _abi
 from ._abi import check, lib
-from .int8_kv_ops import _DTYPES, _stream, context
+from .int8_kv_ops import _DTYPES, _stream, context, current_stream_handle
 
 KINDS = {"int8": _abi.PPK_KV_INT8, torch.bfloat16: _abi.PPK_KV_BF16, torch.float16: _abi.PPK_KV_F16,
          torch.float32: _abi.PPK_KV_F32}
@@ -35,6 +35,12 @@ def _hip_runtime() -> ctypes.CDLL:
                                           ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int, ctypes.c_void_p]
         _hip.hipMemcpy2DAsync.restype = ctypes.c_int
     return _hip
+
+
+def _device_stream(device: torch.device | int | None) -> ctypes.c_void_p:
+    if device is None or not torch.cuda.is_initialized():
+        return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return current_stream_handle(torch.device("cuda", device) if isinstance(device, int) else torch.device(device))
 
 
 def _write(k: torch.Tensor, v: torch.Tensor, tokens: int, commit: bool) -> _abi.PpkKvWrite:
@@ -202,7 +208,7 @@ class LayerCache:
         if k is None and v is None:
             w = _abi.PpkKvWrite(struct_size=ctypes.sizeof(_abi.PpkKvWrite), src_dtype=_abi.PPK_BF16, tokens=1,
                                 commit=int(bool(commit)), k=None, v=None)
-            stream = ctypes.c_void_p(torch.cuda.current_stream(caches[0].device).cuda_stream) if b else None
+            stream = _device_stream(caches[0].device) if b else None
         else:
             if k.dim() != 4 or k.shape[0] != b or k.shape[2] != 1:
                 raise ValueError("batch KV requires [B,H,1,D] scratch and matching row histories")
@@ -259,9 +265,10 @@ def decode_step(view: _abi.PpkKvView, q: torch.Tensor, k_new: torch.Tensor, v_ne
     step = _step_args(a, k_new, v_new, flags, d)
     ctx = context(q.device)
     nbytes = workspace_bytes(a, ctx)
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=q.device)
-    step.attn.workspace = ws.data_ptr()
-    step.attn.workspace_bytes = nbytes
+    if nbytes:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+        step.attn.workspace = ws.data_ptr()
+        step.attn.workspace_bytes = nbytes
     check(lib().ppk_decode_step(ctx, _stream(q), ctypes.byref(step)), "ppk_decode_step")
     return out
 
