@@ -394,7 +394,7 @@ __device__ __forceinline__ void raise_flags(uint32_t* flags, uint32_t bits) {
 // (one value at one address): a lane-0 branch here would make the compiler
 // restructure the control flow around it, and the decode kernels' streaming
 // loops then wait for loads of paths that never reach them.
-template <int D>
+template <int D, bool ONE = false>
 __device__ __forceinline__ bool quantize_values(const float (&x)[D / ppk::kWave], uint8_t* codes, float* scale,
                                                 int lane) {
 #pragma clang fp contract(off)
@@ -415,7 +415,7 @@ __device__ __forceinline__ bool quantize_values(const float (&x)[D / ppk::kWave]
   if constexpr (EPL == 1) *out = uint8_t(packed);
   else if constexpr (EPL == 2) *reinterpret_cast<uint16_t*>(out) = uint16_t(packed);
   else *reinterpret_cast<uint32_t*>(out) = packed;
-  *scale = s;
+  if (!ONE || lane == 0) *scale = s;
   return __any(!finite);
 }
 
@@ -426,7 +426,7 @@ __device__ __forceinline__ void quantize_row(const void* src, size_t src_row, ui
   constexpr int EPL = D / ppk::kWave;
   float x[EPL];
   load_vec<EPL>(src, src_row * D + size_t(lane) * EPL, dtype, x);
-  if (quantize_values<D>(x, codes, scale, lane) && flags && lane == 0) atomicOr(flags, 1u);
+  if (quantize_values<D, true>(x, codes, scale, lane) && flags && lane == 0) atomicOr(flags, 1u);
 }
 
 template <int D>
