@@ -1188,9 +1188,10 @@ __device__ __forceinline__ void write_block_record(float* rec, int ch, int lane,
 // Log-sum-exp combine of a block's W <= MAXW records (stride floats apart) and
 // a score s0 that joins the maximum (-inf for none), by one wave: lane w takes
 // record w's (m, z), the y rows of this lane's channels are requested eight
-// records at a time (past W: the last record again, with weight 0). One LDS
-// round trip for the weights and one for the rows; a loop over the records
-// took two per record, ~0.7 us at the end of every 8-wave block.
+// records at a time (past W: the last record again, left out of the sum: a
+// weight of 0 would make an infinite y of that record NaN). One LDS round trip
+// for the weights and one for the rows; a loop over the records took two per
+// record, ~0.7 us at the end of every 8-wave block.
 template <int D, int MAXW>
 __device__ __forceinline__ void combine_block(const float* recs, uint32_t stride, uint32_t W, int lane, float s0,
                                               float& m, float& z, float (&y)[D / ppk::kWave]) {
@@ -1217,6 +1218,7 @@ __device__ __forceinline__ void combine_block(const float* recs, uint32_t stride
   auto add = [&](uint32_t w0) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
+      if (w0 + uint32_t(k) >= W) break;  // uniform
       const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wt), int(w0) + k));
 #pragma unroll
       for (int e = 0; e < EPL; ++e) y[e] = fmaf(wk, v[k][e], y[e]);
