@@ -1540,12 +1540,15 @@ __device__ __forceinline__ void combine_records(const float* mz, const float* py
       }
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        // Record i + k's weight sits in that lane (a uniform index): one readlane, no LDS.
-        const float wk = i + uint32_t(k) < cnt
-                             ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), int(i) + k))
-                             : 0.f;
+        // Record i + k's weight sits in that lane (a uniform index, 0 past the
+        // last record): one readlane, no LDS. Past it the y row counts as 0
+        // too (0 times an infinite y would be NaN); selected, not branched: a
+        // branch per record would hold the next eight records' loads back
+        // (36 records, 8 rows of D = 128: 10.4 us against 8.9).
+        const bool live = i + uint32_t(k) < cnt;
+        const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), int(i) + k));
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) y[e] = fmaf(wk, v[k][e], y[e]);
+        for (int e = 0; e < EPL; ++e) y[e] = fmaf(wk, live ? v[k][e] : 0.f, y[e]);
       }
     }
   }

@@ -1,7 +1,7 @@
 """Infinite values in a float KV store reach the output as the plain softmax has them: the channel that holds one
-is infinite, every other channel finite. The value lies in the share of the block's last wave (and not in its
-last token), for blocks of one to twelve waves: the combine of a block's records may not give the records that
-are not there a say."""
+is infinite, every other channel finite. The value lies in the share of the row's last wave (and not in its
+last token), for blocks of one to twelve waves and for rows of several blocks: the combines of a block's and of a
+row's records may not give the records that are not there a say."""
 from __future__ import annotations
 
 import numpy as np
@@ -15,9 +15,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("kv", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("waves", [1, 2, 3, 5, 7, 8, 9, 12])
+@pytest.mark.parametrize("waves,blocks", [(1, 1), (2, 1), (3, 1), (5, 1), (7, 1), (8, 1), (9, 1), (12, 1), (18, 2), (39, 3),
+                                          (144, 9), (272, 17)])
 @pytest.mark.parametrize("D", [64, 256])
-def test_infinite_value_in_the_last_wave(device, kv, waves, D):
+def test_infinite_value_in_the_last_wave(device, kv, waves, blocks, D):
     share, rows, heads = 32, 4, 2  # 32 tokens: whole batches at every width, so no token is read twice
     n = waves * share
     rng = np.random.default_rng(SEED + waves + D)
@@ -30,7 +31,7 @@ def test_infinite_value_in_the_last_wave(device, kv, waves, D):
     lengths = torch.full((rows // heads,), n, dtype=torch.int32, device=device)
     args, _ = ppk.fused_attention.decode_attention_args(q, k, v, lengths, heads, share)
     info = ppk.fused_attention.plan_info(args, ppk.context(device))
-    assert (info["nsplits"], info["waves_per_block"]) == (1, waves)
+    assert (info["nsplits"], info["waves_per_block"]) == (blocks, waves // blocks)
     out = ppk.fused_attention.decode_attention(q, k, v, lengths, heads, share)
     torch.cuda.synchronize()
     got = out.reshape(rows, D).double().cpu().numpy()
