@@ -1068,21 +1068,6 @@ AttentionPlan plan_float_attention(const ppk_context* ctx, const PpkFloatAttenti
              per_row_waves_uneven(batch, host, span, plan.split)) {
     plan = plan_flat(ctx, a.rows, a.heads, host, span, a.head_dim);
   }
-  if (!plan.flat) {
-    // Shares of 16 batches or more: the row's waves take its batches in turn,
-    // as on the int8 path. Shorter shares: one contiguous range per wave, each
-    // wave starting at a batch of its own (turns would have the waves of rows
-    // a power of two apart meet in the same memory banks). Same-box A/B, bf16,
-    // H = 16, us per step, contiguous / turns: B = 32 x 8192 D = 128 310.0 /
-    // 302.5, x 1024 in 1024 slots 42.3 / 41.3, B = 16 x 4096 in 4096 81.8 /
-    // 79.0, B = 32 x 4000 D = 64 79.0 / 76.4; shares of eight batches, B = 8 x
-    // 4000 D = 64 23.4 / 23.9, B = 16 x 2000 21.1 / 21.5, of four, x 1000 11.9
-    // / 12.4.
-    const uint32_t batch = 4 * std::max<uint32_t>(tpl, 1u);
-    plan.turn = plan_turns(plan, batch);
-    plan.turn.shift = plan.split > 15 * batch ? 0 : 31;
-    plan.turn.chunk = 1;
-  }
   plan.span = uint32_t(span);
   return plan;
 }
@@ -1134,7 +1119,6 @@ void run_float_attention(ppk_context* ctx, hipStream_t stream, const PpkFloatAtt
   d.size = a.size;
   d.split_tokens = plan.split;
   d.ngroups = plan.ngroups;
-  d.turn = plan.turn;
   d.q_dtype = a.q_dtype;
   d.out_dtype = a.out_dtype;
   d.scale_log2 = scale * 1.4426950408889634f;

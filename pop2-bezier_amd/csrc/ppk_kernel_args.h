@@ -217,7 +217,6 @@ struct FloatDecodeArgs {
   uint32_t span;            // most tokens a row may attend (<= size)
   uint32_t new_dtype;
   FastDiv row_div, head_div;  // by rows, by heads
-  Turns turn;               // per-row plan: shift 0, turns of one batch; else contiguous ranges of split_tokens
 };
 
 struct FloatMergeArgs {

@@ -2031,17 +2031,15 @@ struct FloatWavePartial {
   float acc[FloatGeom<D, BF16KV>::kEpc];
 };
 
-// One wave streams its share of a row: phase K scores into LDS, phase V
-// accumulation; A/B batches ping-pong, and the last phase-K iteration already
-// fetches the first V batches. The share is the n tokens from `begin`, or, when
-// the row's waves take its batches in turn (a.turn.shift == 0), the batches
-// bt of the row's n tokens. early() leaves the query chunk in qr, with the
-// first two batches in flight.
+// One wave streams n tokens of a row from `begin`: phase K scores into LDS,
+// phase V accumulation; A/B batches ping-pong, and the last phase-K iteration
+// already fetches the first V batches. early() leaves the query chunk in qr,
+// with the first two batches in flight.
 template <int D, bool BF16KV, class Early>
 __device__ __forceinline__ void fwave_attention(const ppk::FloatDecodeArgs& a, uint32_t row, uint32_t begin,
-                                                uint32_t n, const Batches& bt,
-                                                const float (&qr)[FloatGeom<D, BF16KV>::kEpc], float* s_lds, int lane,
-                                                FloatWavePartial<D, BF16KV>& out, Early early) {
+                                                uint32_t n, const float (&qr)[FloatGeom<D, BF16KV>::kEpc],
+                                                float* s_lds, int lane, FloatWavePartial<D, BF16KV>& out,
+                                                Early early) {
   using G = FloatGeom<D, BF16KV>;
   constexpr int U = 4;
   constexpr int TPB = U * G::kTpl;
@@ -2051,8 +2049,7 @@ __device__ __forceinline__ void fwave_attention(const ppk::FloatDecodeArgs& a, u
   out.z = 0.f;
 #pragma unroll
   for (int i = 0; i < G::kEpc; ++i) out.acc[i] = 0.f;
-  const bool turns = a.turn.shift == 0;
-  const uint32_t nb = turns ? bt.count : (n + TPB - 1) / TPB;
+  const uint32_t nb = (n + TPB - 1) / TPB;
   if (nb == 0) {  // uniform per wave
     early();
     return;
@@ -2063,7 +2060,7 @@ __device__ __forceinline__ void fwave_attention(const ppk::FloatDecodeArgs& a, u
   const char* vb = static_cast<const char*>(a.v) +
                    (size_t(row) * a.v_stride + size_t(begin) * D) * G::kElemBytes + size_t(c) * ppk::kLaneBytes;
   const float sl2 = a.scale_log2;
-  // A contiguous range is taken in a rotated order: the wave starts at batch rot of
+  // Each wave takes its batches in a rotated order: it starts at batch rot of
   // its nb batches and wraps, and phase V follows the same order. Waves that
   // start at the same offset of rows a power of two apart (a store of 4096 or
   // 8192 tokens) otherwise move through the same HBM channels in step. rot is
@@ -2078,32 +2075,35 @@ __device__ __forceinline__ void fwave_attention(const ppk::FloatDecodeArgs& a, u
   // 8192 D=128 310.5 -> 309.0 us. It costs where a few long rows stream one
   // wave per CU: 4 x 8192 + 28 x 512 tokens on the per-row plan 112.2 ->
   // 115.7 us (the balanced plan, which host lengths select, does not rotate).
+  // Contiguous at any share: taking a row's batches in turn, as the int8 kernel
+  // does, gained up to 3 % on uniform rows of a power of two tokens (B=32 x
+  // 8192 D=128 309.9 -> 301.1 us) and lost up to 12 % on ragged ones (B=32 of
+  // 256..8192 175.2 -> 181.8); over 544 shapes it was 2-3 % slower.
   const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
-  const uint32_t rot = turns ? 0u : ((wave_id * 0x9E37u & 0xFFFFu) * nb) >> 16;
-  // Logical batch b: its place among the wave's batches (its scores' place in
-  // LDS) and its first tile. Past the end: a tile past the row's or range's.
-  auto place = [&](uint32_t b) { return b < nb ? (b + rot >= nb ? b + rot - nb : b + rot) : nb; };
-  auto tile = [&](uint32_t b) { return turns ? bt.tile(b) : (b < nb ? place(b) : b) * U; };
+  const uint32_t rot = ((wave_id * 0x9E37u & 0xFFFFu) * nb) >> 16;
+  // Logical batch b -> its place in the range; past the end: past the range.
+  auto place = [&](uint32_t b) { return b < nb ? (b + rot >= nb ? b + rot - nb : b + rot) : b; };
 
   u4 ra[U], rb[U];
   float mloc = -INFINITY;
   auto score = [&](const u4 (&r)[U], uint32_t b) {
-    if (b < nb) mloc = fscore_batch<D, BF16KV, U>(r, tile(b), n, j, c, qr, sl2, s_lds + place(b) * TPB, mloc);
+    if (b < nb)
+      mloc = fscore_batch<D, BF16KV, U>(r, place(b) * U, n, j, c, qr, sl2, s_lds + place(b) * TPB, mloc);
   };
   // Both first batches go out before anything waits for the query: with the
   // second behind that wait, rows of a few batches paid up to one more memory
   // round trip (captured sequences, us: 8 rows x 1145 tokens at D = 128 7.58 /
   // 7.43, step 7.93 / 7.70; 256 rows of up to 28 at D = 128 4.34 / 4.25).
-  load_fbatch<D, BF16KV, U>(kb, tile(0), n, j, ra);
-  load_fbatch<D, BF16KV, U>(kb, tile(1), n, j, rb);
+  load_fbatch<D, BF16KV, U>(kb, place(0) * U, n, j, ra);
+  load_fbatch<D, BF16KV, U>(kb, place(1) * U, n, j, rb);
   issue_here();
   early();
   for (uint32_t b = 0; b < nb; b += 2) {
     const bool last = b + 2 >= nb;
     score(ra, b);
-    load_fbatch<D, BF16KV, U>(last ? vb : kb, tile(last ? 0 : b + 2), n, j, ra);
+    load_fbatch<D, BF16KV, U>(last ? vb : kb, place(last ? 0 : b + 2) * U, n, j, ra);
     score(rb, b + 1);
-    load_fbatch<D, BF16KV, U>(last ? vb : kb, tile(last ? 1 : b + 3), n, j, rb);
+    load_fbatch<D, BF16KV, U>(last ? vb : kb, place(last ? 1 : b + 3) * U, n, j, rb);
   }
   float m = mloc;
   m = groups_max<G::kLpt>(m);
@@ -2112,13 +2112,13 @@ __device__ __forceinline__ void fwave_attention(const ppk::FloatDecodeArgs& a, u
   float z = 0.f;
   auto accumulate = [&](const u4 (&r)[U], uint32_t b) {
     if (b < nb)
-      faccumulate_batch<D, BF16KV, U>(r, tile(b), n, j, lane, m, s_lds + place(b) * TPB, z, out.acc);
+      faccumulate_batch<D, BF16KV, U>(r, place(b) * U, n, j, lane, m, s_lds + place(b) * TPB, z, out.acc);
   };
   for (uint32_t b = 0; b < nb; b += 2) {
     accumulate(ra, b);
-    load_fbatch<D, BF16KV, U>(vb, tile(b + 2), n, j, ra);
+    load_fbatch<D, BF16KV, U>(vb, place(b + 2) * U, n, j, ra);
     accumulate(rb, b + 1);
-    load_fbatch<D, BF16KV, U>(vb, tile(b + 3), n, j, rb);
+    load_fbatch<D, BF16KV, U>(vb, place(b + 3) * U, n, j, rb);
   }
   z = wave_sum(z);
   reduce_scatter_groups<G::kLpt, G::kEpc>(out.acc, lane);
@@ -2171,8 +2171,7 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
   const uint32_t len = a.lengths ? a.lengths[seq] : a.size;
   __asm__ volatile("" ::"s"(seq), "s"(a.q), "s"(a.k), "s"(a.v), "s"(a.k_new), "s"(a.v_new), "s"(a.q_stride), "s"(a.k_stride),
                    "s"(a.v_stride), "s"(a.size), "s"(a.split_tokens), "s"(a.ngroups), "s"(a.q_dtype),
-                   "s"(a.new_dtype), "s"(a.scale_log2), "s"(a.span), "s"(a.turn.div.mul), "s"(a.turn.div.shift),
-                   "s"(a.turn.shift), "s"(a.turn.chunk), "s"(a.turn.tokens), "s"(blockDim.x));
+                   "s"(a.new_dtype), "s"(a.scale_log2), "s"(a.span), "s"(blockDim.x));
   const int W = blockDim.x >> 6;
   const uint32_t S = a.split_tokens;
   bool valid;
@@ -2196,12 +2195,8 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
   if (kw || cur) load_raw<EPL>(a.k_new, own, a.new_dtype, kn_raw);
   if (vw || cur) load_raw<EPL>(a.v_new, own, a.new_dtype, vn_raw);
   if (cur) load_raw<EPL>(a.q, size_t(row) * a.q_stride + size_t(lane) * EPL, a.q_dtype, qc_raw);
-  // This wave's share: a contiguous range of S tokens, or (a.turn) its turns of the row.
-  const bool turns = a.turn.shift == 0;
-  const uint32_t place = group * W + wave;
-  const uint32_t begin = turns ? 0u : place * S;
-  const uint32_t n = !valid || begin >= len ? 0u : turns ? len : min(S, len - begin);
-  const Batches bt = row_batches<4 * G::kTpl>(a.turn, turns ? n : 0u, place, a.ngroups * W);
+  const uint32_t begin = (group * W + wave) * S;
+  const uint32_t n = (valid && begin < len) ? min(S, len - begin) : 0u;
 
   float qr[G::kEpc], kcur[EPL], vcur[EPL];
   float s_cur = -INFINITY;
@@ -2228,10 +2223,11 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
     if (vw) raise |= write_current<EPL, BF16KV>(const_cast<void*>(a.v), a.v_stride, row, len, a.size, vcur, lane);
   };
   FloatWavePartial<D, BF16KV> part;
-  // LDS of this wave alone: a score per token of its share, then its record.
-  const uint32_t lds_stride = max(a.turn.tokens, uint32_t(D + 4));
+  // LDS of this wave alone: a score per token of its batches, then its record.
+  constexpr uint32_t TPB = 4 * G::kTpl;
+  const uint32_t lds_stride = max((S + TPB - 1) / TPB * TPB, uint32_t(D + 4));
   float* s_lds = lds + size_t(wave) * lds_stride;
-  fwave_attention<D, BF16KV>(a, row, begin, n, bt, qr, s_lds, lane, part, early);
+  fwave_attention<D, BF16KV>(a, row, begin, n, qr, s_lds, lane, part, early);
 
   // Combine the block's waves through LDS: each wave's record replaces its
   // scores (its own LDS, so no barrier is needed before).
