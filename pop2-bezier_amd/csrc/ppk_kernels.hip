@@ -1311,8 +1311,7 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   constexpr int TPB = U * TPL;
   const uint32_t place = group * W + wave, turns = a.ngroups * W;
   const uint64_t cover = uint64_t(turns) * S;
-  const uint32_t nspec = a.speculate ? uint32_t(min(uint64_t(a.capacity), cover)) : 0u;
-  const Batches early = row_batches<TPB>(a.turn, nspec, place, turns);
+  uint32_t nspec = uint32_t(min(uint64_t(a.capacity), cover));
   const size_t tok0 = size_t(row) * a.capacity;
   const uint8_t* kb = a.k + tok0 * D + size_t(c) * 16;
   const uint8_t* vb = a.v + tok0 * D + size_t(c) * 16;
@@ -1397,8 +1396,20 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   auto load_v = [&](int b, const Batches& of, uint32_t limit) {
     load_batch<D, U>(vb, vsb, of.tile(uint32_t(b)), limit, j, lane, va[b], vsa[b]);
   };
-  auto prologue = [&]() {
+  // The batches to request: the covered row's, or, without speculation, the
+  // row's own (then its length is waited for here; the operands that came with
+  // it wait until the batches are on their way). Either way a wave of one or
+  // two batches requests K and V together, and does no arithmetic on a batch
+  // that is not there: with ragged host lengths and the bf16 history, which
+  // that arithmetic bounds, one-batch waves took 8.4 us where they did both
+  // (64 rows of 181..362 tokens at D = 64), now 6.0.
+  if (!a.speculate) {
     length_here();
+    nspec = n;
+  }
+  const Batches early = row_batches<TPB>(a.turn, nspec, place, turns);
+  auto prologue = [&]() {
+    if (a.speculate) length_here();
     operands_here();
   };
   // The paths differ in what is in flight when the prologue runs; each runs
@@ -1415,30 +1426,24 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
     load_v(0, early, nspec);
     load_v(1, early, nspec);
     prologue();
-    if (bt.count > 0) short_attention<D, BF16H, 2>(rr, rs, va, vsa, early, n, lane, query, part);
+    if (bt.count == 2) short_attention<D, BF16H, 2>(rr, rs, va, vsa, early, n, lane, query, part);
+    else if (bt.count == 1) short_attention<D, BF16H, 1>(rr, rs, va, vsa, early, n, lane, query, part);
+  } else if (early.count == 0) {
+    prologue();
   } else {
-    if (early.count > 0) {
 #pragma unroll
-      for (int b = 0; b < NB; ++b) load_k(b, early, nspec);
-      prologue();
-    } else {
-      // The length decides the first batches; the operands that came with it wait until those are on their way.
-      length_here();
-      if (bt.count > 0) {
-#pragma unroll
-        for (int b = 0; b < NB; ++b) load_k(b, bt, n);
-        operands_here();
-      } else {
-        operands_here();
-      }
-    }
+    for (int b = 0; b < NB; ++b) load_k(b, early, nspec);
+    prologue();
     if (bt.count > 2) {
       settle_all();  // long done, but not on every edge the compiler gives this block
       ring_attention<D, BF16H, NB>(kb, vb, ksb, vsb, bt, n, query, s_lds, lane, part, rr, rs);
-    } else if (bt.count > 0) {
+    } else if (bt.count == 2) {
       load_v(0, bt, n);
       load_v(1, bt, n);
       short_attention<D, BF16H, 2>(rr, rs, va, vsa, bt, n, lane, query, part);
+    } else if (bt.count == 1) {
+      load_v(0, bt, n);
+      short_attention<D, BF16H, 1>(rr, rs, va, vsa, bt, n, lane, query, part);
     }
   }
   PPK_CLK(4);
