@@ -505,15 +505,26 @@ uint64_t row_cover(const uint32_t* host, uint32_t batch, uint64_t limit) {
   return std::max<uint64_t>(longest_live(host, batch, limit), 1);
 }
 
+// Of a row's batches of `batch` tokens, those that are among the first
+// kRing of their wave: what the waves request early, summed over the row's
+// waves (turns of two counted as turns of one).
+static uint64_t early_batches(const AttentionPlan& p, uint64_t tokens, uint32_t batch) {
+  constexpr uint64_t kRing = 3;  // as in ppk_kernels.hip
+  const uint64_t waves = uint64_t(p.ngroups) * p.waves, batches = (tokens + batch - 1) / batch;
+  if (p.turn.shift != 31) return std::min(batches, waves * kRing);
+  const uint64_t chunk = p.turn.chunk, whole = batches / chunk;
+  if (whole >= waves) return waves * std::min(chunk, kRing);
+  return whole * std::min(chunk, kRing) + std::min(batches % chunk, kRing);
+}
+
 bool per_row_speculates(const AttentionPlan& p, uint32_t rows, uint32_t heads, const uint32_t* host, uint64_t span,
                         uint64_t limit, uint32_t batch) {
-  const uint64_t per_row = uint64_t(p.ngroups) * p.waves;
+  if (!host) return true;
+  const uint64_t batches = rows / heads;
   uint64_t live = 0;
-  for (uint32_t b = 0; b < rows / heads; ++b) {
-    const uint64_t len = host ? (host[b] <= limit ? host[b] : 0) : span;
-    live += heads * std::min<uint64_t>(per_row, (len + batch - 1) / batch);
-  }
-  const uint64_t total = per_row * rows;
+  for (uint64_t b = 0; b < batches; ++b)
+    if (host[b] <= limit) live += early_batches(p, host[b], batch);
+  const uint64_t total = early_batches(p, span, batch) * batches;
   return (total - live) * 16 < total;
 }
 
