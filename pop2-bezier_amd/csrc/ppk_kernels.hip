@@ -1267,8 +1267,8 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   const int j = lane / LPT;
   const int c = lane % LPT;
   // Blocks are numbered group-major: consecutive blocks belong to different
-  // rows, so the empty tail groups of short rows (ragged batches) spread over
-  // the CUs instead of leaving some CUs with only live blocks.
+  // rows, so the short blocks of short rows (with contiguous ranges, their
+  // empty tail groups) spread over the CUs.
   const uint32_t group = fast_div(blockIdx.x, a.row_div);
   const uint32_t row = blockIdx.x - group * a.rows;
   const uint32_t S = a.split_tokens;
