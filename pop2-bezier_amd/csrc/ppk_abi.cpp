@@ -155,28 +155,47 @@ static uint32_t score_tokens(uint32_t split, uint32_t batch) {
 }
 
 // How a row's waves take its batches, by the batches of one wave's share
-// (q = ceil(split / batch)). Shares of six batches or more within 1/16 of
-// whole pairs, and below 32: two batches at a time in turn. Shares of three, at
-// least 2.5 batches: one contiguous range per wave (the whole of K is in flight at
-// once, and turns only mix the waves' pages). Others: one batch at a time.
-// Same-box A/B, H = 16, us per step, contiguous ranges / turns of one / turns
-// of two / turns of four: B = 32 x 8192 D = 128 161.2 / 159.1 / 160.3 /
+// (q = ceil(split / batch)). One contiguous range per wave: shares of three
+// batches, at least 2.5 (the whole of K is in flight at once, and turns only
+// mix the waves' pages), and at D >= 128 shares above 16 where the grid is one
+// eight-wave block on (nearly) every CU. Two batches at a time in turn: the
+// other shares of six or more and below 32 within 1/16 of whole pairs. Others:
+// one batch at a time.
+// Measured over 840 drawn shapes of more than two batches a share (D = 64 /
+// 128 / 256, step and attention alone, 40 % bf16 history, uniform and ragged,
+// arenas of L + 1 and of a power of two slots; captured sequences), against
+// the kernels before turns existed, geometric mean and shapes more than 1.5 %
+// slower: contiguous ranges everywhere 1.034 / 90, turns of one 1.066 / 56,
+// of two 1.061 / 57, this rule 1.065 / 51; the best of the three for each shape
+// 1.075 / 11. No rule on sizes comes closer: what decides between them is how
+// ragged the lengths are and which rows share a CU (turns: 5 rows of 14062..878
+// tokens at D = 128 45.4 -> 35.4 us, 13 rows x 32 heads of 8183..511 81.8 ->
+// 95). One block per CU, shares above 16 batches: turns 4 % slower over the 13
+// such shapes (B = 16 x 4188 45.8 / 48.2 us, B = 4 x 9186 of 32 heads 47.7 /
+// 52.8); with half the CUs idle they gain again.
+// Shapes the rule was first fitted to, H = 16, us per step, contiguous / turns
+// of one / of two / of four: B = 32 x 8192 D = 128 161.2 / 159.1 / 160.3 /
 // 161.3, D = 64 89.0 / 85.7 / 86.6 / 86.6; B = 16 x 4096 D = 128 46.3 / 44.5 /
-// 43.9 / 44.5, x 3000 32.8 / 35.1 / 32.9 / 33.5, x 1500 18.3 / 19.7 / 18.3 / -,
-// x 1400 (5.5 batches) 17.3 / 16.9 / 17.7 / -; B = 32 x 1100 (9 batches) 25.0
-// / 24.3 / 26.1 / -; D = 64, B = 16 x 1500 (three batches) 10.8 / 11.3 / - /
-// -, x 1600 (3.25) 13.2 / 11.5 / - / -, x 300..700 7.4 / 6.8 / - / -. (The
-// arena's capacity has no say: a row's result does not depend on it. Where rows
-// start on 4 KiB boundaries turns of one would be up to 4 % faster: B = 32 x
-// 4000 D = 64 in 4096 slots 47.2 / 44.7 / 46.6 / -.)
-static Turns plan_turns(const AttentionPlan& p, uint32_t batch) {
+// 43.9 / 44.5, x 3000 32.8 / 35.1 / 32.9 / 33.5, x 1400 (5.5 batches) 17.3 /
+// 16.9 / 17.7 / -; D = 64, B = 16 x 1500 (three batches) 10.8 / 11.3 / - / -,
+// x 1600 (3.25) 13.2 / 11.5 / - / -. The arena's capacity has no say where the
+// call gives max_past or host lengths (without them the plan spans it).
+static Turns plan_turns(const ppk_context* ctx, const AttentionPlan& p, uint32_t rows, uint32_t batch) {
   Turns t;
-  const uint32_t q = (p.split + batch - 1) / batch;
+  const uint32_t q = (p.split + batch - 1) / batch, waves = p.ngroups * p.waves;
   const uint32_t pairs = (p.split + 2 * batch - 1) / (2 * batch) * 2 * batch;
-  t.shift = q >= 6 && q < 32 && 16 * (pairs - p.split) <= p.split ? 1 : q == 3 && 2 * p.split >= 5 * batch ? 31 : 0;
-  t.chunk = t.shift == 31 ? 3 : 1u << t.shift;
+  const uint64_t cus = uint64_t(std::max(ctx ? ctx->cu_count : 256, 1));
+  const uint64_t blocks = uint64_t(rows) * p.ngroups;
+  const bool one_per_cu = p.waves == kInt8WavesPerCu && blocks <= cus && 8 * blocks > 7 * cus;
+  if ((q == 3 && 2 * p.split >= 5 * batch) || (p.head_dim >= 128 && q > 16 && one_per_cu)) {
+    t.shift = 31;
+    t.chunk = q;
+  } else {
+    t.shift = q >= 6 && q < 32 && 16 * (pairs - p.split) <= p.split ? 1 : 0;
+    t.chunk = 1u << t.shift;
+  }
   t.tokens = score_tokens(p.split, batch);
-  t.div = fast_divisor(p.ngroups * p.waves);
+  t.div = fast_divisor(waves);
   return t;
 }
 
@@ -494,7 +513,7 @@ AttentionPlan plan_attention(const ppk_context* ctx, const PpkAttentionArgs& a) 
     }
   }
   if (!plan.flat) {
-    plan.turn = plan_turns(plan, 4 * tpl);
+    plan.turn = plan_turns(ctx, plan, a.rows, 4 * tpl);
     plan.speculate = per_row_speculates(plan, a.rows, a.heads, host, cover, limit, 4 * tpl);
     plan.span = uint32_t(span);
   }
