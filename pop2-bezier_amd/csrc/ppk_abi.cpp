@@ -776,7 +776,7 @@ AttentionPlan plan_flat(const ppk_context* ctx, uint32_t rows, uint32_t heads, c
 // flight between chunks. 512 x 8192 rows of D = 128, up to 128 / 1024 blocks per
 // CU: f32 494 / 436 us, bf16 260 / 255. Returns false (nothing launched) when the
 // operands do not fit these conditions.
-bool launch_stream_quantize(ppk_context* ctx, hipStream_t stream, int prof_kernel, QuantizeArgs k,
+bool launch_stream_quantize(ppk_context* ctx, hipStream_t stream, int prof_kernel, const QuantizeArgs& k,
                             uint32_t head_dim) {
   const uint32_t per_lane = k.src_dtype == PPK_F32 ? 4u : 8u;
   for (uint32_t t = 0; t < k.ntensors; ++t)
@@ -791,10 +791,9 @@ bool launch_stream_quantize(ppk_context* ctx, hipStream_t stream, int prof_kerne
   if (units < cus * 1024 && uint64_t(k.rows) * k.ntensors < cus * 48) return false;
   const uint64_t chunks = k.ntensors * ((units / k.ntensors + 255) / 256);
   const uint64_t grid = std::min<uint64_t>((chunks + 3) / 4, cus * 1024);
-  k.token_div = fast_divisor(k.tokens);
-  k.head_div = fast_divisor(k.heads);
+  StreamQuantizeArgs s{k, fast_divisor(k.tokens), fast_divisor(k.heads)};
   const Fn fn = Fn((k.capacity ? kQuantizeAppend64 : kQuantizeDense64) + dim_index(head_dim));
-  launch(ctx, prof_kernel, fn, uint32_t(grid), 256, 0, stream, k);
+  launch(ctx, prof_kernel, fn, uint32_t(grid), 256, 0, stream, s);
   return true;
 }
 

@@ -648,7 +648,7 @@ __device__ __forceinline__ float row_scale(float amax) {
 // of D = 128: 92.3 -> 65.0 us (6.1 TB/s), 8 x 16 x 3000 of D = 256: 133.6 ->
 // 90.9; dense 1 M rows of D = 128: 77 -> 70 us.
 template <int D, int E, uint32_t DT, bool ARENA>
-__device__ __forceinline__ void quantize_stream_units(const ppk::QuantizeArgs& a) {
+__device__ __forceinline__ void quantize_stream_units(const ppk::StreamQuantizeArgs& a) {
 #pragma clang fp contract(off)
   constexpr int G = D / E;
   constexpr int R = 4;
@@ -821,7 +821,7 @@ __device__ __forceinline__ void quantize_stream_units(const ppk::QuantizeArgs& a
 }
 
 template <int D, bool ARENA>
-__device__ __forceinline__ void quantize_stream_dtype(const ppk::QuantizeArgs& a) {
+__device__ __forceinline__ void quantize_stream_dtype(const ppk::StreamQuantizeArgs& a) {
   if (a.src_dtype == kF32) quantize_stream_units<D, 4, kF32, ARENA>(a);
   else if (a.src_dtype == kBF16) quantize_stream_units<D, 8, kBF16, ARENA>(a);
   else quantize_stream_units<D, 8, kF16, ARENA>(a);
@@ -3092,10 +3092,10 @@ extern "C" __global__ __launch_bounds__(256) void ppk_dequantize(ppk::Dequantize
 // (ppk_quantize_append, KV arena writes), separate kernels so the dense path
 // keeps its smaller register footprint.
 #define PPK_QSTREAM(D)                                                                              \
-  extern "C" __global__ __launch_bounds__(256) void ppk_quantize_dense_d##D(ppk::QuantizeArgs a) {  \
+  extern "C" __global__ __launch_bounds__(256) void ppk_quantize_dense_d##D(ppk::StreamQuantizeArgs a) {  \
     quantize_stream_dtype<D, false>(a);                                                             \
   }                                                                                                 \
-  extern "C" __global__ __launch_bounds__(256) void ppk_quantize_append_d##D(ppk::QuantizeArgs a) { \
+  extern "C" __global__ __launch_bounds__(256) void ppk_quantize_append_d##D(ppk::StreamQuantizeArgs a) { \
     quantize_stream_dtype<D, true>(a);                                                              \
   }
 PPK_QSTREAM(64)
