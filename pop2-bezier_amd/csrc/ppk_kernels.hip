@@ -2696,7 +2696,7 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
   __shared__ float s_sum[T], s_sum_a[T];
   __shared__ float s_wmax[T / 64], s_wmin[T / 64];
   __shared__ uint32_t s_wid[T / 64], s_wbad[T / 64];
-  __shared__ __attribute__((aligned(16))) uint32_t s_bins[BINS];
+  __shared__ __attribute__((aligned(16))) uint32_t s_bins[BINS + 64];
   __shared__ float s_list_v[LIST];
   __shared__ uint32_t s_list_i[LIST];
   __shared__ uint32_t s_listed;
@@ -2795,11 +2795,18 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
 
   // Strided partial sums in candidate order, then the halving tree. The bins
   // of the selection are counted beside them: bin = (maximum - v) scaled to
-  // BINS, a rounded subtraction and a rounded product, so a larger value never
-  // has a higher bin.
+  // BINS over the range or kSpan, whichever is less, a rounded subtraction and
+  // a rounded product, so a larger value never has a higher bin. Values further
+  // down than kSpan (masked ones, an outlier: weight below 2e-7 each) go to a
+  // word of their lane that nothing reads: in the range they would stretch the
+  // bins until nearly all values shared one, in the last bin they would queue
+  // at its word (32 rows x 2048 with guidance 6.2 us, with one outlier 11.8, now
+  // 6.3 both; in the last bin 7.5, with a branch around the count 6.5).
+  constexpr float kSpan = 16.0f;
   const float range = maximum - minimum;
-  const float bin_scale = float(BINS) / range;
-  const bool binned = range > 0.f && finite_bits(range) && finite_bits(bin_scale);
+  const float beyond = range > kSpan ? float(BINS) : INFINITY;
+  const float bin_scale = float(BINS) / fminf(range, kSpan);
+  const bool binned = range > 0.f && finite_bits(bin_scale);
   float vals[PER];
   uint32_t bins[PER];
   float sum = 0.f, sum_a = 0.f;
@@ -2813,7 +2820,8 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
       sum += expf(shifted);
       sum_a += expf(a.alpha * shifted);
       if (binned) {
-        bins[k] = min(uint32_t((maximum - vals[k]) * bin_scale), uint32_t(BINS - 1));
+        const float at = (maximum - vals[k]) * bin_scale;
+        bins[k] = at < beyond ? uint32_t(fminf(at, float(BINS - 1))) : uint32_t(BINS + lane);
         atomicAdd(&s_bins[bins[k]], 1u);
       }
     }
@@ -2865,8 +2873,11 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
 
   // The bin that holds rank r (every wave finds it, from BINS / 64 bins per
   // lane and a prefix sum over the lanes); its few candidates go to a list and
-  // are ordered by direct comparison. A bin of more than LIST candidates (heavy
-  // ties, or one outlier that stretches the range) is left to the radix passes.
+  // are ordered by direct comparison. More than LIST candidates that are all
+  // equal (heavy ties) are ordered by index below; other crowded bins, and a
+  // rank among the values that are not counted, are left to the radix passes.
+  uint32_t prefix = 0, pmask = 0;
+  bool tied = false;
   if (binned) {
     constexpr int PL = BINS / 64;
     uint32_t h[PL], total = 0;
@@ -2891,11 +2902,11 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
         }
       }
     }
-    const int owner = __builtin_ctzll(here);  // one lane: the bins hold all `count` > r candidates
+    const int owner = here ? __builtin_ctzll(here) : 0;  // one lane at most
     bin = __builtin_amdgcn_readlane(bin, owner);
     in_bin = __builtin_amdgcn_readlane(in_bin, owner);
     below = __builtin_amdgcn_readlane(below, owner);
-    if (in_bin <= LIST) {  // uniform
+    if (here != 0 && in_bin <= LIST) {  // uniform
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
         if (bins[k] == bin) {
@@ -2918,6 +2929,31 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
       if (uint32_t(lane) < in_bin && rank == r) write_sample(a, row, a.token_offset + start + ci, 1, support);
       return;
     }
+    if (here != 0) {  // uniform
+      float hi = -INFINITY, lo = INFINITY;
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        hi = bins[k] == bin ? fmaxf(hi, vals[k]) : hi;
+        lo = bins[k] == bin ? fminf(lo, vals[k]) : lo;
+      }
+      hi = wave_max(hi);
+      lo = wave_reduce(lo, [](float x, float y) { return fminf(x, y); });
+      if (lane == 0) {  // last read before the sums' barrier
+        s_wmax[wave] = hi;
+        s_wmin[wave] = lo;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < T / 64; ++w) {
+        hi = fmaxf(hi, s_wmax[w]);
+        lo = fminf(lo, s_wmin[w]);
+      }
+      tied = hi == lo;
+      if (tied) {
+        prefix = descending_key(hi);
+        r -= below;
+      }
+    }
   }
 
   // Radix select, 8 key bits per pass from the top: after four passes the
@@ -2925,8 +2961,7 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
   uint32_t keys[PER];
 #pragma unroll
   for (int k = 0; k < PER; ++k) keys[k] = descending_key(vals[k]);
-  uint32_t prefix = 0, pmask = 0;
-  for (int shift = 24; shift >= 0; shift -= 8) {
+  for (int shift = tied ? -8 : 24; shift >= 0; shift -= 8) {
     s_hist[t] = 0;
     __syncthreads();
 #pragma unroll

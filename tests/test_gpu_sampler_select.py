@@ -1,8 +1,9 @@
 """The sampler's choice of the rank-th candidate, at the edges of its bins.
 
-The kernel counts values into 512 equal bins and orders the selected bin's
-candidates by comparison where they are at most 64, by radix passes where they
-are more. Which path a row takes may not show: the token is the rank-th legal
+The kernel counts values into 512 equal bins over at most 16 below the maximum
+and orders the selected bin's candidates by comparison where they are at most
+64, by index where they are more and all equal, by radix passes otherwise and
+where the rank lies further down than the bins. Which path a row takes may not show: the token is the rank-th legal
 candidate by (value descending, index ascending), with the kernel's own
 support, exactly.
 """
@@ -63,3 +64,38 @@ def test_rank_names_the_sorted_candidate(device, kind, choices):
         rank = min(int(F32(uniform[b] * F32(sup[b]))), int(sup[b]) - 1)
         want = 5 + start[b] + np.argsort(-legal.astype(np.float64), kind="stable")[rank]
         assert tok[b] == want, (kind, choices, b, rank, sup[b])
+
+
+@pytest.mark.parametrize("choices", [2, 65, 300, 2048])
+@pytest.mark.parametrize("kind", ["masked", "few_values", "crowded_unequal", "below_the_bins"])
+def test_beyond_the_bins_and_crowded_bins(device, kind, choices):
+    rng = np.random.default_rng(SEED + 3 * choices)
+    batch, alpha = 40, 3.5
+    x = (rng.standard_normal((batch, choices)) * 0.5).astype(F32)
+    if kind == "masked":  # most values far below, at one value and at several
+        x[rng.random((batch, choices)) < 0.9] = -1e4
+        x[: batch // 2, ::3] = -60.0
+    elif kind == "few_values":  # bins of equal values, zeros of both signs among them
+        x = rng.choice(np.array([0.0, -0.0, 0.25, -3.0, -40.0], F32), (batch, choices))
+    elif kind == "crowded_unequal":  # more than 64 unequal values in one bin, stretched by one at 15 below
+        x = (x * 1e-3).astype(F32)
+        x[:, -1] = -15.0
+    else:  # alpha next to 1: the entropy's rounding makes supports of all sizes, ranks past the bins among them
+        x[:] = np.linspace(0, -200, choices, dtype=F32)[rng.permutation(choices)]
+        alpha = float(np.nextafter(F32(1), F32(2)))
+    count = np.full(batch, choices, np.uint32)
+    uniform = np.linspace(0, 0.999, batch, dtype=F32)
+    bounds = np.stack([np.zeros(batch, np.uint32), count], 1)
+    tok, val, sup = ppk.sampling.sample(
+        torch.from_numpy(x).to(device), torch.from_numpy(uniform.reshape(-1, 1)).to(device),
+        torch.from_numpy(bounds.view(np.int32)).to(device), alpha, 1.0, 1, 5)
+    tok, val, sup = (t.reshape(-1).cpu().numpy().view(np.uint32) for t in (tok, val, sup))
+    assert np.all(val == 1)
+    below = 0
+    for b in range(batch):
+        rank = min(int(F32(uniform[b] * F32(sup[b]))), int(sup[b]) - 1)
+        order = np.argsort(-x[b].astype(np.float64), kind="stable")
+        assert tok[b] == 5 + order[rank], (kind, choices, b, rank, sup[b])
+        below += x[b, order[rank]] < x[b].max() - 16
+    if kind == "below_the_bins" and choices == 2048:  # (smaller supports may round to none)
+        assert below > 0, "no rank past the bins"
