@@ -1188,11 +1188,13 @@ __device__ __forceinline__ void write_block_record(float* rec, int ch, int lane,
 // Log-sum-exp combine of a block's W <= MAXW records (stride floats apart) and
 // a score s0 that joins the maximum (-inf for none), by one wave: lane w takes
 // record w's (m, z), the y rows of this lane's channels are requested eight
-// records at a time (past W: the last record again, counted as 0: a weight of
-// 0 alone would make an infinite y of that record NaN). One LDS round trip
-// for the weights and one for the rows; a loop over the records took two per
-// record, ~0.7 us at the end of every 8-wave block.
-template <int D, int MAXW>
+// records at a time (past W: the last record again, with weight 0). One LDS
+// round trip for the weights and one for the rows; a loop over the records
+// took two per record, ~0.7 us at the end of every 8-wave block. MAYBE_INF: a
+// y may be infinite (a float store that holds infinities; codes times finite
+// scales are not), and the places past W count as 0, since a weight of 0 alone
+// would make it NaN.
+template <int D, int MAXW, bool MAYBE_INF>
 __device__ __forceinline__ void combine_block(const float* recs, uint32_t stride, uint32_t W, int lane, float s0,
                                               float& m, float& z, float (&y)[D / ppk::kWave]) {
   constexpr int EPL = D / ppk::kWave;
@@ -1215,21 +1217,25 @@ __device__ __forceinline__ void combine_block(const float* recs, uint32_t stride
   z = wave_sum(wt * zw);
 #pragma unroll
   for (int e = 0; e < EPL; ++e) y[e] = 0.f;
-  // One and two records by themselves, the rest of eight without a branch each
-  // (a branch per record cost blocks of eight waves 0.1-0.2 us).
-  auto add1 = [&](uint32_t w0, int k) {
-    const bool there = k < 2 || w0 + uint32_t(k) < W;
+  auto add1 = [&](uint32_t w0, int k, bool there) {
     const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wt), int(w0) + k));
 #pragma unroll
     for (int e = 0; e < EPL; ++e) y[e] = fmaf(wk, there ? v[k][e] : 0.f, y[e]);
   };
   auto add = [&](uint32_t w0) {
-    add1(w0, 0);
-    if (W - w0 < 2) return;  // uniform
-    add1(w0, 1);
-    if (W - w0 < 3) return;
+    if constexpr (MAYBE_INF) {
+      // One and two records by themselves, the rest of eight without a branch
+      // each (a branch per record cost blocks of eight waves 0.1-0.2 us).
+      add1(w0, 0, true);
+      if (W - w0 < 2) return;  // uniform
+      add1(w0, 1, true);
+      if (W - w0 < 3) return;
 #pragma unroll
-    for (int k = 2; k < 8; ++k) add1(w0, k);
+      for (int k = 2; k < 8; ++k) add1(w0, k, w0 + uint32_t(k) < W);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) add1(w0, k, true);
+    }
   };
   add(0);
   if constexpr (MAXW > 8) {
@@ -1463,7 +1469,7 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   }
 
   float m, y[EPL], zsum;
-  combine_block<D, 8>(lds, lds_stride, uint32_t(W), lane, s_cur, m, zsum, y);
+  combine_block<D, 8, false>(lds, lds_stride, uint32_t(W), lane, s_cur, m, zsum, y);
   if (final_out) {
     const float wc = __builtin_amdgcn_exp2f(s_cur - m);
     zsum += wc;
@@ -2249,7 +2255,7 @@ __device__ __forceinline__ void fdecode_body(const ppk::FloatDecodeArgs& a) {
   if (wave != 0) return;
 
   float m, y[EPL], zsum;
-  combine_block<D, 16>(lds, lds_stride, uint32_t(W), lane, s_cur, m, zsum, y);
+  combine_block<D, 16, true>(lds, lds_stride, uint32_t(W), lane, s_cur, m, zsum, y);
   if (cur) {
     const float wc = __builtin_amdgcn_exp2f(s_cur - m);
     zsum += wc;
