@@ -71,6 +71,8 @@ const char* kFnNames[ppk::kFnCount] = {
     "ppk_fstep_f32_d64", "ppk_fstep_f32_d128", "ppk_fstep_f32_d256",
     "ppk_fstep_flat_bf16_d64", "ppk_fstep_flat_bf16_d128", "ppk_fstep_flat_bf16_d256",
     "ppk_fstep_flat_f32_d64", "ppk_fstep_flat_f32_d128", "ppk_fstep_flat_f32_d256",
+    "ppk_decode_late_d64", "ppk_decode_late_d128", "ppk_decode_late_d256",
+    "ppk_decode_late_bf16h_d64", "ppk_decode_late_bf16h_d128", "ppk_decode_late_bf16h_d256",
 };
 
 std::string default_code_object() {
@@ -950,7 +952,6 @@ void run_attention(ppk_context* ctx, hipStream_t stream, const PpkAttentionArgs&
   d.scratch_dtype = a.scratch_dtype;
   d.out_dtype = a.out_dtype;
   d.scale_log2 = scale_log2;
-  d.speculate = plan.speculate ? 1u : 0u;
   d.span = plan.span;
   if (ctx && ctx->wave_clock) {
     std::lock_guard<std::mutex> lock(ctx->prof_mutex);
@@ -995,7 +996,8 @@ void run_attention(ppk_context* ctx, hipStream_t stream, const PpkAttentionArgs&
   // The int8 plan's blocks hold at most 8 waves: the kernels are bounded to
   // 512 threads (two waves per SIMD, up to 256 VGPRs, three batches in flight).
   require(plan.waves <= 8, "internal: int8 decode block of more than 8 waves");
-  const Fn decode = Fn((bf16h ? kDecodeBf16h64 : kDecode64) + di);
+  const Fn decode = Fn((plan.speculate ? bf16h ? kDecodeBf16h64 : kDecode64
+                                       : bf16h ? kDecodeLateBf16h64 : kDecodeLate64) + di);
   DeviceGuard guard(ctx->device);
   launch(ctx, PPK_KERNEL_ATTENTION, decode, plan.ngroups * a.rows, 64 * plan.waves, plan.lds_bytes, stream, d, 1,
          traceable);

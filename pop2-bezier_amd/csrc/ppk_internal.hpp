@@ -60,6 +60,8 @@ enum Fn : int {
   kFStepF32_64, kFStepF32_128, kFStepF32_256,
   kFStepFlatBf16_64, kFStepFlatBf16_128, kFStepFlatBf16_256,
   kFStepFlatF32_64, kFStepFlatF32_128, kFStepFlatF32_256,
+  kDecodeLate64, kDecodeLate128, kDecodeLate256,
+  kDecodeLateBf16h64, kDecodeLateBf16h128, kDecodeLateBf16h256,
   kFnCount
 };
 

@@ -134,7 +134,6 @@ struct DecodeArgs {
   float scale_log2;         // softmax_scale * log2(e)
   uint32_t span;            // max_past or capacity: balanced plan, rows with past[b] > span give NaN; per-row
                             // plan, a past[b] <= span past the plan's coverage flags stale host lengths
-  uint32_t speculate;       // per-row plan: request each wave's first K batches before past[] arrives
   FastDiv row_div, head_div;  // by rows, by heads
   Turns turn;               // per-row plan
   uint32_t clock_seq;       // wave-clock builds only: the launch's sequence number in the records

@@ -1246,7 +1246,7 @@ __device__ __forceinline__ void combine_block(const float* recs, uint32_t stride
   }
 }
 
-template <int D, bool BF16H, int NB>
+template <int D, bool BF16H, int NB, bool EARLY>
 __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   constexpr int LPT = D / 16;
   constexpr int TPL = ppk::kWave / LPT;
@@ -1261,7 +1261,7 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   // another).
   __asm__ volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.ks), "s"(a.vs), "s"(a.sk), "s"(a.sv), "s"(a.past),
                    "s"(a.k_new), "s"(a.v_new), "s"(a.rows), "s"(a.capacity), "s"(a.split_tokens), "s"(a.ngroups),
-                   "s"(a.q_dtype), "s"(a.scratch_dtype), "s"(a.new_dtype), "s"(a.append), "s"(a.speculate),
+                   "s"(a.q_dtype), "s"(a.scratch_dtype), "s"(a.new_dtype), "s"(a.append),
                    "s"(a.row_div.mul), "s"(a.row_div.shift), "s"(a.head_div.mul), "s"(a.head_div.shift),
                    "s"(a.turn.div.mul), "s"(a.turn.div.shift), "s"(a.turn.shift), "s"(a.turn.chunk), "s"(blockDim.x));
   const int lane = threadIdx.x & 63;
@@ -1293,7 +1293,7 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   // 24 layers of 2048 tokens at D = 128 204.8, now 187.8; B = 16 x 1500 at D =
   // 64 11.16, now 10.62; B = 32 x 8192 unchanged (162.2). The slot the commit
   // writes is past every wave's length, so the speculative reads of it are
-  // masked. The host turns the early batches off (a.speculate = 0) when it
+  // masked. The host turns the early batches off (the kernel without EARLY) when it
   // knows many waves have no history (ragged host lengths, or waves past the
   // span): their speculative reads would be wasted bandwidth (config 4: 9 %
   // more HBM traffic than the history, 18.7 -> 18.3 us without).
@@ -1409,13 +1409,13 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
   // that is not there: with ragged host lengths and the bf16 history, which
   // that arithmetic bounds, one-batch waves took 8.4 us where they did both
   // (64 rows of 181..362 tokens at D = 64), now 6.0.
-  if (!a.speculate) {
+  if constexpr (!EARLY) {
     length_here();
     nspec = n;
   }
   const Batches early = row_batches<TPB>(a.turn, nspec, place, turns);
   auto prologue = [&]() {
-    if (a.speculate) length_here();
+    if constexpr (EARLY) length_here();
     operands_here();
   };
   // The paths differ in what is in flight when the prologue runs; each runs
@@ -3146,15 +3146,26 @@ PPK_QSTREAM(256)
 
 // Blocks of up to 8 waves (the plan never makes larger int8 blocks): two
 // waves per SIMD, up to 256 VGPRs each, a ring of kRing batches in flight.
+// The late kernels wait for the row's length before their first batches; one
+// kernel with both ways was 1-4 % slower on rows of one batch a wave (16 rows
+// x 512 tokens at D = 64 4.45 us, now 4.38).
 constexpr int kRing = 3;
 #define PPK_ATTN(D)                                                                          \
   extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))    \
   void ppk_decode_d##D(ppk::DecodeArgs a) {                                                  \
-    decode_body<D, false, kRing>(a);                                                         \
+    decode_body<D, false, kRing, true>(a);                                                   \
   }                                                                                          \
   extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))    \
   void ppk_decode_bf16h_d##D(ppk::DecodeArgs a) {                                            \
-    decode_body<D, true, kRing>(a);                                                          \
+    decode_body<D, true, kRing, true>(a);                                                    \
+  }                                                                                          \
+  extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))    \
+  void ppk_decode_late_d##D(ppk::DecodeArgs a) {                                             \
+    decode_body<D, false, kRing, false>(a);                                                  \
+  }                                                                                          \
+  extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))    \
+  void ppk_decode_late_bf16h_d##D(ppk::DecodeArgs a) {                                       \
+    decode_body<D, true, kRing, false>(a);                                                   \
   }                                                                                          \
   extern "C" __global__ __launch_bounds__(64) void ppk_attn_merge_d##D(ppk::MergeArgs a) {   \
     attn_merge_body<D>(a);                                                                   \
