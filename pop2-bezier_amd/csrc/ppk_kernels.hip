@@ -2803,14 +2803,14 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
   // of the selection are counted beside them: bin = (maximum - v) scaled to
   // BINS over the range or kSpan, whichever is less, a rounded subtraction and
   // a rounded product, so a larger value never has a higher bin. Values further
-  // down than kSpan (masked ones, an outlier: weight below 2e-7 each) go to a
-  // word of their lane that nothing reads: in the range they would stretch the
+  // down than kSpan (masked ones, an outlier: weight below 2e-7 each) go to words
+  // past the bins, spread by lane, that nothing reads: in the range they would stretch the
   // bins until nearly all values shared one, in the last bin they would queue
   // at its word (32 rows x 2048 with guidance 6.2 us, with one outlier 11.8, now
   // 6.3 both; in the last bin 7.5, with a branch around the count 6.5).
   constexpr float kSpan = 16.0f;
   const float range = maximum - minimum;
-  const float beyond = range > kSpan ? float(BINS) : INFINITY;
+  const float last = float(range > kSpan ? BINS + lane : BINS - 1);
   const float bin_scale = float(BINS) / fminf(range, kSpan);
   const bool binned = range > 0.f && finite_bits(bin_scale);
   float vals[PER];
@@ -2826,8 +2826,7 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
       sum += expf(shifted);
       sum_a += expf(a.alpha * shifted);
       if (binned) {
-        const float at = (maximum - vals[k]) * bin_scale;
-        bins[k] = at < beyond ? uint32_t(fminf(at, float(BINS - 1))) : uint32_t(BINS + lane);
+        bins[k] = uint32_t(fminf((maximum - vals[k]) * bin_scale, last));
         atomicAdd(&s_bins[bins[k]], 1u);
       }
     }
