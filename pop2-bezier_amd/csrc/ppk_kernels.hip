@@ -390,7 +390,7 @@ __device__ __forceinline__ void raise_flags(uint32_t* flags, uint32_t bits) {
 
 // Quantise one row of D values into codes[0..D) and *scale; the whole wave
 // participates, lane l holding elements l*D/64 ... (l+1)*D/64 - 1 of the
-// row. Returns whether any value was non-finite. Every lane stores the scale
+// row. Returns whether a value of the lane was non-finite. Every lane stores the scale
 // (one value at one address): a lane-0 branch here would make the compiler
 // restructure the control flow around it, and the decode kernels' streaming
 // loops then wait for loads of paths that never reach them.
@@ -416,7 +416,7 @@ __device__ __forceinline__ bool quantize_values(const float (&x)[D / ppk::kWave]
   else if constexpr (EPL == 2) *reinterpret_cast<uint16_t*>(out) = uint16_t(packed);
   else *reinterpret_cast<uint32_t*>(out) = packed;
   if (!ONE || lane == 0) *scale = s;
-  return __any(!finite);
+  return !finite;
 }
 
 // The same for row src_row of src[rows, D] in dtype.
@@ -426,7 +426,8 @@ __device__ __forceinline__ void quantize_row(const void* src, size_t src_row, ui
   constexpr int EPL = D / ppk::kWave;
   float x[EPL];
   load_vec<EPL>(src, src_row * D + size_t(lane) * EPL, dtype, x);
-  if (quantize_values<D, true>(x, codes, scale, lane) && flags && lane == 0) atomicOr(flags, 1u);
+  const bool bad = quantize_values<D, true>(x, codes, scale, lane);
+  if (flags && __any(bad) && lane == 0) atomicOr(flags, 1u);
 }
 
 template <int D>
@@ -1379,11 +1380,11 @@ __device__ __forceinline__ void decode_body(const ppk::DecodeArgs& a) {
         float t[EPL];
         if (kw) {
           widen<EPL>(kn_raw, a.new_dtype, t);
-          if (quantize_values<D>(t, a.k + slot * D, a.ks + slot, lane)) raise |= 1u;
+          if (__any(quantize_values<D>(t, a.k + slot * D, a.ks + slot, lane))) raise |= 1u;
         }
         if (vw) {
           widen<EPL>(vn_raw, a.new_dtype, t);
-          if (quantize_values<D>(t, a.v + slot * D, a.vs + slot, lane)) raise |= 1u;
+          if (__any(quantize_values<D>(t, a.v + slot * D, a.vs + slot, lane))) raise |= 1u;
         }
       }
     }
@@ -1817,7 +1818,7 @@ __device__ __forceinline__ void decode_flat_body(const ppk::DecodeFlatArgs& fa) 
       const bool value = (wid & 1u) != 0;
       float x[EPL];
       widen<EPL>(new_raw, a.new_dtype, x);
-      if (quantize_values<D>(x, (value ? a.v : a.k) + dst * D, (value ? a.vs : a.ks) + dst, lane)) raise |= 1u;
+      if (__any(quantize_values<D>(x, (value ? a.v : a.k) + dst * D, (value ? a.vs : a.ks) + dst, lane))) raise |= 1u;
     }
   };
   auto report = [&]() { raise_flags(a.flags, raise); };
