@@ -194,13 +194,8 @@ __device__ __forceinline__ void issue_here() {
   __asm__ volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
-// x / d for x < 2^31 by the host's precomputed FastDiv of d (scalar: one
-// multiply-high and a shift, where the compiler's division takes ~30
-// dependent instructions, on the path of every wave's first load).
-__device__ __forceinline__ uint32_t fast_div(uint32_t x, const ppk::FastDiv& d) {
-  const uint32_t q = uint32_t((uint64_t(x) * d.mul) >> 32) >> d.shift;
-  return d.mul ? q : x;
-}
+using ppk::fast_div;
+using ppk::row_scale;
 // A zero the compiler takes for a per-lane value: added to a uniform index it
 // makes the load a vector load, which waits in order with the wave's other
 // vector loads. A scalar load of the same word shares its counter with the
@@ -454,7 +449,7 @@ __device__ __forceinline__ void quantize_body(const ppk::QuantizeArgs& a) {
 }
 
 // ---------------------------------------------------------------------------
-// Dequantize: 16 codes per thread (one dwordx4), grid-stride.
+// Dequantize
 // ---------------------------------------------------------------------------
 // Dequantization in units of one 16-byte output chunk: E = 8 codes for a
 // 16-bit output, 4 for f32. A wave takes chunks of R * 64 consecutive units,
@@ -617,17 +612,6 @@ __device__ __forceinline__ float group_max_nonneg(float x) {
 #pragma unroll
   for (int o = 16; o < G; o <<= 1) step(uint32_t(__shfl_xor(int(b), o)));
   return __uint_as_float(b);
-}
-
-// absmax / 127 correctly rounded for every finite absmax whose quotient is not
-// below the scale's floor: the product with the rounded reciprocal, corrected
-// once by its exact remainder (Markstein's division by a constant). With the
-// floor applied it equals the IEEE division for all finite non-negative floats
-// (checked over all 2^31 of them). 3 instructions instead of ~12.
-__device__ __forceinline__ float row_scale(float amax) {
-  constexpr float kInv = 1.0f / 127.0f;
-  const float q = amax * kInv;
-  return fmaxf(__builtin_fmaf(__builtin_fmaf(-127.0f, q, amax), kInv, q), 1e-12f);
 }
 
 // Quantization at streaming rates: dense (int8_kv_ops::quantize over [rows,
@@ -2772,7 +2756,7 @@ __device__ __forceinline__ void renyi_sample_body(const ppk::RenyiArgs& a) {
   {
     const float wmax = wave_max(lmax);
     const float wmin = wave_reduce(lmin, [](float x, float y) { return fminf(x, y); });
-    // The least index of the wave's maximum, on the bit patterns of indexes (below 2^24: exact as floats).
+    // The least index of the wave's maximum, with the indexes as floats (below 2^24: exact).
     const float id = wave_reduce(lmax == wmax && lid != 0xffffffffu ? float(lid) : 16777216.f,
                                  [](float x, float y) { return fminf(x, y); });
     const bool wbad = __any(lbad != 0);
